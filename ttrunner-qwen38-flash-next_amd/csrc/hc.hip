@@ -13,7 +13,8 @@
 // and after it _reinject (reference/model.py:79-81) adds the branch output back
 // into every stream, scaled by that stream's inject weight.
 //
-// At decode M is a handful of rows, so both products are streams over the
+// From a few rows on the matrix-core kernels of hc_rows.hip do this (see
+// hc_takes_rows). Here M is a handful of rows, so both products are streams over the
 // weights (down|inject [rank + streams, K], up [K, rank]: about 5 MB each at
 // K = 8192, rank 320) and the rest is elementwise. Two launches do the mix:
 //
@@ -32,7 +33,7 @@
 // the same point (F.linear outputs, the division by streams, silu, sigmoid,
 // the gated product, the mean), so bf16 results differ from it only by the
 // order of the f32 sums.
-#include "common.h"
+#include "rows_mma.h"
 #include "qwen4mix_internal.h"
 
 namespace {
@@ -71,33 +72,6 @@ __device__ __forceinline__ float chunk_dot(const uint4& w, const uint4& x, float
   acc = fmaf(__uint_as_float(w.z), __uint_as_float(x.z), acc);
   return fmaf(__uint_as_float(w.w), __uint_as_float(x.w), acc);
 }
-
-// element i (0..VE-1) of a 16-byte chunk as float, and back
-template <typename T> struct Chunk;
-template <> struct Chunk<bf16_t> {
-  static constexpr int VE = 8;
-  __device__ __forceinline__ static float get(const uint4& c, int i) {
-    const unsigned w = i < 2 ? c.x : i < 4 ? c.y : i < 6 ? c.z : c.w;
-    return __uint_as_float((i & 1) ? (w & 0xffff0000u) : (w << 16));
-  }
-  __device__ __forceinline__ static uint4 pack(const float* v) {
-    uint4 c;
-    c.x = f32_to_bf16(v[0]) | (static_cast<unsigned>(f32_to_bf16(v[1])) << 16);
-    c.y = f32_to_bf16(v[2]) | (static_cast<unsigned>(f32_to_bf16(v[3])) << 16);
-    c.z = f32_to_bf16(v[4]) | (static_cast<unsigned>(f32_to_bf16(v[5])) << 16);
-    c.w = f32_to_bf16(v[6]) | (static_cast<unsigned>(f32_to_bf16(v[7])) << 16);
-    return c;
-  }
-};
-template <> struct Chunk<float> {
-  static constexpr int VE = 4;
-  __device__ __forceinline__ static float get(const uint4& c, int i) {
-    return __uint_as_float(i == 0 ? c.x : i == 1 ? c.y : i == 2 ? c.z : c.w);
-  }
-  __device__ __forceinline__ static uint4 pack(const float* v) {
-    return make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3]));
-  }
-};
 
 // ---------------------------------------------------------------------------
 // normalise + down|inject products. grid (ceil(n_rows / R), ceil(M / MG)).
@@ -379,6 +353,19 @@ const char* hc_check(const qm_hc_geom* g) {
   return nullptr;
 }
 
+// Where the matrix-core kernels (hc_rows.hip) take over. They would be faster
+// from 3 rows on (whole mix, us, here and there: bf16 13.7 / 10.5 at 4 rows,
+// 16.0 / 10.6 at 5, 24.7 / 10.9 at 14; float 18.9 / 17.4 at 5, 35.6 / 18.2 at
+// 14), but these kernels give a row the same bits at every row count, and a
+// verify step's few drafted tokens should see the inputs that their single
+// steps saw: with another order of the sums the first layer's states came out
+// 1.4e-3 apart instead of below 1e-3. So up to 8 rows stay here.
+constexpr int HC_ROWS_MIN = 9;
+
+bool hc_takes_rows(const qm_hc_geom& g) {
+  return g.rows >= HC_ROWS_MIN && qm_hc_rows_covers(g) && qm_hc_rows_workspace(g) <= hc_layout(g).total;
+}
+
 template <typename T, int MG, int NQ>
 void launch_up_mg(const HcArgs<T>& A, hipStream_t stream) {
   constexpr int HB = HcTile<T>::HB;
@@ -472,6 +459,8 @@ extern "C" int qm_hc_mix(const qm_hc_geom* g, const void* hyper, const float* no
     return qm_fail(QM_ERR_ARG, "qm_hc_mix: hyper, weights and workspace must be 16-byte aligned");
   if (with_inject && !inject) return qm_fail(QM_ERR_ARG, "qm_hc_mix: with_inject needs an inject output");
   if (workspace_bytes < hc_layout(*g).total) return qm_fail(QM_ERR_WORKSPACE, "qm_hc_mix: workspace too small");
+  if (hc_takes_rows(*g) && aligned16(mixed))
+    return qm_hc_mix_rows(*g, hyper, norm_w, down_inject_w, with_inject, up_w, mixed, inject, workspace, stream);
   if (g->act_dtype == QM_ACT_BF16)
     return run_mix<bf16_t>(*g, hyper, norm_w, down_inject_w, with_inject, up_w, mixed, inject, workspace, stream);
   return run_mix<float>(*g, hyper, norm_w, down_inject_w, with_inject, up_w, mixed, inject, workspace, stream);
