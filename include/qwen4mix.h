@@ -394,6 +394,16 @@ int qm_gemv(int act_dtype, int m, int n, int k, const void* w, const void* x, in
 int qm_gemv_reinject(int act_dtype, int m, int n, int k, const void* w, const void* x, int streams,
                      const void* inject, void* hyper, hipStream_t stream);
 
+/* qm_gemv and qm_gemv_reinject for up to 64 activation rows (a batch of
+ * sequences decoding, the tokens of a verify step), on the matrix cores: the
+ * same products, segments, epilogue and roundings, the float sums in another
+ * order. w and x (and hyper) 16-byte aligned; n of the reinjection a multiple
+ * of 4; k as qm_gemv. */
+int qm_gemm_rows(int act_dtype, int m, int n, int k, const void* w, const void* x, int n_seg, const int* seg_rows,
+                 void* const* seg_out, hipStream_t stream);
+int qm_gemm_rows_reinject(int act_dtype, int m, int n, int k, const void* w, const void* x, int streams,
+                          const void* inject, void* hyper, hipStream_t stream);
+
 /* ------------------------------------------------------------------------ */
 /* Hyper-connections around each branch                                     */
 /* ------------------------------------------------------------------------ */

@@ -1,5 +1,6 @@
 """The matrix-core kernels over token rows: the hyper-connection mix
-(hc_rows.hip) against the oracle's _gated_residual.
+(hc_rows.hip) against the oracle's _gated_residual, and the projections
+(gemm_rows.hip) against float64 products.
 
 Row counts at the edges of the row tiles (16, 32, 64, 256) and of the dispatch
 (8/9: one-row kernels to few-rows; 192/193 and 512/513: few to many).
@@ -9,6 +10,7 @@ every step, as the kernels do), 1e-4 in float32 (another summation order).
 
 from __future__ import annotations
 
+import ctypes
 import os
 import sys
 
@@ -52,3 +54,75 @@ def test_hyper_mix_rows_match_oracle(gpu, dtype, hidden, rows):
             assert inject is None
         else:
             assert rel_err(inject, want_inject, tol) < tol
+
+
+def _gemm_rows(qm, w, x, rows):
+    m, k = x.shape
+    outs = [torch.full((m, r), float("nan"), dtype=x.dtype, device=DEV) for r in rows]
+    seg_rows = (ctypes.c_int * len(rows))(*rows)
+    seg_out = (ctypes.c_void_p * len(rows))(*[o.data_ptr() for o in outs])
+    qm.native.call("qm_gemm_rows", qm.native.act_code(x.dtype), m, w.shape[0], k, w.data_ptr(), x.data_ptr(),
+                   len(rows), seg_rows, seg_out, qm.native.stream_handle())
+    torch.cuda.synchronize()
+    return outs
+
+
+@pytest.mark.parametrize("dtype,k", [(BF, 2048), (BF, 4096), (F32, 1024), (F32, 2048), (F32, 4096)])
+@pytest.mark.parametrize("m", [1, 5, 15, 16, 17, 33, 64])
+def test_gemm_rows_matches_fp64_product(gpu, dtype, k, m):
+    """qm_gemm_rows against a float64 product of the same operands: bf16 within
+    one rounding of the result (2^-8 of its row's largest value), float32 within
+    1e-5 (the sums' order). Segments: the DeltaNet layer's, a ragged split whose
+    bounds and lengths are no multiples of 4, and fewer rows than a tile."""
+    qm = gpu
+    g = torch.Generator(device=DEV).manual_seed(m * 7 + k)
+    for rows in ([8192, 4096, 32, 32], [600, 1, 398], [7]):
+        n = sum(rows)
+        print(f"gemm_rows {dtype} m={m} k={k} rows={rows}", flush=True)
+        w = (torch.randn(n, k, generator=g, device=DEV) * 0.02).to(dtype)
+        x = torch.randn(m, k, generator=g, device=DEV).to(dtype)
+        want = x.double() @ w.double().t()
+        got = torch.cat([o.double() for o in _gemm_rows(qm, w, x, rows)], 1)
+        bar = 2 ** -8 if dtype == BF else 1e-5
+        assert float(((got - want).abs().amax(1) / want.abs().amax(1)).max()) < bar
+
+
+@pytest.mark.parametrize("dtype,k", [(BF, 4096), (F32, 2048)])
+@pytest.mark.parametrize("m,streams", [(5, 4), (17, 4), (64, 1), (20, 10)])
+def test_gemm_rows_reinject_equals_its_two_steps(gpu, dtype, k, m, streams):
+    """qm_gemm_rows_reinject == qm_gemm_rows, then the reinjection's two
+    roundings in torch, bit for bit."""
+    qm = gpu
+    n = 2048
+    g = torch.Generator(device=DEV).manual_seed(31 * m + k + streams)
+    print(f"gemm_rows_reinject {dtype} m={m} k={k} streams={streams}", flush=True)
+    w = (torch.randn(n, k, generator=g, device=DEV) * k ** -0.5).to(dtype)
+    x = torch.randn(m, k, generator=g, device=DEV).to(dtype)
+    hyper = torch.randn(m, streams * n, generator=g, device=DEV).to(dtype)
+    inject = (2 * torch.sigmoid(torch.randn(m, streams, generator=g, device=DEV))).to(dtype)
+    branch = _gemm_rows(qm, w, x, [n])[0]
+    scaled = (branch.float()[:, None, :] * inject.float()[:, :, None]).to(dtype).float()
+    want = (hyper.float().view(m, streams, n) + scaled).to(dtype).view(m, streams * n)
+    got = hyper.clone()
+    qm.native.call("qm_gemm_rows_reinject", qm.native.act_code(dtype), m, n, k, w.data_ptr(), x.data_ptr(), streams,
+                   inject.data_ptr(), got.data_ptr(), qm.native.stream_handle())
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+
+
+def test_project_routes_by_rows(gpu):
+    """Layer projections at 5 and 64 rows (qm_gemm_rows) and at 65 (the library)
+    equal F.linear; an input that is differentiated, or not 16-byte aligned,
+    keeps F.linear."""
+    qm = gpu
+    store = gi.FakeStore(gi.dn_weights(0, 31, BF))
+    model = qm.Qwen4MixModel(qm.MixConfig(), store, device=DEV, max_ctx=256)
+    for seq in (5, 64, 65):
+        hidden = gi.normal(gi.rng(32 + seq), (1, seq, gi.HIDDEN)).to(BF).to(DEV)
+        for x in (hidden, hidden.clone().requires_grad_(),
+                  torch.cat([hidden.new_zeros(1), hidden.flatten()])[1:].view_as(hidden)):
+            got = model.project(x, 0, "dn_in")
+            assert got[0].requires_grad == x.requires_grad
+            for t, name in zip(got, model.PROJ_GROUPS["dn_in"]):
+                want = torch.nn.functional.linear(hidden.float(), store.get(f"blk.0.{name}").to(DEV).float())
+                assert rel_err(t.detach(), want, 1e-2) < 1e-2, (seq, name)

@@ -80,8 +80,8 @@ class _LayerStep:
         self.ins = [torch.empty(B, 1, r, dtype=dtype, device=dev) for r in rows_in]
         self.branch = torch.empty(B, 1, rows_out[0], dtype=dtype, device=dev)
         self.rows_in, self.rows_out = rows_in, rows_out
-        self.gemv_in = model._gemv_fits(dtype, B, c.hidden_size)
-        self.gemv_out = model._gemv_fits(dtype, B, int(self.w_out.shape[1]))
+        self.proj_in = model._proj_entry(dtype, B, c.hidden_size, len(rows_in))
+        self.proj_out = model._proj_entry(dtype, B, int(self.w_out.shape[1]), 1)
         self._seg_in = (ctypes.c_int * len(rows_in))(*rows_in)
         self._out_in = (ctypes.c_void_p * len(rows_in))(*[t.data_ptr() for t in self.ins])
         self._seg_out = (ctypes.c_int * 1)(rows_out[0])
@@ -93,9 +93,9 @@ class _LayerStep:
             self.core = DnDecodePlan(model, cache, layer, dtype)
         self.core.positions = positions
 
-    def _project(self, x, w, rows, outs, seg_rows, seg_out, use_gemv, stream):
-        if use_gemv:
-            native.call("qm_gemv", self.act, self.rows, int(w.shape[0]), int(w.shape[1]), w.data_ptr(),
+    def _project(self, x, w, rows, outs, seg_rows, seg_out, entry, stream):
+        if entry:
+            native.call(entry, self.act, self.rows, int(w.shape[0]), int(w.shape[1]), w.data_ptr(),
                         x.data_ptr(), len(rows), seg_rows, seg_out, stream)
             return
         x2 = x.view(self.rows, -1)
@@ -108,20 +108,20 @@ class _LayerStep:
         native.call("qm_hc_mix", ctypes.byref(self.hc_geom), hyper.data_ptr(), self.norm_w.data_ptr(),
                     self.w_di.data_ptr(), 1, self.w_up.data_ptr(), self.mixed.data_ptr(), self.inject.data_ptr(),
                     self.hc_ws.data_ptr(), self.hc_ws.numel(), stream)
-        self._project(self.mixed, self.w_in, self.rows_in, self.ins, self._seg_in, self._out_in, self.gemv_in, stream)
+        self._project(self.mixed, self.w_in, self.rows_in, self.ins, self._seg_in, self._out_in, self.proj_in, stream)
         if self.is_qsa:
             qg, k, v, iq, ik = self.ins
             out = self.core.run(qg, k, v, iq, ik, stream)
         else:
             qkv, z, b, a = self.ins
             out = self.core.run(qkv, z, a, b, stream)
-        if self.gemv_out:
+        if self.proj_out:
             # the output projection with the reinjection as its epilogue
-            native.call("qm_gemv_reinject", self.act, self.rows, self.rows_out[0], int(self.w_out.shape[1]),
+            native.call(self.proj_out + "_reinject", self.act, self.rows, self.rows_out[0], int(self.w_out.shape[1]),
                         self.w_out.data_ptr(), out.data_ptr(), self.hc, self.inject.data_ptr(), hyper.data_ptr(),
                         stream)
             return
-        self._project(out, self.w_out, self.rows_out, [self.branch], self._seg_out, self._out_out, False, stream)
+        self._project(out, self.w_out, self.rows_out, [self.branch], self._seg_out, self._out_out, None, stream)
         native.call("qm_hc_reinject", ctypes.byref(self.ri_geom), hyper.data_ptr(), self.branch.data_ptr(),
                     self.inject.data_ptr(), hyper.data_ptr(), stream)
 
@@ -129,7 +129,7 @@ class _LayerStep:
 class _LayerStepN:
     """One layer's token-mixing half for k consecutive tokens of one sequence
     (the captured verify step), every buffer bound: the hyper-connection mix
-    over k rows, the input projections (one GEMV launch up to 4 rows), the
+    over k rows, the input projections (one launch up to 64 rows), the
     core on its chunk path at the device position (qm_dn_prefill, or
     qm_qsa_prep + qm_qsa_select_chunk + qm_qsa_attend_chunk_filed), and the
     output projection with the reinjection as its epilogue. The same kernels
@@ -160,8 +160,8 @@ class _LayerStepN:
         self.w_out, self.rows_out = model._wcat(layer, g_out, dtype)
         self.ins = [torch.empty(1, k, r, dtype=dtype, device=dev) for r in self.rows_in]
         self.branch = torch.empty(1, k, self.rows_out[0], dtype=dtype, device=dev)
-        self.gemv_in = model._gemv_fits(dtype, k, c.hidden_size)
-        self.gemv_out = model._gemv_fits(dtype, k, int(self.w_out.shape[1]))
+        self.proj_in = model._proj_entry(dtype, k, c.hidden_size, len(self.rows_in))
+        self.proj_out = model._proj_entry(dtype, k, int(self.w_out.shape[1]), 1)
         self._seg_in = (ctypes.c_int * len(self.rows_in))(*self.rows_in)
         self._out_in = (ctypes.c_void_p * len(self.rows_in))(*[t.data_ptr() for t in self.ins])
         self._seg_out = (ctypes.c_int * 1)(self.rows_out[0])
@@ -193,9 +193,9 @@ class _LayerStepN:
                                                               ("ssm_norm.weight", torch.float32))}
             self.out = torch.empty(1, k, c.linear_value_dim, dtype=dtype, device=dev)
 
-    def _project(self, x, w, rows, outs, seg_rows, seg_out, use_gemv, stream):
-        if use_gemv:
-            native.call("qm_gemv", self.act, self.k, int(w.shape[0]), int(w.shape[1]), w.data_ptr(),
+    def _project(self, x, w, rows, outs, seg_rows, seg_out, entry, stream):
+        if entry:
+            native.call(entry, self.act, self.k, int(w.shape[0]), int(w.shape[1]), w.data_ptr(),
                         x.data_ptr(), len(rows), seg_rows, seg_out, stream)
             return
         x2 = x.view(self.k, -1)
@@ -208,7 +208,7 @@ class _LayerStepN:
         native.call("qm_hc_mix", ctypes.byref(self.hc_geom), hyper.data_ptr(), self.norm_w.data_ptr(),
                     self.w_di.data_ptr(), 1, self.w_up.data_ptr(), self.mixed.data_ptr(), self.inject.data_ptr(),
                     self.hc_ws.data_ptr(), self.hc_ws.numel(), stream)
-        self._project(self.mixed, self.w_in, self.rows_in, self.ins, self._seg_in, self._out_in, self.gemv_in, stream)
+        self._project(self.mixed, self.w_in, self.rows_in, self.ins, self._seg_in, self._out_in, self.proj_in, stream)
         lc, k, pos = self.lc, self.k, self.positions.data_ptr()
         if self.is_qsa:
             qg, kk, v, iq, ik = self.ins
@@ -232,12 +232,12 @@ class _LayerStepN:
                         w["ssm_conv1d.weight"].data_ptr(), w["ssm_norm.weight"].data_ptr(), pos,
                         lc.conv_ring.data_ptr(), lc.recurrent_state.data_ptr(), self.out.data_ptr(),
                         self.ws.data_ptr(), self.ws.numel(), stream)
-        if self.gemv_out:
-            native.call("qm_gemv_reinject", self.act, self.k, self.rows_out[0], int(self.w_out.shape[1]),
+        if self.proj_out:
+            native.call(self.proj_out + "_reinject", self.act, self.k, self.rows_out[0], int(self.w_out.shape[1]),
                         self.w_out.data_ptr(), self.out.data_ptr(), self.hc, self.inject.data_ptr(),
                         hyper.data_ptr(), stream)
             return
-        self._project(self.out, self.w_out, self.rows_out, [self.branch], self._seg_out, self._out_out, False, stream)
+        self._project(self.out, self.w_out, self.rows_out, [self.branch], self._seg_out, self._out_out, None, stream)
         native.call("qm_hc_reinject", ctypes.byref(self.ri_geom), hyper.data_ptr(), self.branch.data_ptr(),
                     self.inject.data_ptr(), hyper.data_ptr(), stream)
 
@@ -402,11 +402,11 @@ class MixDecoder:
         g = self._graphs.get(bucket)
         if g is None:
             steps = self._layer_steps(bucket)
-            if not all(st.gemv_in and st.gemv_out for st in steps):
+            if not all(st.proj_in and st.proj_out for st in steps):
                 # the library GEMMs initialise their handles on first use: not inside a capture
                 for st in steps:
                     st._project(st.mixed, st.w_in, st.rows_in, [torch.empty_like(t) for t in st.ins], None, None,
-                                False, 0)
+                                None, 0)
                 torch.cuda.synchronize(self.model.device)
             g = torch.cuda.CUDAGraph()
             side = torch.cuda.Stream(self.model.device)
@@ -477,11 +477,11 @@ class MixDecoder:
             steps = self._layer_steps_n(k)
             c = self.model.config
             rows = torch.zeros(1, k, c.hc_count * c.hidden_size, dtype=self.dtype, device=self.model.device)
-            if not all(st.gemv_in and st.gemv_out for st in steps):
+            if not all(st.proj_in and st.proj_out for st in steps):
                 # the library GEMMs initialise their handles on first use: not inside a capture
                 for st in steps:
                     st._project(st.mixed, st.w_in, st.rows_in, [torch.empty_like(t) for t in st.ins], None, None,
-                                False, 0)
+                                None, 0)
                 torch.cuda.synchronize(self.model.device)
             g = torch.cuda.CUDAGraph()
             side = torch.cuda.Stream(self.model.device)

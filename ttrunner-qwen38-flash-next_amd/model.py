@@ -102,19 +102,50 @@ class Qwen4MixModel:
         ks = (2048, 4096) if dtype == torch.bfloat16 else (1024, 2048, 4096)
         return m <= 4 and k in ks and dtype in (torch.bfloat16, torch.float32)
 
+    # rows up to which qm_gemm_rows is faster than the library's GEMMs, by dtype:
+    # for a group of projections of one input (one launch instead of four or
+    # five; DeltaNet input, us, library / here, weights from memory: bf16 45.5 /
+    # 13.8 at 16 rows, 45.5 / 33.9 at 64; float 50.8 / 31.7 at 16, 52.7 / 50.6 at
+    # 32, 59.0 / 68.0 at 48) and for a single one (output: bf16 11.8 / 6.5 at
+    # 16, 9.4 / 6.6 at 32, 9.5 / 10.6 at 48; float 12.2 / 13.2 at 5)
+    GEMM_ROWS_MAX = {torch.bfloat16: (64, 32), torch.float32: (32, 0)}
+
+    def _proj_entry(self, dtype, m: int, k: int, n_proj: int):
+        """The entry point for n_proj projections of m rows over k columns (and,
+        with ``_reinject`` appended, the output projection's): qm_gemv,
+        qm_gemm_rows, or None where the library's GEMM does it."""
+        if self._gemv_fits(dtype, m, k):
+            return "qm_gemv"
+        if not self._gemv_fits(dtype, 1, k):
+            return None
+        group, single = self.GEMM_ROWS_MAX[dtype]
+        return "qm_gemm_rows" if m <= (group if n_proj > 1 else single) else None
+
+    @staticmethod
+    def _plain_input(x: torch.Tensor, w: torch.Tensor) -> bool:
+        """Whether the product can bypass F.linear: nothing here is differentiated
+        or transformed, and the operands are aligned device memory."""
+        if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
+            return False
+        if torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0:
+            return False
+        return x.device == w.device and x.is_cuda and x.data_ptr() % 16 == 0
+
     def project(self, x: torch.Tensor, layer: int, group: str) -> list:
         """The group's projections of x [B, S, K] (F.linear with each weight), as
         a list of [B, S, rows] tensors. Up to 4 rows of x: one qm_gemv launch over
-        the concatenated weights; more: a library GEMM per projection."""
+        the concatenated weights; more (GEMM_ROWS_MAX): one qm_gemm_rows
+        launch; beyond: a library GEMM per projection."""
         dt = x.dtype
         w, rows = self._wcat(layer, group, dt)
         batch, seq, k = x.shape
-        if self._gemv_fits(dt, batch * seq, k):
-            xc = x.contiguous()
+        entry = self._proj_entry(dt, batch * seq, k, len(rows))
+        xc = x.contiguous() if entry else x
+        if entry == "qm_gemv" or (entry and self._plain_input(xc, w)):
             outs = [torch.empty(batch, seq, r, dtype=dt, device=self.device) for r in rows]
             seg_rows = (ctypes.c_int * len(rows))(*rows)
             seg_out = (ctypes.c_void_p * len(rows))(*[o.data_ptr() for o in outs])
-            native.call("qm_gemv", native.act_code(dt), batch * seq, int(w.shape[0]), k, native.ptr(w),
+            native.call(entry, native.act_code(dt), batch * seq, int(w.shape[0]), k, native.ptr(w),
                         native.ptr(xc), len(rows), seg_rows, seg_out, native.stream_handle(self.device))
             return outs
         outs, start = [], 0

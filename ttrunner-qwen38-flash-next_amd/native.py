@@ -76,6 +76,8 @@ SIGNATURES = {
     "qm_qsa_pool_blocks": (_i, [ctypes.POINTER(QsaGeom), _vp, _vp, _vp, _vp, _i, _i, _vp, _vp]),
     "qm_gemv": (_i, [_i, _i, _i, _i, _vp, _vp, _i, _vp, _vp, _vp]),
     "qm_gemv_reinject": (_i, [_i, _i, _i, _i, _vp, _vp, _i, _vp, _vp, _vp]),
+    "qm_gemm_rows": (_i, [_i, _i, _i, _i, _vp, _vp, _i, _vp, _vp, _vp]),
+    "qm_gemm_rows_reinject": (_i, [_i, _i, _i, _i, _vp, _vp, _i, _vp, _vp, _vp]),
     "qm_dn_prefill_workspace": (_sz, [ctypes.POINTER(DnGeom), _i]),
     "qm_dn_prefill": (_i, [ctypes.POINTER(DnGeom), _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                            _vp, _vp, _sz, _vp]),
