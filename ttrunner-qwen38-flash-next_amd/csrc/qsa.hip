@@ -1124,9 +1124,10 @@ __device__ void rank_topk(const unsigned long long* keys, int n, int topk, int* 
   }
 }
 
-// File one selected entry: row s of sequence b took block j as its slot-th selection.
-__device__ __forceinline__ void file_entry(uint16_t* tab, int b, int max_blocks, int seq, int j, int s, int slot) {
-  tab[((long)b * max_blocks + j) * seq + s] = static_cast<uint16_t>(slot + 1);
+// Blocks of the slot table's rows that a chunk's entries can name: those some
+// row of it may select. The rest of a table row is neither written nor read.
+__device__ __forceinline__ int table_blocks(int pos0, int seq, int ratio, int max_blocks) {
+  return min((pos0 + seq) / ratio, max_blocks);
 }
 
 // The (max, sum) pairs of a row's slot that holds no partial.
@@ -1227,22 +1228,23 @@ __device__ void select_row(const SelArgs& A, SelShared& S, int row, int b, int p
   }
   if (tid == 0) A.n_sel[row] = n_sel;
   if (A.tab) {
-    // the chunk path's slot table, as qsa_chunk_bucket_kernel fills it: every
-    // selected block files the row's slot, and the slots this row leaves
-    // empty get (max, sum) = (-inf, 0)
+    // the row of the chunk path's slot table, as qsa_chunk_bucket_kernel
+    // writes it, formed in LDS (the page list is only for items), and (max,
+    // sum) = (-inf, 0) for the slots this row leaves empty
+    uint16_t* slots = reinterpret_cast<uint16_t*>(S.pages);
+    const int nb = table_blocks(p - row % A.seq, A.seq, A.ratio, A.max_blocks);
+    for (int j = tid; j < nb; j += NT) slots[j] = 0;
     __syncthreads();
-    const int s = row % A.seq;
+    for (int i = tid; i < n_sel; i += NT) slots[S.sel[i]] = static_cast<uint16_t>(i + 1);
     const int nslot = A.topk + 1;
     for (int i = tid; i < nslot; i += NT) {
-      bool empty;
-      if (i < A.topk) {
-        empty = i >= n_sel;
-        if (!empty) file_entry(A.tab, b, A.max_blocks, A.seq, S.sel[i], s, i);
-      } else {
-        empty = ((p + 1) / A.ratio) * A.ratio > p;      // the row completes its block: no tail
-      }
+      // past the selection; the tail's slot when the row completes its block
+      const bool empty = i < A.topk ? i >= n_sel : ((p + 1) / A.ratio) * A.ratio > p;
       if (empty) empty_partial(A.part_ml, row, A.hkv, nslot, i);
     }
+    __syncthreads();
+    uint16_t* trow = A.tab + (long)row * A.max_blocks;
+    for (int j = tid; j < nb; j += NT) trow[j] = slots[j];
   }
   if (!A.items) return;
   __syncthreads();
@@ -1648,10 +1650,6 @@ template <typename T, typename PO = float>
 struct CombineArgs {
   const PO* part_o; const float* part_ml; const T* qg; T* out;
   int hq, hkv, splits;
-  // the chunk path's slot table, cleared here once the attention has read
-  // it: its length in 16-byte words
-  uint16_t* tab = nullptr;
-  long tab_words = 0;
 };
 
 __device__ __forceinline__ float part_value(const float* p, long i) { return p[i]; }
@@ -1669,12 +1667,6 @@ __global__ __launch_bounds__(QSA_D) void qsa_combine_kernel(CombineArgs<T, PO> A
   __shared__ float s_w[MAX_SPLITS];
   __shared__ float s_red[QSA_D / 64];
   const float gate = Act<T>::load(A.qg, ((long)row * A.hq + hq) * (2 * QSA_D) + QSA_D + d);
-  if (A.tab) {
-    // each workgroup clears 4 KB stretches of the table, spread over the grid
-    const long wg = blockIdx.x + (long)gridDim.x * blockIdx.y, n_wg = (long)gridDim.x * gridDim.y;
-    for (long w = wg * QSA_D + d; w < A.tab_words; w += n_wg * QSA_D)
-      reinterpret_cast<u32x4_t*>(A.tab)[w] = u32x4_t{0u, 0u, 0u, 0u};
-  }
   // every split's (max, sum) in parallel, then the weights in LDS
   float m = -INFINITY, l = 0.f;
   for (int s = d; s < A.splits; s += QSA_D) {
@@ -1721,18 +1713,21 @@ __global__ __launch_bounds__(QSA_D) void qsa_combine_kernel(CombineArgs<T, PO> A
 // The attention of a chunk of query rows reads each key/value block once. A
 // row's entries are its (row, slot) pairs: slot i < n_sel its i-th selected
 // block, slot topk its tail block (keys ts..p, when the row does not complete
-// its block). The entries are filed in a slot table, [B][max_blocks][seq]
-// uint16 in the workspace: entry (b, j, s) holds slot + 1 when row s selected
-// block j, else 0. Plain stores fill it (no atomics, so no round trip holds up
-// the filing), the attention reads a block's row of it, and the merge clears
-// it, so every call leaves the table zero. qm_qsa_attend_chunk is three
+// its block). The entries are filed in a slot table, [B][seq][max_blocks]
+// uint16 in the workspace: entry (b, s, j) holds slot + 1 when row s selected
+// block j, else 0. Each row writes its whole row of the table (plain stores, no
+// atomics, so no round trip holds up the filing), and the attention gathers a
+// block's column of it. Nothing is kept in it between calls: a table that the
+// calls left zero for one another ([max_blocks][seq], cleared by the merge) lay
+// under the partials of shorter chunks on the same workspace, whose bits the
+// next longer chunk then read as slots. qm_qsa_attend_chunk is three
 // launches:
-//   qsa_chunk_bucket   one 64-thread workgroup per row: files the row's
-//                      selected entries and writes the empty partials (max
+//   qsa_chunk_bucket   one 64-thread workgroup per row: writes the row's table
+//                      row and writes the empty partials (max
 //                      -inf) of its unused slots (qm_qsa_select_chunk does the
 //                      same inside the selection);
 //   qsa_chunk_attend   grid (blocks + tail workgroups, kv head, sequence): the
-//                      workgroup of block j reads its table row and the page
+//                      workgroup of block j reads its table column and the page
 //                      with its first loads, then the block's 64 tokens of key
 //                      pieces straight into LDS (16 KB per 32 tokens) and of
 //                      value pieces into registers; each wave scores two
@@ -1745,10 +1740,9 @@ __global__ __launch_bounds__(QSA_D) void qsa_combine_kernel(CombineArgs<T, PO> A
 //                      workgroup takes the tail entries of 8 rows (one or two
 //                      blocks), which would otherwise pile onto two blocks'
 //                      workgroups;
-//   qsa_combine        merges a row's topk + 1 slots, applies the gate and
-//                      clears the slot table.
-// The workspace is zero-filled before its first use; the selection (or the
-// bucket kernel) and the attention of one call use the same seq.
+//   qsa_combine        merges a row's topk + 1 slots and applies the gate.
+// The selection (or the bucket kernel) and the attention of one call use the
+// same seq.
 constexpr int CA_MAX_BLOCKS = 4096;
 constexpr int CA_NT = 256;        // attention workgroup: four waves
 constexpr int CA_TAIL_ROWS = 8;   // rows per tail workgroup
@@ -1774,12 +1768,17 @@ __global__ __launch_bounds__(64) void qsa_chunk_bucket_kernel(ChunkBucketArgs A)
   const int b = row / A.seq, s = row % A.seq;
   const int nslot = A.topk + 1;
   const int nsel = A.n_sel[row];
-  const int p = A.positions[b] + s;
+  const int pos0 = A.positions[b], p = pos0 + s;
+  // the whole row, then its entries behind a barrier
+  uint16_t* trow = A.tab + (long)row * A.max_blocks;
+  const int nb = table_blocks(pos0, A.seq, A.ratio, A.max_blocks);
+  for (int j = lane; j < nb; j += 64) trow[j] = 0;
+  __syncthreads();
   for (int i = lane; i < nslot; i += 64) {
     bool empty;
     if (i < A.topk) {
       empty = i >= nsel;
-      if (!empty) file_entry(A.tab, b, A.max_blocks, A.seq, A.ids[(long)row * A.topk + i], s, i);
+      if (!empty) trow[A.ids[(long)row * A.topk + i]] = static_cast<uint16_t>(i + 1);
     } else {
       empty = ((p + 1) / A.ratio) * A.ratio > p;      // the row completes its block: no tail
     }
@@ -2036,18 +2035,19 @@ __global__ __launch_bounds__(CA_NT, 4) void qsa_chunk_attend_kernel(ChunkAttnArg
     // ---- block j = x: the first 128 rows of its table row, its pages and
     // the position in one round trip; then its entries in groups of 8
     const int j = x;
-    const uint16_t* trow = A.tab + ((long)b * A.max_blocks + j) * A.seq;
-    const int ta = lane < A.seq ? trow[lane] : 0;
-    const int tb = 64 + lane < A.seq ? trow[64 + lane] : 0;
+    const uint16_t* tcol = A.tab + row_b * A.max_blocks + j;     // row s's entry for this block at s * max_blocks
+    const int ta = lane < A.seq ? tcol[(long)(lane) * A.max_blocks] : 0;
+    const int tb = 64 + lane < A.seq ? tcol[(long)(64 + lane) * A.max_blocks] : 0;
     int page0, page1;
     pages_of(j, page0, page1);
     const int pos0 = A.positions[b];
+    if (j >= table_blocks(pos0, A.seq, A.ratio, A.max_blocks)) return;     // past every row's blocks: no entries
     bool loaded = false, first = true;
     for (int c = 0; 128 * c < A.seq; ++c) {
       // rows 128 c + lane and 128 c + 64 + lane of the table row
       const int ra = 128 * c + lane, rb = ra + 64;
-      const int tva = c == 0 ? ta : ra < A.seq ? trow[ra] : 0;
-      const int tvb = c == 0 ? tb : rb < A.seq ? trow[rb] : 0;
+      const int tva = c == 0 ? ta : ra < A.seq ? tcol[(long)ra * A.max_blocks] : 0;
+      const int tvb = c == 0 ? tb : rb < A.seq ? tcol[(long)rb * A.max_blocks] : 0;
       unsigned long long la = __ballot(tva != 0), lb = __ballot(tvb != 0);
       if ((la | lb) == 0ull) continue;
       const int nc = __popcll(la) + __popcll(lb);
@@ -3430,8 +3430,8 @@ struct ChunkWs {
   size_t tab, tab_bytes, o, ml, total;
 };
 
-// the slot table first: every call leaves it zero, so a workspace sized for
-// a longer chunk serves a shorter one
+// nothing in it outlives a call, so one workspace serves chunks of any length
+// that fit it, in any order
 ChunkWs chunk_ws_layout(const qm_qsa_geom* g, int seq) {
   const int nslot = g->budget / g->ratio + 1;
   const size_t rows = (size_t)g->batch * seq;
@@ -3508,11 +3508,11 @@ int attend_chunk(const qm_qsa_geom* g, int seq, const void* q, const void* qg, c
   QM_CHECK_LAUNCH();
   if (g->act_dtype == QM_ACT_F32) {
     CombineArgs<float, uint16_t> C{part_o, part_ml, static_cast<const float*>(qg), static_cast<float*>(out), g->n_heads,
-                         g->n_kv_heads, nslot, tab, (long)(L.tab_bytes / 16)};
+                         g->n_kv_heads, nslot};
     hipLaunchKernelGGL((qsa_combine_kernel<float, uint16_t>), dim3(g->n_heads, g->batch * seq), dim3(QSA_D), 0, stream, C);
   } else {
     CombineArgs<bf16_t, uint16_t> C{part_o, part_ml, static_cast<const bf16_t*>(qg), static_cast<bf16_t*>(out), g->n_heads,
-                          g->n_kv_heads, nslot, tab, (long)(L.tab_bytes / 16)};
+                          g->n_kv_heads, nslot};
     hipLaunchKernelGGL((qsa_combine_kernel<bf16_t, uint16_t>), dim3(g->n_heads, g->batch * seq), dim3(QSA_D), 0, stream, C);
   }
   QM_CHECK_LAUNCH();

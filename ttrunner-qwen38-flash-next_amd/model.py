@@ -384,8 +384,7 @@ class Qwen4MixModel:
                     native.ptr(lc.raw_keys), native.ptr(lc.block_keys), native.ptr(q_out), native.ptr(iq_out),
                     stream)
         if chunked:
-            # the chunk attention's own workspace per geometry: the entry
-            # counts it keeps between calls are laid out by batch and block count
+            # the chunk attention's workspace; nothing in it outlives a call
             chunk_ws = self._workspace(f"qsa_attend_chunk_{batch}_{cache.max_blocks}",
                                        lib.qm_qsa_attend_chunk_workspace(ctypes.byref(g), seq))
         if chunked and self.fuse_chunk_select:
