@@ -50,3 +50,23 @@ def test_chunks_of_different_lengths_share_a_workspace(gpu):
         torch.cuda.synchronize()
         assert torch.equal(got, want), (seq, pos)
         pos += seq
+
+
+def test_decode_plans_of_different_sizes_share_a_workspace(gpu):
+    """One layer's eager decode at positions whose plans have 66, 35, 66, 12 and
+    66 items, on one workspace: the flags of a longer plan must not lie under a
+    shorter plan's partials."""
+    (shared, c0), (fresh, c1) = _pair(gpu, 4096)
+    gen = torch.Generator(device=DEV).manual_seed(6)
+    x = _inputs(gen, 2560)
+    for model, cache in ((shared, c0), (fresh, c1)):
+        model.qsa_core(*x, LAYER, cache, 0)
+    for pos in (2500, 1100, 2500, 380, 2500, 1100, 2500):
+        print(f"decode at {pos}", flush=True)
+        x = _inputs(gen, 1)
+        got = shared.qsa_core(*x, LAYER, c0, pos)
+        fresh._ws.clear()
+        want = fresh.qsa_core(*x, LAYER, c1, pos)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want), pos
+    shared.check_handoffs()

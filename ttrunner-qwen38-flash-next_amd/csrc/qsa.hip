@@ -2258,7 +2258,11 @@ struct ItemCount {
 };
 
 // flags of a group: one per workgroup that attends an item or holds a slice
-__host__ __device__ inline int dec_flag_stride(int splits) { return splits > DEC_SLICES ? splits : DEC_SLICES; }
+// The flags of a group, at one stride for every plan: the flags outlive a
+// launch, and at a stride of the plan's own splits a shorter plan's partials lay
+// over a longer one's flags on the same workspace (a (max, sum) word read as a
+// raised flag lets a merge take stale partials).
+constexpr int DEC_FLAG_STRIDE = DEC_MAX_ITEMS;
 
 // Flags of the 128 items of round i0, polled by one wave (the caller's wave
 // 0; its workgroup waits at a barrier): lane l polls items i0 + l and
@@ -2304,7 +2308,7 @@ __device__ void decode_combine_slice(const DecArgs<T>& D, DecShared& sh, int b, 
   const int c = tid & 3, il = tid >> 2;
   const int h = sl / 8, d0 = 32 * (sl % 8) + 8 * c;
   const int bg = b * D.P.hkv + g;
-  const unsigned* flags = D.flags + (long)bg * dec_flag_stride(D.splits);
+  const unsigned* flags = D.flags + (long)bg * DEC_FLAG_STRIDE;
   float M = -INFINITY, L = 0.f, acc[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc[e] = 0.f;
@@ -2540,7 +2544,7 @@ __global__ __launch_bounds__(DEC_NT) void qsa_decode_kernel(const int* positions
     if constexpr (WIDE) {
       // a slice holder past the items: flag raised once the word is read
       if (item < DEC_SLICES) {
-        if (tid == 0) raise_flag(D.flags + (long)bg * dec_flag_stride(D.splits) + item, gen + 1);
+        if (tid == 0) raise_flag(D.flags + (long)bg * DEC_FLAG_STRIDE + item, gen + 1);
         decode_merge<WIDE>(D, sh, b, g, item, n_att, gen, overflow);
       }
     }
@@ -2777,7 +2781,7 @@ __global__ __launch_bounds__(DEC_NT) void qsa_decode_kernel(const int* positions
   wait_all_memory();
   __syncthreads();
   QM_PHASE(8);
-  if (tid == 0) post_flag(D.flags + (long)bg * dec_flag_stride(D.splits) + item, gen + 1);
+  if (tid == 0) post_flag(D.flags + (long)bg * DEC_FLAG_STRIDE + item, gen + 1);
 
   // the stores that outlive this step, after the flag (no merge waits for
   // them; the launch's end does): the token's key/value into its page slot
@@ -3638,8 +3642,8 @@ namespace {
 size_t dec_gen_bytes(const qm_qsa_geom* g) {
   return qm_align256((size_t)g->batch * g->n_kv_heads * DEC_GEN_STRIDE * sizeof(unsigned));
 }
-size_t dec_flag_bytes(const qm_qsa_geom* g, int splits) {
-  return qm_align256((size_t)g->batch * g->n_kv_heads * dec_flag_stride(splits) * sizeof(unsigned));
+size_t dec_flag_bytes(const qm_qsa_geom* g) {
+  return qm_align256((size_t)g->batch * g->n_kv_heads * DEC_FLAG_STRIDE * sizeof(unsigned));
 }
 size_t dec_ml_bytes(const qm_qsa_geom* g, int splits) {
   return qm_align256((size_t)g->batch * g->n_kv_heads * splits * GQA * 2 * sizeof(float));
@@ -3704,13 +3708,13 @@ extern "C" int qm_qsa_decode_check(const qm_qsa_geom* g, int splits, void* works
   delete[] host;
   if (!reset) return QM_OK;
   // generation words, counters and flags back to zero: the state of a fresh workspace
-  const size_t words = (dec_gen_bytes(g) + dec_flag_bytes(g, splits)) / sizeof(unsigned);
+  const size_t words = (dec_gen_bytes(g) + dec_flag_bytes(g)) / sizeof(unsigned);
   return qm_zero_words(workspace, (long)words, stream);
 }
 
 extern "C" size_t qm_qsa_decode_workspace(const qm_qsa_geom* g, int splits) {
   if (!g || splits <= 0) return 0;
-  return dec_gen_bytes(g) + dec_flag_bytes(g, splits) + dec_ml_bytes(g, splits) + dec_o_bytes(g, splits);
+  return dec_gen_bytes(g) + dec_flag_bytes(g) + dec_ml_bytes(g, splits) + dec_o_bytes(g, splits);
 }
 
 extern "C" int qm_qsa_decode(const qm_qsa_geom* g, const void* qg, const void* k_new, const void* v_new, const void* iq,
@@ -3764,8 +3768,8 @@ extern "C" int qm_qsa_decode(const qm_qsa_geom* g, const void* qg, const void* k
   rc = qm_qsa_decode_fits(splits, resident);
   if (rc) return rc;
   unsigned* flags = reinterpret_cast<unsigned*>(ws + dec_gen_bytes(g));
-  float* part_ml = reinterpret_cast<float*>(ws + dec_gen_bytes(g) + dec_flag_bytes(g, splits));
-  uint16_t* part_o = reinterpret_cast<uint16_t*>(ws + dec_gen_bytes(g) + dec_flag_bytes(g, splits) + dec_ml_bytes(g, splits));
+  float* part_ml = reinterpret_cast<float*>(ws + dec_gen_bytes(g) + dec_flag_bytes(g));
+  uint16_t* part_o = reinterpret_cast<uint16_t*>(ws + dec_gen_bytes(g) + dec_flag_bytes(g) + dec_ml_bytes(g, splits));
   const bool wide = splits < DEC_SLICES;
   const dim3 grid(wide ? DEC_SLICES : splits, g->n_kv_heads, g->batch);
   auto run = [&](auto* tag) -> int {
