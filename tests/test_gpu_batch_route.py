@@ -1,0 +1,65 @@
+"""The route of a QSA decode batch: plans of up to 8 sequences (5 with the
+selection on, and 640 scored blocks in all) run in one launch, larger ones as
+prep + select + attend; both give the same step, and bind() takes either."""
+
+from __future__ import annotations
+
+import os
+import sys
+from importlib import import_module
+
+import pytest
+import torch
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden"))
+import inputs as gi  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+LAYER = 3
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("batch,pos,one_launch", [(5, 2500, True), (6, 2500, False), (8, 700, True), (9, 700, False),
+                                                  (9, 200, False)])
+def test_batch_routes_agree(gpu, dtype, batch, pos, one_launch):
+    """Outputs of the two routes within the decode tests' 2e-2 of the largest
+    value, the appended keys and values bit for bit."""
+    qm = gpu
+    plan = import_module(qm.__name__ + ".plan")
+    print(f"decode batch {batch} at {pos} {dtype}", flush=True)
+    model = qm.Qwen4MixModel(qm.MixConfig(), gi.FakeStore(gi.qsa_weights(LAYER, 90, dtype)), device=DEV, max_ctx=4096)
+    gen = torch.Generator(device=DEV).manual_seed(batch + pos)
+    r = lambda *s: torch.randn(*s, generator=gen, device=DEV).to(dtype)  # noqa: E731
+    past = [r(batch, pos, n) for n in (16 * 512, 512, 512, 512, 128)]
+    x = [r(batch, 1, n) for n in (16 * 512, 512, 512, 512, 128)]
+    rows = torch.tensor([max(1, pos - 70 * i) for i in range(batch)], dtype=torch.int32)
+    outs, caches = [], []
+    for fused in (None, not one_launch):
+        cache = qm.MixHybridCache(LAYER + 1, model.config, batch, 4096, DEV, dtype, page_table="random", seed=4)
+        model.qsa_core(*past, LAYER, cache, 0)
+        p = plan.QsaDecodePlan(model, cache, LAYER, pos, dtype, fused=fused)
+        assert p.fused == (one_launch if fused is None else fused)
+        p.positions.copy_(rows)
+        if fused is None:
+            p.bind(*x)(qm.native.stream_handle())
+        else:
+            p.run(*x)
+        torch.cuda.synchronize()
+        assert p.check() == []
+        outs.append(p.out.float().clone())
+        caches.append(cache[LAYER])
+    assert float((outs[0] - outs[1]).abs().max() / outs[1].abs().max()) < 2e-2
+    assert torch.equal(caches[0].k_pool, caches[1].k_pool) and torch.equal(caches[0].v_pool, caches[1].v_pool)
+
+
+def test_bind_refuses_what_one_sequence_refuses(gpu):
+    """A plan whose position alone is past the one-launch decode stays refused."""
+    qm = gpu
+    plan = import_module(qm.__name__ + ".plan")
+    model = qm.Qwen4MixModel(qm.MixConfig(), gi.FakeStore(gi.qsa_weights(LAYER, 90, torch.bfloat16)), device=DEV)
+    cache = qm.MixHybridCache(LAYER + 1, model.config, 1, 49152, DEV)
+    p = plan.QsaDecodePlan(model, cache, LAYER, 45000)
+    x = [torch.zeros(1, 1, n, dtype=torch.bfloat16, device=DEV) for n in (16 * 512, 512, 512, 512, 128)]
+    with pytest.raises(qm.native.QmError):
+        p.bind(*x)

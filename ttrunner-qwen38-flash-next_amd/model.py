@@ -436,21 +436,33 @@ class Qwen4MixModel:
         return (c.indexer_compress_ratio in (32, 64) and cache.max_blocks <= 4096
                 and cache.max_ctx <= 4096 * c.indexer_compress_ratio and c.block_topk <= 510)
 
-    # Up to this many eligible blocks the one-launch decode is the faster path:
-    # each of its workgroups scores and ranks every eligible block itself, so
-    # its time grows with the context (cold, MI355X: 11.0 us at 127 blocks,
-    # 25.3 at 511, 36.8 at 1023, 60.6 at 2047), while prep + the scores spread
-    # over the blocks + the ranking + the attention stay near 28-35 us.
+    # Up to this many eligible blocks, over all sequences of the batch, the
+    # one-launch decode is the faster path: each of its workgroups scores and
+    # ranks every eligible block of its sequence itself, so its time grows with
+    # the context (one sequence, cold, MI355X: 11.0 us at 127 blocks, 25.3 at
+    # 511, 36.8 at 1023, 60.6 at 2047), while prep + the scores spread over the
+    # blocks + the ranking + the attention stay near 28-35 us. A batch
+    # multiplies the workgroups too, past what the device holds at once (us, one
+    # launch / split path: 312 blocks 26 / 23 for 2 sequences, 58 / 28 for 8,
+    # 162 / 44 for 24; 127 blocks 20 / 25 for 4, 36 / 29 for 8, 190 / 69 for 48).
     FUSED_MAX_BLOCKS = 640
+    # ... and up to this many sequences, with the selection on (62 blocks: 20 /
+    # 23 for 4, 35 / 28 for 8) and off (31 blocks: 22 / 24 for 8, 43 / 30 for
+    # 16; 4 blocks: 12 / 20 for 4, 22 / 21 for 8, 122 / 25 for 48)
+    FUSED_MAX_BATCH_SCORED, FUSED_MAX_BATCH = 5, 8
 
-    def fused_decode_fits(self, cache, max_position=None) -> bool:
+    def fused_decode_fits(self, cache, max_position=None, batch=None) -> bool:
         """Whether qm_qsa_decode covers this cache's geometry (and, given a
-        position, whether it is the faster path there)."""
+        position, whether it is the faster path there for ``batch`` sequences,
+        default the cache's)."""
         c = self.config
         fits = (cache.max_blocks <= 2048 and cache.max_pages <= 2048 and c.block_topk <= 256
                 and c.indexer_compress_ratio <= 64)
         if max_position is not None:
-            fits = fits and (max_position + 1) // c.indexer_compress_ratio <= self.FUSED_MAX_BLOCKS
+            batch = cache.batch if batch is None else batch
+            blocks = (max_position + 1) // c.indexer_compress_ratio
+            most = self.FUSED_MAX_BATCH if blocks <= c.block_topk else self.FUSED_MAX_BATCH_SCORED
+            fits = fits and batch * blocks <= self.FUSED_MAX_BLOCKS and batch <= most
         return fits
 
     def decode_group_fits(self, splits: int, dtype) -> bool:

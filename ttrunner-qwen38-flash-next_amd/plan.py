@@ -38,6 +38,17 @@ class BoundCall:
             raise native.QmError(f"{self.name} failed ({rc}): {native.load().qm_last_error().decode(errors='replace')}")
 
 
+class BoundCalls:
+    """Several BoundCalls launched in order."""
+
+    def __init__(self, *calls: BoundCall):
+        self.calls = calls
+
+    def __call__(self, stream: int) -> None:
+        for c in self.calls:
+            c(stream)
+
+
 class DnDecodePlan:
     """One DeltaNet decode step of ``layer`` for a ``batch``-row cache."""
 
@@ -104,6 +115,8 @@ class QsaDecodePlan:
         if fused and not can_fuse:
             raise native.QmError(f"layer {layer}: this geometry does not fit one qm_qsa_decode launch")
         self.fused = (can_fuse and faster) if fused is None else bool(fused)
+        # one sequence here would run in one launch; the batch is what makes the split path the faster one
+        self.batched = fused is None and can_fuse and not faster and model.fused_decode_fits(cache, max_position, 1)
         # the other path: prep, the scores spread over the blocks, the ranking,
         # and the attention (the scores' buffer makes qm_qsa_select split them)
         self.scores = None if self.fused else torch.empty(batch, 1, cache.max_blocks, dtype=torch.float32,
@@ -134,27 +147,34 @@ class QsaDecodePlan:
                     self.iq_out.data_ptr(), self.ids.data_ptr(), self.n_sel.data_ptr(), self.items.data_ptr(),
                     stream)
 
-    def prep(self, qg, k, v, iq, ik, stream):
+    def _prep_args(self, qg, k, v, iq, ik):
         lc, w = self.lc, self.w
-        native.call("qm_qsa_prep", ctypes.byref(self.geom), 1, qg.data_ptr(), k.data_ptr(), v.data_ptr(),
-                    iq.data_ptr(), ik.data_ptr(), w["attn_q_norm.weight"].data_ptr(),
-                    w["attn_k_norm.weight"].data_ptr(), w["indexer.q_norm.weight"].data_ptr(),
-                    w["indexer.k_norm.weight"].data_ptr(), self.cos.data_ptr(), self.sin.data_ptr(),
-                    self.positions.data_ptr(), lc.page_table.data_ptr(), lc.k_pool.data_ptr(),
-                    lc.v_pool.data_ptr(), lc.raw_keys.data_ptr(), lc.block_keys.data_ptr(), self.q_out.data_ptr(),
-                    self.iq_out.data_ptr(), stream)
+        return (ctypes.byref(self.geom), 1, qg.data_ptr(), k.data_ptr(), v.data_ptr(), iq.data_ptr(), ik.data_ptr(),
+                w["attn_q_norm.weight"].data_ptr(), w["attn_k_norm.weight"].data_ptr(),
+                w["indexer.q_norm.weight"].data_ptr(), w["indexer.k_norm.weight"].data_ptr(), self.cos.data_ptr(),
+                self.sin.data_ptr(), self.positions.data_ptr(), lc.page_table.data_ptr(), lc.k_pool.data_ptr(),
+                lc.v_pool.data_ptr(), lc.raw_keys.data_ptr(), lc.block_keys.data_ptr(), self.q_out.data_ptr(),
+                self.iq_out.data_ptr())
+
+    def _select_args(self):
+        return (ctypes.byref(self.geom), 1, self.iq_out.data_ptr(), self.lc.block_keys.data_ptr(),
+                self.positions.data_ptr(), self.lc.page_table.data_ptr(), self.ids.data_ptr(),
+                self.n_sel.data_ptr(), self.items.data_ptr(), None if self.scores is None else self.scores.data_ptr())
+
+    def _attend_args(self, qg):
+        lc = self.lc
+        return (ctypes.byref(self.geom), 1, self.q_out.data_ptr(), qg.data_ptr(), lc.k_pool.data_ptr(),
+                lc.v_pool.data_ptr(), self.items.data_ptr(), self.out.data_ptr(), self.splits, self.ws.data_ptr(),
+                self.ws.numel())
+
+    def prep(self, qg, k, v, iq, ik, stream):
+        native.call("qm_qsa_prep", *self._prep_args(qg, k, v, iq, ik), stream)
 
     def select(self, stream):
-        native.call("qm_qsa_select", ctypes.byref(self.geom), 1, self.iq_out.data_ptr(),
-                    self.lc.block_keys.data_ptr(), self.positions.data_ptr(), self.lc.page_table.data_ptr(),
-                    self.ids.data_ptr(), self.n_sel.data_ptr(), self.items.data_ptr(),
-                    None if self.scores is None else self.scores.data_ptr(), stream)
+        native.call("qm_qsa_select", *self._select_args(), stream)
 
     def attend(self, qg, stream):
-        lc = self.lc
-        native.call("qm_qsa_attend", ctypes.byref(self.geom), 1, self.q_out.data_ptr(), qg.data_ptr(),
-                    lc.k_pool.data_ptr(), lc.v_pool.data_ptr(), self.items.data_ptr(), self.out.data_ptr(),
-                    self.splits, self.ws.data_ptr(), self.ws.numel(), stream)
+        native.call("qm_qsa_attend", *self._attend_args(qg), stream)
 
     def _decode_args(self, qg, k, v, iq, ik):
         lc, w = self.lc, self.w
@@ -169,9 +189,14 @@ class QsaDecodePlan:
         """The whole step in one qm_qsa_decode launch."""
         native.call("qm_qsa_decode", *self._decode_args(qg, k, v, iq, ik), stream)
 
-    def bind(self, qg, k, v, iq, ik) -> BoundCall:
-        """The one-launch step on these inputs as a BoundCall (stream at call
-        time); plans that do not fit one launch are refused."""
+    def bind(self, qg, k, v, iq, ik):
+        """The step on these inputs as a BoundCall (stream at call time), or, where
+        the batch makes the split path the faster one, as its three; plans whose
+        position does not fit one launch are refused."""
+        if self.batched:
+            return BoundCalls(BoundCall("qm_qsa_prep", *self._prep_args(qg, k, v, iq, ik)),
+                              BoundCall("qm_qsa_select", *self._select_args()),
+                              BoundCall("qm_qsa_attend", *self._attend_args(qg)))
         if not self.fused:
             raise native.QmError(f"layer {self.layer}: this plan runs as prep + select + attend, not one launch")
         return BoundCall("qm_qsa_decode", *self._decode_args(qg, k, v, iq, ik))
