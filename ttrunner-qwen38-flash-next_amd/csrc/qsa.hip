@@ -878,14 +878,11 @@ __device__ void score_blocks_seq(const float* __restrict__ iq_row, const float* 
 // number of larger keys). `keys` is padded with zeros (below every real key) to
 // a multiple of 32. Up to 128 keys (n <= NT/2), by counting: two adjacent lanes
 // split the comparisons of one key and add their counts by DPP. Beyond, by
-// a threshold from one histogram over the keys' own range: the upper 32 bits
-// (the score) of every key go into 256 equal buckets between their minimum and
-// maximum (integer arithmetic, so the bucket is monotone in the key), a suffix
-// scan finds the bucket that holds the topk-th largest key, and the keys in it
-// and above (typically topk plus a few) are gathered and ranked among
-// themselves by counting (1024-thread workgroups; the 256-thread decode
-// kernels keep their code small and go straight to radix select). When more
-// than RANK_CAND keys share that bucket
+// a threshold from one histogram over the scores' own range: every key's score
+// goes into 256 equal buckets between the least and the largest, a suffix scan
+// finds the bucket that holds the topk-th largest key, and the keys in it and
+// above (typically topk plus a few) are gathered and ranked among themselves
+// by counting. When more than RANK_CAND keys share that bucket
 // (many equal or clustered scores), radix select instead: eight passes of an
 // 8-bit histogram (LDS atomics, then a suffix scan over the 256 digits) pin the
 // topk-th largest key T exactly, the keys >= T are gathered, and only they are
@@ -922,13 +919,21 @@ __device__ __forceinline__ int wave_incl_sum(int x) {
   return x + (row >= 1 ? r0 : 0) + (row >= 2 ? r1 : 0) + (row >= 3 ? r2 : 0);
 }
 
+// The score of a key's upper word (sel_key). Scores are sums of relus, so a
+// word below 0x80000000 is a negative zero.
+__device__ __forceinline__ float key_score(unsigned u) {
+  return u & 0x80000000u ? __uint_as_float(u & 0x7fffffffu) : 0.f;
+}
+
 // The bucket threshold (above). Returns false, having written nothing to sel,
-// when more than RANK_CAND keys are at or above the threshold bucket. The
-// bucket of a key is ((score bits - min) * mul) >> 32 with width = max - min +
-// 1 and mul = 2^40 / width rounded down with a relative margin of 2^-20 (a
-// single-precision quotient, whose rounding the margin covers): monotone in the
-// key and below 256. Waves exchange partial results through LDS only at the
-// four barriers; within a wave, DPP and lane reads.
+// when more than RANK_CAND keys are at or above the threshold bucket, or the
+// scores have no range. The bucket of a key is floor((score - min) * 255.99 /
+// (max - min)), each step monotone in the score under rounding. Buckets equal
+// in the score, not in its bits: among the bits of floats from 0 up, nearly
+// every score shares the top few of 256, and a row of 2047 blocks went on to
+// radix select (13.6 us for the ranking of such a row, 6.4 now). Waves
+// exchange partial results through LDS only at the four barriers; within a
+// wave, DPP and lane reads.
 // Each wave's range of the keys' score bits to wtot (lows, then highs), and
 // the histogram and counters cleared: the first pass of bucket_topk, which a
 // caller that forms the keys itself (lo / hi over its own keys) runs before
@@ -965,11 +970,11 @@ __device__ bool bucket_topk(const unsigned long long* keys, int n, int topk, int
   QM_PHASE(6);
   const unsigned glo = wave_minmax_u<false>(lane < NW ? static_cast<unsigned>(wtot[lane]) : 0xffffffffu);
   const unsigned ghi = wave_minmax_u<true>(lane < NW ? static_cast<unsigned>(wtot[16 + lane]) : 0u);
-  const float width = static_cast<float>(ghi - glo) + 1.0f;
-  const unsigned long long mul =
-      static_cast<unsigned long long>(1099511627776.0f * (1.0f - 9.5367431640625e-07f) / width);
+  const float lo_s = key_score(glo), width = key_score(ghi) - lo_s;
+  if (!(width > 1e-30f && width < 1e30f)) return false;      // one score, or infinities and NaN among them
+  const float mul = 255.99f / width;
   auto bucket = [&](unsigned long long k) {
-    return static_cast<int>((static_cast<unsigned long long>(static_cast<unsigned>(k >> 32) - glo) * mul) >> 32);
+    return min(255, static_cast<int>((key_score(static_cast<unsigned>(k >> 32)) - lo_s) * mul));
   };
   for (int j = tid; j < n; j += NT) atomicAdd(&hist[bucket(keys[j])], 1);
   __syncthreads();                        // every wave has read the range: wtot is free
@@ -1069,8 +1074,7 @@ __device__ void rank_topk(const unsigned long long* keys, int n, int topk, int* 
   int* state = scr + 256 + 32;            // prefix lo, prefix hi, remaining, count
   int* cand = scr + 256 + 40;             // [topk]
   const int lane = tid & 63, wv = tid >> 6;
-  if constexpr (NT >= 1024)
-    if (topk <= RANK_CAND && bucket_topk<NT>(keys, n, topk, sel, hist, wtot, state, cand, range_in)) return;
+  if (topk <= RANK_CAND && bucket_topk<NT>(keys, n, topk, sel, hist, wtot, state, cand, range_in)) return;
   unsigned long long prefix = 0ull;
   int r = topk;
   for (int shift = 56; shift >= 0; shift -= 8) {
@@ -1151,22 +1155,28 @@ struct SelArgs {
   const float* scores_in = nullptr;
 };
 
-struct SelShared {
+// LDS of a row's ranking over at most MAXB blocks
+template <int MAXB>
+struct RankShared {
+  static constexpr int MAXK = MAXB / 2;
+  unsigned long long key[MAXB];
+  int pages[MAXB];
+  int sel[MAXK];
+  alignas(16) int rscr[rank_scratch(MAXK)];
+};
+struct SelShared : RankShared<SEL_MAX_BLOCKS> {
   float q[4 * IDX_D];
   float dsc[4][SELP_NT / 4];            // a scoring round's relu'd dot products (several-rows order)
   float newkey[IDX_D];
-  unsigned long long key[SEL_MAX_BLOCKS];
-  int pages[SEL_MAX_BLOCKS];
-  int sel[SEL_MAX_BLOCKS / 2];
-  alignas(16) int rscr[rank_scratch(SEL_MAX_BLOCKS / 2)];
 };
 
 // Selection for one query row at position p, by a whole SEL_NT-thread block.
 // The indexer query must already be in S.q (heads past idx_heads zero). Block
 // keys come from the cache, except block new_j (>= 0 when this very launch
 // completed it), whose key is in S.newkey.
-template <int NT>
-__device__ void select_row(const SelArgs& A, SelShared& S, int row, int b, int p, int new_j, float* stage) {
+// SCORED: the scores come from A.scores_in (S is then a RankShared alone).
+template <int NT, bool SCORED, typename SH>
+__device__ void select_row(const SelArgs& A, SH& S, int row, int b, int p, int new_j, float* stage) {
   const int tid = threadIdx.x;
   const int n_elig = min((p + 1) / A.ratio, A.max_blocks);
   const int n_sel = min(n_elig, A.topk);
@@ -1181,7 +1191,7 @@ __device__ void select_row(const SelArgs& A, SelShared& S, int row, int b, int p
       if (j >= n_elig) A.scores_out[(long)row * A.max_blocks + j] = -INFINITY;
 
   bool range_in = false;
-  if (A.scores_in) {
+  if constexpr (SCORED) {
     if (n_elig > A.topk) {
       const float* sc = A.scores_in + (long)row * A.max_blocks;
       unsigned lo = 0xffffffffu, hi = 0u;
@@ -1194,10 +1204,8 @@ __device__ void select_row(const SelArgs& A, SelShared& S, int row, int b, int p
       const int npad = (n_elig + 31) & ~31;
       for (int j = n_elig + tid; j < npad; j += NT) S.key[j] = 0ull;
       // the bucket threshold's key range, published by the barrier below
-      if constexpr (NT >= 1024) {
-        bucket_range<NT>(lo, hi, S.rscr);
-        range_in = true;
-      }
+      bucket_range<NT>(lo, hi, S.rscr);
+      range_in = true;
     }
   } else if (n_elig > A.topk || A.scores_out) {
     const float* bk = A.block_keys + (long)b * A.max_blocks * IDX_D;
@@ -1221,7 +1229,7 @@ __device__ void select_row(const SelArgs& A, SelShared& S, int row, int b, int p
   if (n_elig <= A.topk) {
     for (int i = tid; i < n_elig; i += NT) { out_ids[i] = i; S.sel[i] = i; }
   } else {
-    rank_topk<NT, SEL_MAX_BLOCKS / 2>(S.key, n_elig, A.topk, S.sel, S.rscr, range_in);
+    rank_topk<NT, SH::MAXK>(S.key, n_elig, A.topk, S.sel, S.rscr, range_in);
     __syncthreads();
     QM_PHASE(2);
     for (int i = tid; i < A.topk; i += NT) out_ids[i] = S.sel[i];
@@ -1454,9 +1462,38 @@ __global__ __launch_bounds__(SELP_NT) void qsa_select_kernel(SelArgs A) {
     S.q[i] = i < A.idx_heads * IDX_D ? A.iq[(long)row * A.idx_heads * IDX_D + i] : 0.f;
   __syncthreads();
   __shared__ float4 stage[SEQ_STAGE / 4];   // block rows of a scoring round (several rows per sequence)
-  select_row<SELP_NT>(A, S, row, b, p, -1, reinterpret_cast<float*>(stage));
+  select_row<SELP_NT, false>(A, S, row, b, p, -1, reinterpret_cast<float*>(stage));
   QM_PHASE(3);
   QM_PHASE_FLUSH();
+}
+
+// The same for rows whose scores were formed by a launch before
+// (A.scores_in): 256 threads for up to RANK_SMALL_BLOCKS blocks, in 18 KB of
+// LDS, so that a compute unit holds eight rows at once, and 1024 threads for up
+// to 4096. With 1024 threads and 141 KB for every row (one a compute unit) the
+// ranking took 35 us for 1999 rows over 127 blocks, now 9.6; 8.6 us for 300
+// rows over 312 blocks, now 5.7; one row of 511 blocks is even (5.5).
+template <int NT, int MAXB>
+__global__ __launch_bounds__(NT) void qsa_rank_kernel(SelArgs A) {
+  const int row = blockIdx.x;
+  const int b = row / A.seq, s = row % A.seq;
+  const int p = A.positions[b] + s;
+  __shared__ RankShared<MAXB> S;
+  select_row<NT, true>(A, S, row, b, p, -1, nullptr);
+}
+
+constexpr int RANK_SMALL_BLOCKS = 1024;
+
+// Launch the selection of A's rows.
+int launch_select(const SelArgs& A, int rows, hipStream_t stream) {
+  if (!A.scores_in)
+    hipLaunchKernelGGL(qsa_select_kernel, dim3(rows), dim3(SELP_NT), 0, stream, A);
+  else if (A.max_blocks <= RANK_SMALL_BLOCKS && A.max_pages <= RANK_SMALL_BLOCKS && A.topk <= RANK_SMALL_BLOCKS / 2)
+    hipLaunchKernelGGL((qsa_rank_kernel<256, RANK_SMALL_BLOCKS>), dim3(rows), dim3(256), 0, stream, A);
+  else
+    hipLaunchKernelGGL((qsa_rank_kernel<SELP_NT, SEL_MAX_BLOCKS>), dim3(rows), dim3(SELP_NT), 0, stream, A);
+  QM_CHECK_LAUNCH();
+  return QM_OK;
 }
 
 // Decode (one token per sequence) front end in one launch: the query, key and
@@ -1501,7 +1538,7 @@ __global__ __launch_bounds__(SEL_NT) void qsa_front_kernel(PrepArgs<T> A, SelArg
     if (tid < IDX_D) S.newkey[tid] = y;
   }
   __syncthreads();
-  select_row<SEL_NT>(SA, S, b, b, p, new_j, nullptr);
+  select_row<SEL_NT, false>(SA, S, b, b, p, new_j, nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -3356,9 +3393,7 @@ extern "C" int qm_qsa_select(const qm_qsa_geom* g, int seq, const float* iq, con
     A.scores_in = scores_out;
     A.scores_out = nullptr;
   }
-  hipLaunchKernelGGL(qsa_select_kernel, dim3(g->batch * seq), dim3(SELP_NT), 0, stream, A);
-  QM_CHECK_LAUNCH();
-  return QM_OK;
+  return launch_select(A, g->batch * seq, stream);
 }
 
 
@@ -3556,9 +3591,7 @@ extern "C" int qm_qsa_select_chunk(const qm_qsa_geom* g, int seq, const float* i
   A.tab = reinterpret_cast<uint16_t*>(base + L.tab);
   A.part_ml = reinterpret_cast<float*>(base + L.ml);
   A.hkv = g->n_kv_heads;
-  hipLaunchKernelGGL(qsa_select_kernel, dim3(g->batch * seq), dim3(SELP_NT), 0, stream, A);
-  QM_CHECK_LAUNCH();
-  return QM_OK;
+  return launch_select(A, g->batch * seq, stream);
 }
 
 extern "C" int qm_qsa_attend_chunk_filed(const qm_qsa_geom* g, int seq, const void* q, const void* qg,
