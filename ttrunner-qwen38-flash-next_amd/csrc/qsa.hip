@@ -20,7 +20,7 @@
 
 #include <type_traits>
 
-#include "common.h"
+#include "rows_mma.h"
 #include "qwen4mix_internal.h"
 
 namespace {
@@ -1687,7 +1687,16 @@ template <typename T, typename PO = float>
 struct CombineArgs {
   const PO* part_o; const float* part_ml; const T* qg; T* out;
   int hq, hkv, splits;
+  // the chunk path: this launch's rows [row0, row0 + rows) of each sequence of
+  // seq rows (part_o holds those alone); 0: every row, one per grid row
+  int seq = 0, row0 = 0, rows = 0;
 };
+
+// the row (of [B * seq]) of a merge workgroup
+template <typename A>
+__device__ __forceinline__ int combine_row(const A& a, int local) {
+  return a.rows ? local / a.rows * a.seq + a.row0 + local % a.rows : local;
+}
 
 __device__ __forceinline__ float part_value(const float* p, long i) { return p[i]; }
 __device__ __forceinline__ float part_value(const uint16_t* p, long i) { return bf16_to_f32(p[i]); }
@@ -1697,10 +1706,11 @@ constexpr int MAX_SPLITS = 1024;
 template <typename T, typename PO = float>
 __global__ __launch_bounds__(QSA_D) void qsa_combine_kernel(CombineArgs<T, PO> A) {
   constexpr bool normed = sizeof(PO) == 2;
-  const int hq = blockIdx.x, row = blockIdx.y;
+  const int hq = blockIdx.x, row = combine_row(A, blockIdx.y);
   const int d = threadIdx.x;
   const int g = hq / GQA, hh = hq % GQA;
   const long base = (((long)row * A.hkv + g) * A.splits) * GQA + hh;
+  const long obase = (((long)blockIdx.y * A.hkv + g) * A.splits) * GQA + hh;
   __shared__ float s_w[MAX_SPLITS];
   __shared__ float s_red[QSA_D / 64];
   const float gate = Act<T>::load(A.qg, ((long)row * A.hq + hq) * (2 * QSA_D) + QSA_D + d);
@@ -1736,12 +1746,83 @@ __global__ __launch_bounds__(QSA_D) void qsa_combine_kernel(CombineArgs<T, PO> A
   // zero weight (never written, or under the max by ~88) adds exactly 0
 #pragma unroll 8
   for (int s = 0; s < A.splits; ++s) {
-    const float v = part_value(A.part_o, (base + (long)s * GQA) * QSA_D + d);
+    const float v = part_value(A.part_o, (obase + (long)s * GQA) * QSA_D + d);
     o += s_w[s] != 0.f ? v * s_w[s] : 0.f;
   }
   const float att = Act<T>::round(o / L);
   const float sg = Act<T>::round(sigmoid_f(gate));
   Act<T>::store(A.out, ((long)row * A.hq + hq) * QSA_D + d, att * sg);
+}
+
+// The chunk path's merge for many rows: one workgroup per (kv head, row) takes
+// all 8 query heads, wave w heads 2 w and 2 w + 1, lane l channels 8 (l % 32) ..
+// + 7 of head 2 w + l / 32, so that a slot's partials (4 KB in a run) are one
+// 16-byte load per lane (a channel per thread loads 2 bytes, 128 a wave): 138 MB
+// of 512 rows in 23.7 us (5.8 TB/s from the memory-side cache) against 26.8.
+template <typename T>
+__global__ __launch_bounds__(QSA_D) void qsa_combine_rows_kernel(CombineArgs<T, uint16_t> A) {
+  extern __shared__ float2 s_ml[];             // [splits][8]: (max, sum), then (weight, -)
+  __shared__ float s_red[2][4][GQA];
+  const int g = blockIdx.x, row = combine_row(A, blockIdx.y);
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int hh = 2 * wv + (lane >> 5), ch = 8 * (lane & 31);
+  const int hq = g * GQA + hh;
+  const long base = ((long)row * A.hkv + g) * A.splits * GQA;
+  const T* gp = A.qg + ((long)row * A.hq + hq) * (2 * QSA_D) + QSA_D + ch;
+  float gate[8];
+#pragma unroll
+  for (int i = 0; i < 8; i += 4) {
+    float q[4];
+    load_act4(gp + i, q);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) gate[i + u] = q[u];
+  }
+  // the weights: thread t takes head t % 8 of slots t / 8, + 32, ...
+  const int n = A.splits * GQA;
+  const float2* ml = reinterpret_cast<const float2*>(A.part_ml) + base;
+  float m = -INFINITY;
+  for (int i = tid; i < n; i += QSA_D) {
+    const float2 v = ml[i];
+    s_ml[i] = v;
+    m = fmaxf(m, v.x);
+  }
+  m = fmaxf(m, dpp_f<0x128>(m));               // lane ^ 8 of a 16-lane row (row_ror:8)
+  m = xor32_max(xor16_max(m));
+  if (lane < GQA) s_red[0][wv][lane] = m;
+  __syncthreads();
+  const int h8 = tid & 7;
+  const float M = fmaxf(fmaxf(s_red[0][0][h8], s_red[0][1][h8]), fmaxf(s_red[0][2][h8], s_red[0][3][h8]));
+  float l = 0.f;
+  for (int i = tid; i < n; i += QSA_D) {
+    const float2 v = s_ml[i];
+    const float lw = v.x == -INFINITY ? 0.f : v.y * __expf(v.x - M);
+    l += lw;
+    s_ml[i].x = lw;
+  }
+  l += dpp_f<0x128>(l);
+  l = xor32_sum(xor16_sum(l));
+  if (lane < GQA) s_red[1][wv][lane] = l;
+  __syncthreads();
+  const float L = (s_red[1][0][hh] + s_red[1][1][hh]) + (s_red[1][2][hh] + s_red[1][3][hh]);
+  float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  const uint16_t* po = A.part_o + (((long)blockIdx.y * A.hkv + g) * A.splits * GQA + hh) * QSA_D + ch;
+  // loads unconditional so that eleven are in flight; a slot of zero weight
+  // (never written, or under the max by ~88) adds exactly 0
+#pragma unroll 11
+  for (int s = 0; s < A.splits; ++s) {
+    const uint4 v = *reinterpret_cast<const uint4*>(po + (long)s * GQA * QSA_D);
+    const float w = s_ml[s * GQA + hh].x;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o[i] += w != 0.f ? Chunk<bf16_t>::get(v, i) * w : 0.f;
+  }
+  T* out = A.out + ((long)row * A.hq + hq) * QSA_D + ch;
+#pragma unroll
+  for (int i = 0; i < 8; i += 4) {
+    float y[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) y[u] = Act<T>::round(o[i + u] / L) * Act<T>::round(sigmoid_f(gate[i + u]));
+    store_act4(out + i, y);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1791,6 +1872,8 @@ struct ChunkAttnArgs {
   uint16_t* part_o; float* part_ml;      // part_o: bf16, normalised by l
   const uint16_t* tab;                    // [B][max_blocks][seq]: slot + 1, or 0
   int batch, seq, hq, hkv, page_size, max_pages, ratio, topk, max_blocks, nwg_sel;
+  int seg_spans, nseg;                    // 128-row spans of a block's table column per workgroup, segments of a column
+  int row0, rows;                         // the rows of each sequence this launch takes (row0 a multiple of 128)
   float scale;
 };
 
@@ -1867,6 +1950,10 @@ __device__ __forceinline__ unsigned pick4(const unsigned (&v)[4], int w) {
 __device__ __forceinline__ long chunk_partial_row(const ChunkAttnArgs& A, unsigned pk, long row_b, int g, int nslot,
                                                   int hh) {
   return (((row_b + (pk >> 16)) * A.hkv + g) * nslot + (pk & 511)) * GQA + hh;
+}
+// The same among the launch's own rows, where its outputs go.
+__device__ __forceinline__ long chunk_output_row(const ChunkAttnArgs& A, unsigned pk, int b, int g, int nslot, int hh) {
+  return ((((long)b * A.rows + static_cast<int>(pk >> 16) - A.row0) * A.hkv + g) * nslot + (pk & 511)) * GQA + hh;
 }
 
 // One wave's scores over the block for its two entries x 8 query heads (lane
@@ -1964,7 +2051,7 @@ __device__ __forceinline__ void chunk_no_scores(ChunkShared& S) {
 // stores together 64 contiguous bytes of a partial row). pko/oko: the entries
 // of column block cw's lanes (entry il of wave cw) and whether they exist.
 __device__ __forceinline__ void chunk_outputs(const ChunkAttnArgs& A, ChunkShared& S, const bf16x8_t (&vr)[2][4],
-                                              const unsigned (&pko)[4], const bool (&oko)[4], long row_b, int g,
+                                              const unsigned (&pko)[4], const bool (&oko)[4], int b, int g,
                                               int nslot, bool mark = false) {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, quad = lane >> 4, hh = lane & 7;
   const int gpb = A.ratio / 32;
@@ -1985,7 +2072,7 @@ __device__ __forceinline__ void chunk_outputs(const ChunkAttnArgs& A, ChunkShare
     // quad then holds channels 4 quad .. + 7 of the pair's first block (its
     // own and the next quad's), an odd quad channels 4 (quad - 1) .. + 7 of
     // the second, so every lane stores 16 contiguous bytes
-    uint16_t* dst = A.part_o + chunk_partial_row(A, pko[cw], row_b, g, nslot, hh) * QSA_D + 64 * wv +
+    uint16_t* dst = A.part_o + chunk_output_row(A, pko[cw], b, g, nslot, hh) * QSA_D + 64 * wv +
                     16 * (quad & 1) + 4 * (quad & 2);
 #pragma unroll
     for (int cp = 0; cp < 4; cp += 2) {
@@ -2068,23 +2155,25 @@ __global__ __launch_bounds__(CA_NT, 4) void qsa_chunk_attend_kernel(ChunkAttnArg
     page1 = ptab[min((j * A.ratio + (gpb > 1 ? 32 : 0)) / A.page_size, A.max_pages - 1)];
   };
 
-  if (x < A.nwg_sel) {
-    // ---- block j = x: the first 128 rows of its table row, its pages and
-    // the position in one round trip; then its entries in groups of 8
-    const int j = x;
+  if (x < A.nwg_sel * A.nseg) {
+    // ---- block j, a segment of its table row: the first 128 rows of it, its
+    // pages and the position in one round trip; then its entries in groups of 8
+    const int sg = x / A.nwg_sel, j = x - sg * A.nwg_sel;
+    const int row_end = A.row0 + A.rows;
+    const int c0 = (A.row0 >> 7) + sg * A.seg_spans, c1 = min(c0 + A.seg_spans, (row_end + 127) >> 7);
     const uint16_t* tcol = A.tab + row_b * A.max_blocks + j;     // row s's entry for this block at s * max_blocks
-    const int ta = lane < A.seq ? tcol[(long)(lane) * A.max_blocks] : 0;
-    const int tb = 64 + lane < A.seq ? tcol[(long)(64 + lane) * A.max_blocks] : 0;
+    const int ta = 128 * c0 + lane < row_end ? tcol[(long)(128 * c0 + lane) * A.max_blocks] : 0;
+    const int tb = 128 * c0 + 64 + lane < row_end ? tcol[(long)(128 * c0 + 64 + lane) * A.max_blocks] : 0;
     int page0, page1;
     pages_of(j, page0, page1);
     const int pos0 = A.positions[b];
     if (j >= table_blocks(pos0, A.seq, A.ratio, A.max_blocks)) return;     // past every row's blocks: no entries
     bool loaded = false, first = true;
-    for (int c = 0; 128 * c < A.seq; ++c) {
+    for (int c = c0; c < c1; ++c) {
       // rows 128 c + lane and 128 c + 64 + lane of the table row
       const int ra = 128 * c + lane, rb = ra + 64;
-      const int tva = c == 0 ? ta : ra < A.seq ? tcol[(long)ra * A.max_blocks] : 0;
-      const int tvb = c == 0 ? tb : rb < A.seq ? tcol[(long)rb * A.max_blocks] : 0;
+      const int tva = c == c0 ? ta : ra < row_end ? tcol[(long)ra * A.max_blocks] : 0;
+      const int tvb = c == c0 ? tb : rb < row_end ? tcol[(long)rb * A.max_blocks] : 0;
       unsigned long long la = __ballot(tva != 0), lb = __ballot(tvb != 0);
       if ((la | lb) == 0ull) continue;
       const int nc = __popcll(la) + __popcll(lb);
@@ -2117,22 +2206,22 @@ __global__ __launch_bounds__(CA_NT, 4) void qsa_chunk_attend_kernel(ChunkAttnArg
 #pragma unroll
         for (int cw = 0; cw < 4; ++cw) oko[cw] = g0 + 2 * cw + il < nc;
         __syncthreads();
-        chunk_outputs(A, S, vr, pko, oko, row_b, g, nslot, first);
+        chunk_outputs(A, S, vr, pko, oko, b, g, nslot, first);
         first = false;
       }
     }
   } else {
     // ---- the tail entries (keys ts..p) of rows tr0 .. tr0 + 7: block jt, then
     // block jt + 1 when the rows cross a block boundary
-    const int tr0 = (x - A.nwg_sel) * CA_TAIL_ROWS;
+    const int tr0 = A.row0 + (x - A.nwg_sel * A.nseg) * CA_TAIL_ROWS;
     const int pos0 = A.positions[b];
     const int jt = (pos0 + tr0) / A.ratio;
     // entry e of the workgroup (row tr0 + e): its packed (row, tail, slot) and
     // whether its tail lies in block j
     auto tail_entry = [&](int e, int j, unsigned& pk) __attribute__((always_inline)) {
       const int r = tr0 + e, p = pos0 + r;
-      pk = (static_cast<unsigned>(min(r, A.seq - 1)) << 16) | (1u << 9) | static_cast<unsigned>(A.topk);
-      return r < A.seq && ((p + 1) / A.ratio) * A.ratio <= p && p / A.ratio == j;
+      pk = (static_cast<unsigned>(min(r, A.row0 + A.rows - 1)) << 16) | (1u << 9) | static_cast<unsigned>(A.topk);
+      return r < A.row0 + A.rows && ((p + 1) / A.ratio) * A.ratio <= p && p / A.ratio == j;
     };
     int pa0, pa1, pb0, pb1;
     pages_of(jt, pa0, pa1);
@@ -2165,7 +2254,7 @@ __global__ __launch_bounds__(CA_NT, 4) void qsa_chunk_attend_kernel(ChunkAttnArg
       if (__builtin_amdgcn_ballot_w64(mine) != 0ull) chunk_scores(A, S, qhi, j, pk, mine, row_b, pos0, g, nslot);
       else chunk_no_scores(S);
       __syncthreads();
-      chunk_outputs(A, S, vr, pko, oko, row_b, g, nslot);
+      chunk_outputs(A, S, vr, pko, oko, b, g, nslot);
     }
   }
   QM_PHASE(4);
@@ -3505,6 +3594,37 @@ extern "C" size_t qm_qsa_attend_chunk_workspace(const qm_qsa_geom* g, int seq) {
 }
 
 namespace {
+// Rows from which the merge takes whole-slot loads (us, a channel per thread /
+// here: 8.2 / 9.4 at 128 rows, 17.1 / 16.8 at 300, 26.8 / 23.7 at 512).
+constexpr int COMBINE_MANY_ROWS = 256;
+// A block's entries are taken by a workgroup per 128 rows, so that a long chunk
+// over few blocks fills the device (512 rows over 117 blocks: 54.9 us, with 256
+// rows a workgroup 63.5; 1999 rows over 127 blocks, one workgroup per block and
+// kv head: 297 us, now 207).
+constexpr int CA_SEG_SPANS = 1;
+// A long chunk's rows go through the attention and the merge in parts whose
+// partial outputs (270 KB a row) stay in the 256 MB memory-side cache from the
+// one to the other, each over the last one's: 1999 rows (540 MB) 207 + 96 us in
+// two parts, 193 + 150 in one, 233 + 111 in four.
+constexpr size_t CA_PART_BYTES = 280ull << 20;
+
+template <typename T>
+int launch_combine_chunk(const qm_qsa_geom* g, int seq, int row0, int n_rows, const uint16_t* part_o,
+                         const float* part_ml, const void* qg, void* out, int nslot, hipStream_t stream) {
+  CombineArgs<T, uint16_t> C{part_o, part_ml, static_cast<const T*>(qg), static_cast<T*>(out), g->n_heads,
+                             g->n_kv_heads, nslot, seq, row0, n_rows};
+  const int rows = g->batch * n_rows;
+  // the wide loads need qg and out in 16-byte units (8 in bf16); rows and heads are
+  const bool aligned = ((reinterpret_cast<uintptr_t>(qg) | reinterpret_cast<uintptr_t>(out)) & (4 * sizeof(T) - 1)) == 0;
+  if (rows >= COMBINE_MANY_ROWS && aligned)
+    hipLaunchKernelGGL(qsa_combine_rows_kernel<T>, dim3(g->n_kv_heads, rows), dim3(QSA_D),
+                       (size_t)nslot * GQA * sizeof(float2), stream, C);
+  else
+    hipLaunchKernelGGL((qsa_combine_kernel<T, uint16_t>), dim3(g->n_heads, rows), dim3(QSA_D), 0, stream, C);
+  QM_CHECK_LAUNCH();
+  return QM_OK;
+}
+
 int attend_chunk(const qm_qsa_geom* g, int seq, const void* q, const void* qg, const void* k_pool, const void* v_pool,
                  const int* positions, const int* page_table, const int* ids, const int* n_sel, void* out,
                  void* workspace, size_t workspace_bytes, bool filed, hipStream_t stream) {
@@ -3541,20 +3661,23 @@ int attend_chunk(const qm_qsa_geom* g, int seq, const void* q, const void* qg, c
   // pipelined within one (measured at 512 blocks x 2 kv heads: 31.5 us, two
   // blocks per workgroup 33.4 us, four 47.0 us)
   A.nwg_sel = g->max_blocks;
-  const int n_tail = (seq + CA_TAIL_ROWS - 1) / CA_TAIL_ROWS;
-  hipLaunchKernelGGL(qsa_chunk_attend_kernel, dim3(A.nwg_sel + n_tail, g->n_kv_heads, g->batch), dim3(CA_NT),
-                     0, stream, A);
-  QM_CHECK_LAUNCH();
-  if (g->act_dtype == QM_ACT_F32) {
-    CombineArgs<float, uint16_t> C{part_o, part_ml, static_cast<const float*>(qg), static_cast<float*>(out), g->n_heads,
-                         g->n_kv_heads, nslot};
-    hipLaunchKernelGGL((qsa_combine_kernel<float, uint16_t>), dim3(g->n_heads, g->batch * seq), dim3(QSA_D), 0, stream, C);
-  } else {
-    CombineArgs<bf16_t, uint16_t> C{part_o, part_ml, static_cast<const bf16_t*>(qg), static_cast<bf16_t*>(out), g->n_heads,
-                          g->n_kv_heads, nslot};
-    hipLaunchKernelGGL((qsa_combine_kernel<bf16_t, uint16_t>), dim3(g->n_heads, g->batch * seq), dim3(QSA_D), 0, stream, C);
+  A.seg_spans = CA_SEG_SPANS;
+  const size_t row_bytes = (size_t)g->batch * g->n_kv_heads * nslot * GQA * QSA_D * sizeof(uint16_t);
+  const size_t n_part = (seq * row_bytes + CA_PART_BYTES - 1) / CA_PART_BYTES;
+  const int part = (int)(((seq + n_part - 1) / n_part + 127) / 128 * 128);
+  for (int row0 = 0; row0 < seq; row0 += part) {
+    A.row0 = row0;
+    A.rows = part < seq - row0 ? part : seq - row0;
+    A.nseg = (A.rows + 128 * A.seg_spans - 1) / (128 * A.seg_spans);
+    const int n_tail = (A.rows + CA_TAIL_ROWS - 1) / CA_TAIL_ROWS;
+    hipLaunchKernelGGL(qsa_chunk_attend_kernel, dim3(A.nwg_sel * A.nseg + n_tail, g->n_kv_heads, g->batch), dim3(CA_NT),
+                       0, stream, A);
+    QM_CHECK_LAUNCH();
+    rc = g->act_dtype == QM_ACT_F32
+             ? launch_combine_chunk<float>(g, seq, row0, A.rows, part_o, part_ml, qg, out, nslot, stream)
+             : launch_combine_chunk<bf16_t>(g, seq, row0, A.rows, part_o, part_ml, qg, out, nslot, stream);
+    if (rc) return rc;
   }
-  QM_CHECK_LAUNCH();
   return QM_OK;
 }
 }  // namespace
