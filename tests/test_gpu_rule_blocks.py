@@ -1,0 +1,74 @@
+"""The token-loop delta rule (dn_recurrent_kernel) at the edges of its 16-token
+blocks, against the recurrence in float64 (oracle/f64.py is its CPU form; the
+loop here is the same three lines). Bars: float32 outputs and state within 1e-5
+of the largest value (128-term sums in another order), bf16 outputs within one
+rounding (2^-8)."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def rule64(q, k, v, g, beta, S):
+    q, k, v, g, beta, S = (t.double() for t in (q, k, v, g, beta, S))
+    q = q * torch.rsqrt((q * q).sum(-1, keepdim=True) + 1e-6) / q.shape[-1] ** 0.5
+    k = k * torch.rsqrt((k * k).sum(-1, keepdim=True) + 1e-6)
+    out = torch.empty_like(v)
+    for t in range(q.shape[1]):
+        S = S * g[:, t].exp()[..., None, None]
+        d = (v[:, t] - (S * k[:, t][..., None]).sum(-2)) * beta[:, t][..., None]
+        S = S + k[:, t][..., None] * d[..., None, :]
+        out[:, t] = (S * q[:, t][..., None]).sum(-2)
+    return out, S
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("batch,heads,seq", [(1, 32, 1), (2, 3, 15), (1, 32, 16), (1, 5, 17), (3, 2, 33), (1, 32, 64)])
+def test_recurrent_rule_blocks(gpu, dtype, batch, heads, seq):
+    from importlib import import_module
+    layers = import_module(gpu.__name__ + ".layers")
+    print(f"recurrent rule {dtype} batch={batch} heads={heads} seq={seq}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(seq * 31 + heads)
+    r = lambda *s: torch.randn(*s, generator=gen, device=DEV)  # noqa: E731
+    q, k, v = (r(batch, seq, heads, 128).to(dtype) for _ in range(3))
+    g, beta = -r(batch, seq, heads).abs(), torch.sigmoid(r(batch, seq, heads))
+    S = r(batch, heads, 128, 128) * 0.1
+    want, want_S = rule64(q, k, v, g, beta, S)
+    out, state = layers.recurrent_gated_delta_rule(q, k, v, g, beta, S)
+    torch.cuda.synchronize()
+    bar = 1e-5 if dtype == torch.float32 else 2 ** -8
+    # per token: a wrong token of a block would hide in the whole
+    err = (out.double() - want).abs().amax((2, 3)) / want.abs().amax((2, 3))
+    assert float(err.max()) < bar
+    assert float((state.double() - want_S).abs().max() / want_S.abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("seq", [15, 16, 23, 24, 25])
+def test_prefill_rule_at_the_dispatch(gpu, seq):
+    """qm_dn_prefill either side of the line between the token loop and the
+    chunked rule (24 tokens): the same prompt one token at a time through the
+    decode path. bf16 outputs within 2e-2 of the largest value, the state within
+    1e-3 (the bars of the decode and prefill tests)."""
+    qm = gpu
+    import os
+    import sys
+    sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden"))
+    import inputs as gi
+    bf = torch.bfloat16
+    model = qm.Qwen4MixModel(qm.MixConfig(), gi.FakeStore(gi.dn_weights(0, 7, bf)), device=DEV, max_ctx=64)
+    gen = torch.Generator(device=DEV).manual_seed(seq)
+    r = lambda *s: torch.randn(*s, generator=gen, device=DEV).to(bf)  # noqa: E731
+    qkv, z, a, b = r(1, seq, 8192), r(1, seq, 4096), r(1, seq, 32), r(1, seq, 32)
+    print(f"prefill rule seq={seq}", flush=True)
+    one, many = (qm.MixHybridCache(1, model.config, 1, 64, DEV, bf) for _ in range(2))
+    got = model.dn_core(qkv, z, a, b, 0, many[0])
+    rows = [slice(t, t + 1) for t in range(seq)]
+    want = torch.cat([model.dn_core(*(x[:, s].contiguous() for x in (qkv, z, a, b)), 0, one[0]) for s in rows], 1)
+    torch.cuda.synchronize()
+    assert float((got.float() - want.float()).abs().max() / want.float().abs().max()) < 2e-2
+    assert float((many[0].recurrent_state - one[0].recurrent_state).abs().max()) < 1e-3
+    assert torch.equal(many[0].conv_state, one[0].conv_state)

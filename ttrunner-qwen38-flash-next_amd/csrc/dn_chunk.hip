@@ -36,7 +36,8 @@ constexpr int CK_NT = 256;        // four waves
 constexpr int CK_LD = CK_D + 4;   // LDS row stride of [token][dim] tiles, floats
 constexpr int CK_LT = CK_C + 4;   // LDS row stride of [.][token] tiles, floats
 constexpr int CK_COLS = 16;       // d_v columns per scan workgroup
-constexpr int CK_MIN_SEQ = 16;    // shorter prefill chunks take the token loop
+constexpr int CK_MIN_SEQ = 24;    // shorter prefill chunks take the token loop (us, loop / chunked, 32 heads in
+                                  // bf16: 11.9 / 16.9 at 16 tokens, 15.9 / 17.0 at 24, 18.1 / 17.0 at 32)
 constexpr int CK_PARTS = 4;       // prep workgroups per chunk when chunks are few
 
 // One record per (sequence, head, chunk), in floats. A fragment pair is the
@@ -231,7 +232,8 @@ struct ChunkPrepArgs {
   const T* q; const T* k; const T* v;   // token rows of q_stride / v_stride elements
   const float* g; const float* beta;    // [B, S, H]
   float* ws;                            // [B, H, n_chunks] records
-  int batch, seq, heads, hk, n_chunks;  // head h reads q/k head h % hk
+  int batch, seq, heads, hk;            // head h reads q/k head h % hk
+  int c0, n_chunks;                     // this launch's first chunk, and its chunks (and the records') per head
   int parts;                            // workgroups per chunk: 1 or CK_PARTS
   long q_stride, v_stride;
 };
@@ -265,7 +267,7 @@ __global__ __launch_bounds__(CK_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A
   const int bh = wg / A.parts / A.n_chunks;
   const int span = CK_PARTS / A.parts;       // quarters this workgroup writes
   const int h = bh % A.heads, b = bh / A.heads;
-  const int t0 = c * CK_C;
+  const int t0 = (A.c0 + c) * CK_C;
   const int n_valid = min(CK_C, A.seq - t0);
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int g4 = lane >> 4, r16 = lane & 15;
@@ -628,7 +630,8 @@ struct ChunkScanArgs {
   const float* ws;   // [B, H, n_chunks] records
   float* state;      // [B, H, 128, 128]
   T* out;            // [B, S, H, 128]
-  int batch, seq, heads, n_chunks;
+  int batch, seq, heads;
+  int t0, n_chunks;  // this launch's first token, and its chunks (and the records') per head
 };
 
 // A wave's record operands of one chunk, none of which depends on the
@@ -742,7 +745,7 @@ __global__ __launch_bounds__(CK_NT) void dn_chunk_scan_kernel(ChunkScanArgs<T> A
     const Frag va0 = lds_frag(sVh, sVl, SC_SV, r16, 0, g4), va1 = lds_frag(sVh, sVl, SC_SV, r16, 1, g4);
     ao = mfma3(va0, cur.qk[0], ao);
     if (wid >= 2) ao = mfma3(va1, cur.qk[1], ao);
-    const int tok = ci * CK_C + 16 * wid + r16;
+    const int tok = A.t0 + ci * CK_C + 16 * wid + r16;
     if (tok < A.seq) {
       T* o = A.out + (((long)b * A.seq + tok) * A.heads + h) * CK_D + col0 + 4 * g4;
 #pragma unroll
@@ -781,26 +784,41 @@ __global__ __launch_bounds__(CK_NT) void dn_chunk_scan_kernel(ChunkScanArgs<T> A
   QM_PHASE_FLUSH_AT(4096u);
 }
 
+// Long sequences run in segments of chunks, prep and scan in turn, each
+// segment's records over the last one's: the prep's records are written once
+// and read once, and while a segment's stay in the 256 MB memory-side cache the
+// scan does not wait for memory. 4096 tokens of 32 heads (302 MB of records):
+// 343 us in one segment, 296 in two or four, 313 in eight (each scan starts
+// again from the state, about 4 us); 4000 tokens in bf16 315 -> 262 us; 2048
+// tokens (151 MB) 150 us in one segment, 145 in two, bf16 131 and 136.
+constexpr size_t CK_SEG_BYTES = 160ull << 20;
+
 template <typename T>
 int launch_chunked(int batch, int seq, int heads, int hk, long q_stride, long v_stride, const void* q, const void* k,
                    const void* v, const float* g, const float* beta, float* state, void* out, float* ws,
                    hipStream_t stream) {
-  const int n_chunks = (seq + CK_C - 1) / CK_C;
-  ChunkPrepArgs<T> P;
-  P.q = static_cast<const T*>(q); P.k = static_cast<const T*>(k); P.v = static_cast<const T*>(v);
-  P.g = g; P.beta = beta; P.ws = ws;
-  P.batch = batch; P.seq = seq; P.heads = heads; P.hk = hk; P.n_chunks = n_chunks;
-  P.q_stride = q_stride; P.v_stride = v_stride;
-  // few chunks: four workgroups per chunk so that the launch fills the chip;
-  // many: one each, since every workgroup repeats the L and T work
-  P.parts = (long)batch * heads * n_chunks < 256 ? CK_PARTS : 1;
-  hipLaunchKernelGGL(dn_chunk_prep_kernel<T>, dim3(batch * heads * n_chunks * P.parts), dim3(CK_NT), 0, stream, P);
-  QM_CHECK_LAUNCH();
-  ChunkScanArgs<T> S;
-  S.ws = ws; S.state = state; S.out = static_cast<T*>(out);
-  S.batch = batch; S.seq = seq; S.heads = heads; S.n_chunks = n_chunks;
-  hipLaunchKernelGGL(dn_chunk_scan_kernel<T>, dim3(batch * heads * (CK_D / CK_COLS)), dim3(CK_NT), 0, stream, S);
-  QM_CHECK_LAUNCH();
+  const int n_total = (seq + CK_C - 1) / CK_C;
+  const size_t chunk_bytes = (size_t)batch * heads * CK_REC * sizeof(float);
+  const size_t n_seg = (n_total * chunk_bytes + CK_SEG_BYTES - 1) / CK_SEG_BYTES;
+  const int seg = n_seg < (size_t)n_total ? (int)((n_total + n_seg - 1) / n_seg) : 1;
+  for (int c0 = 0; c0 < n_total; c0 += seg) {
+    const int n_chunks = seg < n_total - c0 ? seg : n_total - c0;
+    ChunkPrepArgs<T> P;
+    P.q = static_cast<const T*>(q); P.k = static_cast<const T*>(k); P.v = static_cast<const T*>(v);
+    P.g = g; P.beta = beta; P.ws = ws;
+    P.batch = batch; P.seq = seq; P.heads = heads; P.hk = hk; P.c0 = c0; P.n_chunks = n_chunks;
+    P.q_stride = q_stride; P.v_stride = v_stride;
+    // few chunks: four workgroups per chunk so that the launch fills the chip;
+    // many: one each, since every workgroup repeats the L and T work
+    P.parts = (long)batch * heads * n_chunks < 256 ? CK_PARTS : 1;
+    hipLaunchKernelGGL(dn_chunk_prep_kernel<T>, dim3(batch * heads * n_chunks * P.parts), dim3(CK_NT), 0, stream, P);
+    QM_CHECK_LAUNCH();
+    ChunkScanArgs<T> S;
+    S.ws = ws; S.state = state; S.out = static_cast<T*>(out);
+    S.batch = batch; S.seq = seq; S.heads = heads; S.t0 = c0 * CK_C; S.n_chunks = n_chunks;
+    hipLaunchKernelGGL(dn_chunk_scan_kernel<T>, dim3(batch * heads * (CK_D / CK_COLS)), dim3(CK_NT), 0, stream, S);
+    QM_CHECK_LAUNCH();
+  }
   return QM_OK;
 }
 

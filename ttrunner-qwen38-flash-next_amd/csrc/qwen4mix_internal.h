@@ -17,7 +17,7 @@ int qm_dn_recurrent_strided(int act_dtype, int batch, int seq, int heads, int hk
                             float* state, void* out, hipStream_t stream);
 
 // The delta rule over a chunk of tokens for the prefill path: the WY/UT chunked
-// kernels (64-token chunks) for chunks of 16 tokens or more, the token loop for
+// kernels (64-token chunks) for chunks of 24 tokens or more, the token loop for
 // shorter ones. `ws` holds qm_dn_rule_chunk_workspace(batch, seq, heads) bytes.
 size_t qm_dn_rule_chunk_workspace(int batch, int seq, int heads);
 int qm_dn_rule_chunk(int act_dtype, int batch, int seq, int heads, int hk, long q_stride, long v_stride,
