@@ -1128,8 +1128,8 @@ __device__ void rank_topk(const unsigned long long* keys, int n, int topk, int* 
   }
 }
 
-// Blocks of the slot table's rows that a chunk's entries can name: those some
-// row of it may select. The rest of a table row is neither written nor read.
+// Blocks of the slot table that a chunk's entries can name: those some row of
+// it may select. The other blocks' lists are neither written nor read.
 __device__ __forceinline__ int table_blocks(int pos0, int seq, int ratio, int max_blocks) {
   return min((pos0 + seq) / ratio, max_blocks);
 }
@@ -1224,6 +1224,15 @@ __device__ void select_row(const SelArgs& A, SH& S, int row, int b, int p, int n
                              S.dsc, stage);
     }
   }
+  // the row's place in every block's list of the chunk path's slot table: all
+  // zero here, where the ranking hides the scattered stores, and the entries
+  // after it (behind the barriers)
+  uint16_t* trow = nullptr;
+  if (A.tab) {
+    trow = A.tab + (long)(row / A.seq) * A.max_blocks * A.seq + row % A.seq;
+    const int nb = table_blocks(p - row % A.seq, A.seq, A.ratio, A.max_blocks);
+    for (int j = tid; j < nb; j += NT) trow[(long)j * A.seq] = 0;
+  }
   __syncthreads();
   QM_PHASE(1);
   if (n_elig <= A.topk) {
@@ -1236,23 +1245,15 @@ __device__ void select_row(const SelArgs& A, SH& S, int row, int b, int p, int n
   }
   if (tid == 0) A.n_sel[row] = n_sel;
   if (A.tab) {
-    // the row of the chunk path's slot table, as qsa_chunk_bucket_kernel
-    // writes it, formed in LDS (the page list is only for items), and (max,
-    // sum) = (-inf, 0) for the slots this row leaves empty
-    uint16_t* slots = reinterpret_cast<uint16_t*>(S.pages);
-    const int nb = table_blocks(p - row % A.seq, A.seq, A.ratio, A.max_blocks);
-    for (int j = tid; j < nb; j += NT) slots[j] = 0;
-    __syncthreads();
-    for (int i = tid; i < n_sel; i += NT) slots[S.sel[i]] = static_cast<uint16_t>(i + 1);
+    // its entries, and (max, sum) = (-inf, 0) for the slots this row leaves
+    // empty, as qsa_chunk_bucket_kernel writes them
+    for (int i = tid; i < n_sel; i += NT) trow[(long)S.sel[i] * A.seq] = static_cast<uint16_t>(i + 1);
     const int nslot = A.topk + 1;
     for (int i = tid; i < nslot; i += NT) {
       // past the selection; the tail's slot when the row completes its block
       const bool empty = i < A.topk ? i >= n_sel : ((p + 1) / A.ratio) * A.ratio > p;
       if (empty) empty_partial(A.part_ml, row, A.hkv, nslot, i);
     }
-    __syncthreads();
-    uint16_t* trow = A.tab + (long)row * A.max_blocks;
-    for (int j = tid; j < nb; j += NT) trow[j] = slots[j];
   }
   if (!A.items) return;
   __syncthreads();
@@ -1831,28 +1832,30 @@ __global__ __launch_bounds__(QSA_D) void qsa_combine_rows_kernel(CombineArgs<T, 
 // The attention of a chunk of query rows reads each key/value block once. A
 // row's entries are its (row, slot) pairs: slot i < n_sel its i-th selected
 // block, slot topk its tail block (keys ts..p, when the row does not complete
-// its block). The entries are filed in a slot table, [B][seq][max_blocks]
-// uint16 in the workspace: entry (b, s, j) holds slot + 1 when row s selected
-// block j, else 0. Each row writes its whole row of the table (plain stores, no
-// atomics, so no round trip holds up the filing), and the attention gathers a
-// block's column of it. Nothing is kept in it between calls: a table that the
-// calls left zero for one another ([max_blocks][seq], cleared by the merge) lay
-// under the partials of shorter chunks on the same workspace, whose bits the
-// next longer chunk then read as slots. qm_qsa_attend_chunk is three
-// launches:
+// its block). The entries are filed in a slot table, [B][max_blocks][seq]
+// uint16 in the workspace: entry (b, j, s) holds slot + 1 when row s selected
+// block j, else 0. Each row writes its entry of every block's list (plain
+// stores, no atomics, so no round trip holds up the filing; scattered, but one
+// store where the attention's waves read it 4 n_kv_heads times), and the
+// attention reads a block's list in whole lines (with [B][seq][max_blocks] its
+// 128 gathered lines a wave took the attention of 128 rows at 32K from 26.1 to
+// 27.2 us). Nothing is kept in the table between calls: one that the calls
+// left zero for one another (cleared by the merge) lay under the partials of
+// shorter chunks on the same workspace, whose bits the next longer chunk then
+// read as slots. qm_qsa_attend_chunk is three launches:
 //   qsa_chunk_bucket   one 64-thread workgroup per row: writes the row's table
-//                      row and writes the empty partials (max
-//                      -inf) of its unused slots (qm_qsa_select_chunk does the
-//                      same inside the selection);
+//                      entries and the empty partials (max -inf) of its unused
+//                      slots (qm_qsa_select_chunk does the same inside the
+//                      selection);
 //   qsa_chunk_attend   grid (blocks + tail workgroups, kv head, sequence): the
-//                      workgroup of block j reads its table column and the page
+//                      workgroup of block j reads its table list and the page
 //                      with its first loads, then the block's 64 tokens of key
 //                      pieces straight into LDS (16 KB per 32 tokens) and of
 //                      value pieces into registers; each wave scores two
 //                      entries x 8 query heads on bf16 MFMA and writes one
 //                      partial per (row, slot, head): fp32 max and sum, and the
 //                      output normalised by the sum, in bf16. Every wave finds
-//                      the entries it needs from the table row by ballot, so
+//                      the entries it needs from the block's list by ballot, so
 //                      the workgroup's LDS is the keys and the softmax weights
 //                      alone (40 KB: four workgroups per compute unit). A tail
 //                      workgroup takes the tail entries of 8 rows (one or two
@@ -1872,7 +1875,7 @@ struct ChunkAttnArgs {
   uint16_t* part_o; float* part_ml;      // part_o: bf16, normalised by l
   const uint16_t* tab;                    // [B][max_blocks][seq]: slot + 1, or 0
   int batch, seq, hq, hkv, page_size, max_pages, ratio, topk, max_blocks, nwg_sel;
-  int seg_spans, nseg;                    // 128-row spans of a block's table column per workgroup, segments of a column
+  int seg_spans, nseg;                    // 128-row spans of a block's list per workgroup, segments of a list
   int row0, rows;                         // the rows of each sequence this launch takes (row0 a multiple of 128)
   float scale;
 };
@@ -1889,16 +1892,16 @@ __global__ __launch_bounds__(64) void qsa_chunk_bucket_kernel(ChunkBucketArgs A)
   const int nslot = A.topk + 1;
   const int nsel = A.n_sel[row];
   const int pos0 = A.positions[b], p = pos0 + s;
-  // the whole row, then its entries behind a barrier
-  uint16_t* trow = A.tab + (long)row * A.max_blocks;
+  // the row's place in every block's list, then its entries behind a barrier
+  uint16_t* trow = A.tab + (long)b * A.max_blocks * A.seq + s;
   const int nb = table_blocks(pos0, A.seq, A.ratio, A.max_blocks);
-  for (int j = lane; j < nb; j += 64) trow[j] = 0;
+  for (int j = lane; j < nb; j += 64) trow[(long)j * A.seq] = 0;
   __syncthreads();
   for (int i = lane; i < nslot; i += 64) {
     bool empty;
     if (i < A.topk) {
       empty = i >= nsel;
-      if (!empty) trow[A.ids[(long)row * A.topk + i]] = static_cast<uint16_t>(i + 1);
+      if (!empty) trow[(long)A.ids[(long)row * A.topk + i] * A.seq] = static_cast<uint16_t>(i + 1);
     } else {
       empty = ((p + 1) / A.ratio) * A.ratio > p;      // the row completes its block: no tail
     }
@@ -1914,7 +1917,7 @@ struct ChunkShared {
 };
 static_assert(sizeof(ChunkShared) == 40960, "four workgroups per compute unit");
 
-// The next 8 entries of a 128-row span of a block's table row, in row order:
+// The next 8 entries of a 128-row span of a block's list, in row order:
 // lane l holds rows (span base + l) and (span base + 64 + l) as `ma` / `mb` =
 // row << 16 | slot, and `ra` / `rb` are the rows of the span not yet taken
 // (bit l: lane l's row is an entry). Scalar work: the first set bits, read out
@@ -2156,24 +2159,24 @@ __global__ __launch_bounds__(CA_NT, 4) void qsa_chunk_attend_kernel(ChunkAttnArg
   };
 
   if (x < A.nwg_sel * A.nseg) {
-    // ---- block j, a segment of its table row: the first 128 rows of it, its
+    // ---- block j, a segment of its list: the first 128 rows of it, its
     // pages and the position in one round trip; then its entries in groups of 8
     const int sg = x / A.nwg_sel, j = x - sg * A.nwg_sel;
     const int row_end = A.row0 + A.rows;
     const int c0 = (A.row0 >> 7) + sg * A.seg_spans, c1 = min(c0 + A.seg_spans, (row_end + 127) >> 7);
-    const uint16_t* tcol = A.tab + row_b * A.max_blocks + j;     // row s's entry for this block at s * max_blocks
-    const int ta = 128 * c0 + lane < row_end ? tcol[(long)(128 * c0 + lane) * A.max_blocks] : 0;
-    const int tb = 128 * c0 + 64 + lane < row_end ? tcol[(long)(128 * c0 + 64 + lane) * A.max_blocks] : 0;
+    const uint16_t* tlist = A.tab + ((long)b * A.max_blocks + j) * A.seq;     // row s's entry for this block at s
+    const int ta = 128 * c0 + lane < row_end ? tlist[128 * c0 + lane] : 0;
+    const int tb = 128 * c0 + 64 + lane < row_end ? tlist[128 * c0 + 64 + lane] : 0;
     int page0, page1;
     pages_of(j, page0, page1);
     const int pos0 = A.positions[b];
     if (j >= table_blocks(pos0, A.seq, A.ratio, A.max_blocks)) return;     // past every row's blocks: no entries
     bool loaded = false, first = true;
     for (int c = c0; c < c1; ++c) {
-      // rows 128 c + lane and 128 c + 64 + lane of the table row
+      // rows 128 c + lane and 128 c + 64 + lane of the list
       const int ra = 128 * c + lane, rb = ra + 64;
-      const int tva = c == c0 ? ta : ra < row_end ? tcol[(long)ra * A.max_blocks] : 0;
-      const int tvb = c == c0 ? tb : rb < row_end ? tcol[(long)rb * A.max_blocks] : 0;
+      const int tva = c == c0 ? ta : ra < row_end ? tlist[ra] : 0;
+      const int tvb = c == c0 ? tb : rb < row_end ? tlist[rb] : 0;
       unsigned long long la = __ballot(tva != 0), lb = __ballot(tvb != 0);
       if ((la | lb) == 0ull) continue;
       const int nc = __popcll(la) + __popcll(lb);
