@@ -320,10 +320,13 @@ int hc_up_chunks(const qm_hc_geom& g) {   // 16-byte up chunks of one hc_up_mean
                                     : g.streams * HcTile<float>::HB * (g.rank / 4);
 }
 
-// rows of a workgroup's group: the fewest of 1, 2, 4 that cover M (at most
-// `cap`, and for hc_norm_down at most what fits HC_LDS)
+// rows of a workgroup's group (at most `cap`, and for hc_norm_down at most what
+// fits HC_LDS): all of one or two; pairs up to 8, where more workgroups with
+// half the LDS beat reading the weights once per four rows (bf16 mix, us, four
+// / two: 13.2 / 11.5 at 4 rows, 15.4 / 12.7 at 6, 15.4 / 15.0 at 8; a row's bits
+// are the same); four of more (geometries that hc_rows.hip does not cover)
 int hc_group_rows(int M, int cap) {
-  const int need = M >= 3 ? 4 : M;
+  const int need = M <= 2 ? M : M <= 8 ? 2 : 4;
   return need < cap ? need : cap;
 }
 
@@ -354,8 +357,8 @@ const char* hc_check(const qm_hc_geom* g) {
 }
 
 // Where the matrix-core kernels (hc_rows.hip) take over. They would be faster
-// from 3 rows on (whole mix, us, here and there: bf16 13.7 / 10.5 at 4 rows,
-// 16.0 / 10.6 at 5, 24.7 / 10.9 at 14; float 18.9 / 17.4 at 5, 35.6 / 18.2 at
+// from 4 rows on (whole mix, us, here and there: bf16 11.5 / 10.5 at 4 rows,
+// 12.7 / 10.6 at 5, 24.7 / 10.9 at 14; float 18.9 / 17.4 at 5, 35.6 / 18.2 at
 // 14), but these kernels give a row the same bits at every row count, and a
 // verify step's few drafted tokens should see the inputs that their single
 // steps saw: with another order of the sums the first layer's states came out
