@@ -9,17 +9,16 @@
 // into the residual streams (reference/model.py:79-81), with gemv.hip's
 // roundings.
 //
-// Work split: a workgroup takes TN tiles of 16 weight rows against 16 token
-// rows; its waves split k, 64 units (1 KB) of every row each. A wave reads
-// whole 1 KB row segments (a load that covers 16 rows x 64 bytes, the operand's
-// own shape, costs the address unit four times as much), all of them in flight
-// at once, and turns them into operands through LDS of its own, without a
-// barrier. The waves' partial results meet in LDS.
+// Work split: a workgroup takes TN tiles of 16 weight rows against MT tiles of
+// 16 token rows; its waves split k, 64 units (1 KB) of every row each. A wave
+// reads whole 1 KB row segments (not the operand's own shape, 16 rows x 64 bytes
+// a load: see to_frags), all of them in flight at once, and turns them into
+// operands through LDS of its own, without a barrier. The waves' partial results meet in LDS.
 //
 // Measured with weights from memory, against the library's GEMMs that served
 // these row counts (us): DeltaNet input projections (50 MB) 45.3 -> 13.8 at 16
-// rows (3.7 TB/s), 44.7 -> 20.6 at 32, 45.5 -> 33.9 at 64 (the weights are read
-// again per 16 rows, from cache); output projection (17 MB) 11.8 -> 6.5 at 16,
+// rows (3.7 TB/s), 44.7 -> 17.5 at 32, 45.5 -> 26.2 at 64 (the weights are read
+// once per 32 rows; once per 16 it was 20.6 and 33.9); output projection (17 MB) 11.8 -> 6.5 at 16,
 // with the reinjection's own launch (4.7 us) gone as well.
 #include "rows_mma.h"
 #include "qwen4mix_internal.h"
@@ -42,24 +41,28 @@ struct GemmRowsArgs {
   int streams;
 };
 
-// grid (ceil(N / (16 TN)), ceil(M / 16)), NW waves; K = NW * PASS * 64 units
-template <typename T, int NW, int PASS, int TN, bool RJ>
+// grid (ceil(N / (16 TN)), ceil(M / (16 MT))), NW waves; K = NW * PASS * 64 units
+template <typename T, int NW, int PASS, int TN, int MT, bool RJ>
 __global__ __launch_bounds__(64 * NW) void gemm_rows_kernel(GemmRowsArgs<T> A) {
   constexpr int VE = Chunk<T>::VE;
+  static_assert(TN * MT <= NW, "a wave finishes a 16x16 result");
   __shared__ uint4 s_rows[NW][16 * ROW_US];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int g4 = lane >> 4, r16 = lane & 15;
-  const int n0 = blockIdx.x * 16 * TN, m0 = blockIdx.y * 16;
-  const int m = m0 + r16;
-  RowAcc<T> acc[TN];
+  const int n0 = blockIdx.x * 16 * TN, m0 = blockIdx.y * 16 * MT;
+  // the result this wave finishes: weight tile wid / MT, token tile wid % MT
+  const int m = m0 + 16 * (wid % MT) + r16;
+  RowAcc<T> acc[TN][MT];
   float hv[GR_PRE][4], iv[GR_PRE];
 #pragma unroll
   for (int p = 0; p < PASS; ++p) {
     const long k0 = (long)((p * NW + wid) * 64 + lane) * VE;
-    u32x4_t xr[16], wr[TN][16];
+    u32x4_t xr[MT][16], wr[TN][16];
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
-      xr[r] = *reinterpret_cast<const u32x4_t*>(A.x + (long)min(m0 + r, A.M - 1) * A.K + k0);
+    for (int u = 0; u < MT; ++u)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        xr[u][r] = *reinterpret_cast<const u32x4_t*>(A.x + (long)min(m0 + 16 * u + r, A.M - 1) * A.K + k0);
 #pragma unroll
     for (int t = 0; t < TN; ++t)
 #pragma unroll
@@ -67,9 +70,9 @@ __global__ __launch_bounds__(64 * NW) void gemm_rows_kernel(GemmRowsArgs<T> A) {
         wr[t][r] = *reinterpret_cast<const u32x4_t*>(A.w + (long)min(n0 + 16 * t + r, A.N - 1) * A.K + k0);
     if constexpr (RJ) {
       // the residual values and inject weights of this lane's outputs, in the
-      // weights' round trip (wave t finishes tile t)
-      if (p == 0 && wid < TN) {
-        const int n = min(n0 + 16 * wid + 4 * g4, A.N - 4), mc = min(m, A.M - 1);
+      // weights' round trip
+      if (p == 0 && wid < TN * MT) {
+        const int n = min(n0 + 16 * (wid / MT) + 4 * g4, A.N - 4), mc = min(m, A.M - 1);
 #pragma unroll
         for (int s = 0; s < GR_PRE; ++s) {
           const int sc = min(s, A.streams - 1);
@@ -79,29 +82,34 @@ __global__ __launch_bounds__(64 * NW) void gemm_rows_kernel(GemmRowsArgs<T> A) {
       }
     }
     __builtin_amdgcn_sched_barrier(0);
-    u32x4_t xf[16], wf[16];
-    to_frags(s_rows[wid], xr, lane, r16, g4, xf);
+    u32x4_t xf[MT][16], wf[16];
+#pragma unroll
+    for (int u = 0; u < MT; ++u) to_frags(s_rows[wid], xr[u], lane, r16, g4, xf[u]);
 #pragma unroll
     for (int t = 0; t < TN; ++t) {
       to_frags(s_rows[wid], wr[t], lane, r16, g4, wf);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        acc[t].step(__builtin_bit_cast(uint4, wf[i]), __builtin_bit_cast(uint4, xf[i]));
-        if (i % 4 == 3) acc[t].block();
-      }
+      for (int i = 0; i < 16; ++i)
+#pragma unroll
+        for (int u = 0; u < MT; ++u) {
+          acc[t][u].step(__builtin_bit_cast(uint4, wf[i]), __builtin_bit_cast(uint4, xf[u][i]));
+          if (i % 4 == 3) acc[t][u].block();
+        }
     }
   }
-  // the waves' sums: lane holds rows n0 + 16 t + 4 g4 + i of token row m
-  f32x4_t* red = reinterpret_cast<f32x4_t*>(s_rows);       // [NW][TN][64]
+  // the waves' sums: lane holds rows n0 + 16 t + 4 g4 + i of token row m0 + 16 u + r16
+  f32x4_t* red = reinterpret_cast<f32x4_t*>(s_rows);       // [NW][TN * MT][64]
   __syncthreads();
 #pragma unroll
-  for (int t = 0; t < TN; ++t) red[(wid * TN + t) * 64 + lane] = acc[t].sum();
+  for (int t = 0; t < TN; ++t)
+#pragma unroll
+    for (int u = 0; u < MT; ++u) red[(wid * TN * MT + t * MT + u) * 64 + lane] = acc[t][u].sum();
   __syncthreads();
-  if (wid >= TN) return;
+  if (wid >= TN * MT) return;
   f32x4_t v = red[wid * 64 + lane];
 #pragma unroll
-  for (int w = 1; w < NW; ++w) v += red[(w * TN + wid) * 64 + lane];
-  const int n = n0 + 16 * wid + 4 * g4;
+  for (int w = 1; w < NW; ++w) v += red[(w * TN * MT + wid) * 64 + lane];
+  const int n = n0 + 16 * (wid / MT) + 4 * g4;
   if (m >= A.M || n >= A.N) return;
   if constexpr (RJ) {                                       // N is a multiple of 4
     float y[4];
@@ -143,10 +151,10 @@ __global__ __launch_bounds__(64 * NW) void gemm_rows_kernel(GemmRowsArgs<T> A) {
   }
 }
 
-template <typename T, int NW, int PASS, int TN, bool RJ>
+template <typename T, int NW, int PASS, int TN, int MT, bool RJ>
 int launch_tile(const GemmRowsArgs<T>& A, hipStream_t stream) {
-  hipLaunchKernelGGL((gemm_rows_kernel<T, NW, PASS, TN, RJ>),
-                     dim3((A.N + 16 * TN - 1) / (16 * TN), (A.M + 15) / 16), dim3(64 * NW), 0, stream, A);
+  hipLaunchKernelGGL((gemm_rows_kernel<T, NW, PASS, TN, MT, RJ>),
+                     dim3((A.N + 16 * TN - 1) / (16 * TN), (A.M + 16 * MT - 1) / (16 * MT)), dim3(64 * NW), 0, stream, A);
   QM_CHECK_LAUNCH();
   return QM_OK;
 }
@@ -154,10 +162,12 @@ int launch_tile(const GemmRowsArgs<T>& A, hipStream_t stream) {
 template <typename T, bool RJ>
 int launch_rows(const GemmRowsArgs<T>& A, hipStream_t stream) {
   const int segs = A.K / (64 * Chunk<T>::VE);               // 1 KB segments of a row
-  if (segs == 4) return launch_tile<T, 4, 1, 2, RJ>(A, stream);
-  if (segs == 8) return launch_tile<T, 8, 1, 1, RJ>(A, stream);
+  // four waves hold two weight tiles against one token tile, or one against
+  // two (more than 16 rows: the weights are then read once per 32)
+  if (segs == 4) return A.M <= 16 ? launch_tile<T, 4, 1, 2, 1, RJ>(A, stream) : launch_tile<T, 4, 1, 1, 2, RJ>(A, stream);
+  if (segs == 8) return launch_tile<T, 8, 1, 1, 1, RJ>(A, stream);
   if constexpr (sizeof(T) == 4)
-    if (segs == 16) return launch_tile<T, 8, 2, 1, RJ>(A, stream);
+    if (segs == 16) return launch_tile<T, 8, 2, 1, 1, RJ>(A, stream);
   return qm_fail(QM_ERR_UNSUPPORTED, "qm_gemm_rows: unsupported k");
 }
 

@@ -105,7 +105,7 @@ class Qwen4MixModel:
     # rows up to which qm_gemm_rows is faster than the library's GEMMs, by dtype:
     # for a group of projections of one input (one launch instead of four or
     # five; DeltaNet input, us, library / here, weights from memory: bf16 45.5 /
-    # 13.8 at 16 rows, 45.5 / 33.9 at 64; float 50.8 / 31.7 at 16, 52.7 / 50.6 at
+    # 13.8 at 16 rows, 45.5 / 26.2 at 64; float 50.8 / 31.7 at 16, 52.7 / 50.6 at
     # 32, 59.0 / 68.0 at 48) and for a single one (output: bf16 11.8 / 6.5 at
     # 16, 9.4 / 6.6 at 32, 9.5 / 10.6 at 48; float 12.2 / 13.2 at 5)
     GEMM_ROWS_MAX = {torch.bfloat16: (64, 32), torch.float32: (32, 0)}
