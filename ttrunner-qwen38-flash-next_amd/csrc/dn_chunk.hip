@@ -32,7 +32,9 @@ namespace {
 
 constexpr int CK_C = 64;          // tokens per chunk
 constexpr int CK_D = 128;         // d_k = d_v
-constexpr int CK_NT = 256;        // four waves
+constexpr int CK_NT = 256;        // scan: four waves
+constexpr int CP_NT = 512;        // prep: eight waves, two per SIMD (its LDS leaves one workgroup per compute
+                                  // unit); with four the rule over 4096 tokens took 292 us, now 271
 constexpr int CK_LD = CK_D + 4;   // LDS row stride of [token][dim] tiles, floats
 constexpr int CK_LT = CK_C + 4;   // LDS row stride of [.][token] tiles, floats
 constexpr int CK_COLS = 16;       // d_v columns per scan workgroup
@@ -253,7 +255,7 @@ struct alignas(16) PrepShared {
 };
 
 template <typename T>
-__global__ __launch_bounds__(CK_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A) {
+__global__ __launch_bounds__(CP_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A) {
   __shared__ PrepShared sh;
   QM_PHASE_DECL
   QM_PHASE(0);
@@ -275,10 +277,11 @@ __global__ __launch_bounds__(CK_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A
   const int span_sh = span == 1 ? 0 : 2;     // span is 1 or 4
   auto mine = [&](int quarter) __attribute__((always_inline)) { return (quarter >> span_sh) == part; };
 
-  // q, k, v rows: four threads per token, 32 dims each as four runs of 8
-  const int t = tid >> 2, p = tid & 3;
+  // q, k, v rows: eight threads per token, 16 dims each as two runs of 8; run
+  // j of thread p is unit p % 4 of the 32 dims 32 (2 j + p / 4) ..
+  const int t = tid >> 3, p = tid & 7;
   const bool tok_ok = t < n_valid;
-  float qn[32];
+  float qn[16];
   {
     // every load at once, the gates first (the cumulative decay is the
     // longest chain); indices are clamped so that no load sits in a branch
@@ -289,18 +292,18 @@ __global__ __launch_bounds__(CK_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A
     const float bv_raw = A.beta[tok * A.heads + h];
     const long qo = tok * A.q_stride + (long)(h % A.hk) * CK_D;
     const long vo = tok * A.v_stride + (long)h * CK_D;
-    Raw8<T> xq[4], xk[4], xv[4];
+    Raw8<T> xq[2], xk[2], xv[2];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int d = 8 * (p + 4 * j);
+    for (int j = 0; j < 2; ++j) {
+      const int d = 8 * (p + 8 * j);
       xq[j].load(A.q + qo + d);
       xk[j].load(A.k + qo + d);
       xv[j].load(A.v + vo + d);
     }
     __builtin_amdgcn_sched_barrier(0);
-    float kv[32], vv[32];
+    float kv[16], vv[16];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < 2; ++j) {
       xq[j].get(qn + 8 * j);
       xk[j].get(kv + 8 * j);
       xv[j].get(vv + 8 * j);
@@ -334,7 +337,7 @@ __global__ __launch_bounds__(CK_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A
 
     float sq = 0.f, sk = 0.f;
 #pragma unroll
-    for (int i = 0; i < 32; ++i) {
+    for (int i = 0; i < 16; ++i) {
       sq = fmaf(qn[i], qn[i], sq);
       sk = fmaf(kv[i], kv[i], sk);
     }
@@ -342,18 +345,20 @@ __global__ __launch_bounds__(CK_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A
     sk += dpp_f<0xB1>(sk);
     sq += dpp_f<0x4E>(sq);    // lane ^ 2
     sk += dpp_f<0x4E>(sk);
+    sq += dpp_f<0x141>(sq);   // the other quad of eight (its lanes agree by now)
+    sk += dpp_f<0x141>(sk);
     const float rq = tok_ok ? rsqrt_rn(sq + 1e-6f) : 0.f;
     const float rk = tok_ok ? rsqrt_rn(sk + 1e-6f) : 0.f;
     const float qscale = 0.08838834764831845f;  // 128^-1/2
 #pragma unroll
-    for (int i = 0; i < 32; ++i) {
+    for (int i = 0; i < 16; ++i) {
       qn[i] = mul_rn(mul_rn(qn[i], rq), qscale);
       kv[i] = mul_rn(kv[i], rk);
       vv[i] = vv[i] * bv;
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int d = 8 * (p + 4 * j);
+    for (int j = 0; j < 2; ++j) {
+      const int d = 8 * (p + 8 * j), dj = 2 * j + (p >> 2);      // the run's 32 dims
       float xq[8], xk[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) { xq[e] = qn[8 * j + e]; xk[e] = kv[8 * j + e]; }
@@ -363,15 +368,15 @@ __global__ __launch_bounds__(CK_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A
       *reinterpret_cast<bf16x8_t*>(&sh.kh[t * CK_HS + d]) = fk.hi;
       *reinterpret_cast<bf16x8_t*>(&sh.kl[t * CK_HS + d]) = fk.lo;
       // the [dim][token] copies only where this workgroup reads them: dims
-      // 32 j .. 32 j + 31 of k for its k_dec quarter (j == part) and, with
-      // parts, the w columns of parts 0-1 (k dims 64 part ..) and the u
-      // columns of parts 2-3 (v dims 64 (part - 2) ..); uniform per j
+      // 32 dj .. of k for its k_dec quarter (dj == part) and, with parts, the w
+      // columns of parts 0-1 (k dims 64 part ..) and the u columns of parts 2-3
+      // (v dims 64 (part - 2) ..)
       const bool all = A.parts == 1;
-      if (all || j == part || (part < 2 && j / 2 == part)) {
+      if (all || dj == part || (part < 2 && dj / 2 == part)) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) sh.kT[d + e][t] = kv[8 * j + e];
       }
-      if (all || (part >= 2 && j / 2 == part - 2)) {
+      if (all || (part >= 2 && dj / 2 == part - 2)) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) sh.vT[d + e][t] = vv[8 * j + e];
       }
@@ -381,16 +386,16 @@ __global__ __launch_bounds__(CK_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A
   __syncthreads();
   QM_PHASE(2);
 
-  // q e^cum fragments (QD: token block t / 16, dk step j) from the thread's
-  // own q values: its run j of 8 dims is lane t % 16 + 16 p of fragment j
+  // q e^cum fragments (QD: token block t / 16, dk step = the run's 32 dims)
+  // from the thread's own q values: a run of 8 dims is lane t % 16 + 16 (p % 4)
   if (mine(t >> 4)) {
     const float e = sh.ecum[t];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < 2; ++j) {
       float x[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i) x[i] = qn[8 * j + i] * e;
-      st_frag8(rec + CK_QD + ((t >> 4) * 4 + j) * FRAG2, (t & 15) + 16 * p, x);
+      st_frag8(rec + CK_QD + ((t >> 4) * 4 + 2 * j + (p >> 2)) * FRAG2, (t & 15) + 16 * (p & 3), x);
     }
   }
   QM_PHASE(10);
@@ -401,8 +406,8 @@ __global__ __launch_bounds__(CK_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A
   // ti % 4; this workgroup's tiles go round-robin to its waves
   {
     // this workgroup's tiles in order: ti = part, part + 4, part + 8 (one
-    // quarter) or all 12; the k-th goes to wave k % 4
-    for (int k = wid; k < 3 * span; k += 4) {
+    // quarter) or all 12; the k-th goes to wave k % 8
+    for (int k = wid; k < 3 * span; k += CP_NT / 64) {
       const int ti = span == 1 ? part + 4 * k : k;
       int I, J;
       if (ti < 10) tile_ij(ti, I, J);
@@ -434,43 +439,12 @@ __global__ __launch_bounds__(CK_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A
   float (&L)[CK_C][CK_LT] = sh.L;
   float (&Tm)[CK_C][CK_LT] = sh.u.Tm;
   // L = (k k^T) * beta_i * exp(cum_i - cum_j) for j < i
-  // three tile slots per wave, all fragments read before the first MFMA.
-  // Waves 0-2 take tiles (I, wid) for I = max(wid, 1) .. 3, so that block
-  // wid's fragments serve every slot as the B operand; wave 3 takes (3, 3)
-  // and (0, 0). Slots past a wave's tiles (wave 2's third, wave 3's third)
-  // repeat a tile and store nothing.
-  const int wu = __builtin_amdgcn_readfirstlane(wid);
-  const int ib = wu < 3 ? max(wu, 1) : 0;
-  int tI[3], tJ[3];
-#pragma unroll
-  for (int r = 0; r < 3; ++r) {
-    tI[r] = wu < 3 ? min(ib + r, 3) : (r == 0 ? 3 : 0);
-    tJ[r] = wu < 3 ? wu : tI[r];
-  }
-  Frag fb[4], fa[3][4];
-#pragma unroll
-  for (int st = 0; st < 4; ++st) fb[st] = tile_frag(sh.kh, sh.kl, 16 * tJ[0] + r16, st, g4);
-#pragma unroll
-  for (int r = 0; r < 3; ++r)
-#pragma unroll
-    for (int st = 0; st < 4; ++st) fa[r][st] = tile_frag(sh.kh, sh.kl, 16 * tI[r] + r16, st, g4);
-  __builtin_amdgcn_sched_barrier(0);
-  f32x4_t lacc[3];
-#pragma unroll
-  for (int r = 0; r < 3; ++r) lacc[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int st = 0; st < 4; ++st)
-#pragma unroll
-    for (int r = 0; r < 3; ++r) {
-      // wave 3's (0, 0) tile takes its own block as the B operand
-      const Frag& b = (wu == 3 && r > 0) ? fa[r][st] : fb[st];
-      lacc[r] = mfma3(fa[r][st], b, lacc[r]);
-    }
-#pragma unroll
-  for (int r = 0; r < 3; ++r) {
-    if (wu < 3 ? ib + r > 3 : r == 2) break;
-    const int I = tI[r], J = tJ[r];
-    const f32x4_t acc = lacc[r];
+  // ten tiles: wave w takes tile w, waves 4 and 5 (which had one q k^T tile
+  // fewer when a workgroup forms all of them) tiles 8 and 9 as well
+  for (int ti = wid; ti < 10; ti += ti == wid ? (wid == 4 || wid == 5 ? 4 : 10) : 10) {
+    int I, J;
+    tile_ij(ti, I, J);
+    const f32x4_t acc = gram16(sh.kh, sh.kl, 16 * I + r16, sh.kh, sh.kl, 16 * J + r16, g4);
     const int j = 16 * J + r16;
     const float cj = sh.cum[j];
     const float4 ci = lds4(&sh.cum[16 * I + 4 * g4]), bi = lds4(&sh.beta[16 * I + 4 * g4]);
@@ -515,15 +489,15 @@ __global__ __launch_bounds__(CK_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A
   } else {
     // the zero blocks (0, 1) and (2, 3) of T, which the 32-wide k-steps of
     // the w and u products read
-    for (int idx = tid - 64; idx < 2 * 256; idx += CK_NT - 64) {
+    for (int idx = tid - 64; idx < 2 * 256; idx += CP_NT - 64) {
       const int blk = idx >> 8, r = (idx >> 4) & 15, cc = idx & 15;
       Tm[32 * blk + r][32 * blk + 16 + cc] = 0.f;
     }
     // k_dec fragments (KD: dk blocks 2 quarter, 2 quarter + 1, token steps
     // 0..1): lane (dk 16 D + r16, tokens 32 s + 8 g4 ..); this workgroup's
-    // fragments are f0 .. f0 + 4 span, the i-th to wave 1 + i % 3
+    // fragments are f0 .. f0 + 4 span, the i-th to wave 1 + i % 7
     const int f0 = 4 * span * part;
-    for (int i = wid - 1; i < 4 * span; i += 3) {
+    for (int i = wid - 1; i < 4 * span; i += CP_NT / 64 - 1) {
       const int f = f0 + i;
       const int D = f >> 1, s = f & 1;
       const int c0 = 32 * s + 8 * g4;
@@ -563,9 +537,8 @@ __global__ __launch_bounds__(CK_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A
   // w = T (k beta e^cum) and u = T (v beta), as w^T = (k beta e^cum)^T T^T so
   // that a lane holds 4 consecutive dims of one token: quarter r holds column
   // tiles 4 r .. 4 r + 3 of the 16 (w: 0..7, u: 8..15, 16 dims each), one per
-  // wave; T is lower triangular, so row block I needs k-steps 0 .. I / 2
-  for (int qr = span * part; qr < span * (part + 1); ++qr) {
-    const int tile = 4 * qr + wid;
+  // wave at a time; T is lower triangular, so row block I needs k-steps 0 .. I / 2
+  for (int tile = 4 * span * part + wid; tile < 4 * span * (part + 1); tile += CP_NT / 64) {
     const bool is_u = tile >= 8;
     const int D = tile & 7;
     const float* arow = is_u ? &sh.vT[16 * D + r16][0] : &sh.kT[16 * D + r16][0];
@@ -811,7 +784,7 @@ int launch_chunked(int batch, int seq, int heads, int hk, long q_stride, long v_
     // few chunks: four workgroups per chunk so that the launch fills the chip;
     // many: one each, since every workgroup repeats the L and T work
     P.parts = (long)batch * heads * n_chunks < 256 ? CK_PARTS : 1;
-    hipLaunchKernelGGL(dn_chunk_prep_kernel<T>, dim3(batch * heads * n_chunks * P.parts), dim3(CK_NT), 0, stream, P);
+    hipLaunchKernelGGL(dn_chunk_prep_kernel<T>, dim3(batch * heads * n_chunks * P.parts), dim3(CP_NT), 0, stream, P);
     QM_CHECK_LAUNCH();
     ChunkScanArgs<T> S;
     S.ws = ws; S.state = state; S.out = static_cast<T*>(out);
