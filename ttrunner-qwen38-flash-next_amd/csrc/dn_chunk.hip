@@ -28,13 +28,15 @@
 #include "common.h"
 #include "qwen4mix_internal.h"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int CK_C = 64;          // tokens per chunk
 constexpr int CK_D = 128;         // d_k = d_v
 constexpr int CK_NT = 256;        // scan: four waves
-constexpr int CP_NT = 512;        // prep: eight waves, two per SIMD (its LDS leaves one workgroup per compute
-                                  // unit); with four the rule over 4096 tokens took 292 us, now 271
+constexpr int CP_NT = 512;        // prep: eight waves (the rule over 4096 tokens took 292 us with four, 271 with
+                                  // eight, one workgroup per compute unit by its LDS; 248 with two: PrepShared)
 constexpr int CK_LD = CK_D + 4;   // LDS row stride of [token][dim] tiles, floats
 constexpr int CK_LT = CK_C + 4;   // LDS row stride of [.][token] tiles, floats
 constexpr int CK_COLS = 16;       // d_v columns per scan workgroup
@@ -210,19 +212,16 @@ __device__ __forceinline__ Frag tile_frag(const uint16_t* hi, const uint16_t* lo
   return Frag{*reinterpret_cast<const bf16x8_t*>(hi + o), *reinterpret_cast<const bf16x8_t*>(lo + o)};
 }
 
-// 16x16 tile of X Y^T over the 128 dims from split [token][dim] tiles:
-// rows xr + l%16 of X and yr + l%16 of Y
-__device__ __forceinline__ f32x4_t gram16(const uint16_t* xh, const uint16_t* xl, int xr, const uint16_t* yh,
-                                          const uint16_t* yl, int yr, int g4) {
-  // every operand read before the first product, so that the reads' LDS
-  // latencies overlap instead of each product waiting on its own
-  Frag a[4], b[4];
-#pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    a[s] = tile_frag(xh, xl, xr, s, g4);
-    b[s] = tile_frag(yh, yl, yr, s, g4);
-  }
-  __builtin_amdgcn_sched_barrier(0);
+// the same operand from fp32 [row][dim] LDS rows (stride CK_LD), split on the way
+__device__ __forceinline__ Frag row_frag(const float* rows, int row, int s, int g4) {
+  const float* o = rows + row * CK_LD + 32 * s + 8 * g4;
+  const float4 a = lds4(o), b = lds4(o + 4);
+  const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+  return split8(x);
+}
+
+// 16x16 tile over the 128 dims of the products of two operands' rows
+__device__ __forceinline__ f32x4_t gram16(const Frag (&a)[4], const Frag (&b)[4]) {
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < 4; ++s) acc = mfma3(a[s], b[s], acc);
@@ -240,22 +239,30 @@ struct ChunkPrepArgs {
   long q_stride, v_stride;
 };
 
+// 71 KB, so that two workgroups of a compute unit run under each other's
+// barriers and latencies: k is held once, in fp32, and split as it is read;
+// L and T take q's place once the products with q and k are done; v, loaded
+// again only then, takes k's once w and k_dec are. 1024 chunks of fp32 took
+// 70.9 us with 158 KB and one workgroup, now 58.7 (240 KB of rows and record a
+// chunk: 4.3 TB/s); 64 chunks in parts 10.7 and 11.2, which is one workgroup
+// per compute unit either way.
 struct alignas(16) PrepShared {
   union {
     struct {
       uint16_t h[CK_C * CK_HS], l[CK_C * CK_HS];   // normalised q * d^-1/2, split
     } q;
-    float Tm[CK_C][CK_LT];     // (I + L)^-1, lower: after the q k^T tiles are done with q
+    struct {
+      float L[CK_C][CK_LT];    // (k beta k^T) * decay, strictly lower
+      float Tm[CK_C][CK_LT];   // (I + L)^-1, lower
+    } m;
   } u;
-  float L[CK_C][CK_LT];        // (k beta k^T) * decay, strictly lower (formed beside the q k^T tiles)
-  uint16_t kh[CK_C * CK_HS], kl[CK_C * CK_HS];     // normalised k, split
-  float kT[CK_D][CK_LT];       // normalised k, [dim][token]
-  float vT[CK_D][CK_LT];       // v * beta, [dim][token]
+  float kv[CK_C][CK_LD];       // normalised k, then v * beta: [token][dim]
   float cum[CK_C], beta[CK_C], ecum[CK_C], bec[CK_C], kds[CK_C];
 };
+static_assert(2 * (sizeof(PrepShared) + 256) <= 160 * 1024, "two workgroups per compute unit");
 
 template <typename T>
-__global__ __launch_bounds__(CP_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A) {
+__global__ __launch_bounds__(CP_NT, 4) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A) {
   __shared__ PrepShared sh;
   QM_PHASE_DECL
   QM_PHASE(0);
@@ -277,7 +284,7 @@ __global__ __launch_bounds__(CP_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A
   const int span_sh = span == 1 ? 0 : 2;     // span is 1 or 4
   auto mine = [&](int quarter) __attribute__((always_inline)) { return (quarter >> span_sh) == part; };
 
-  // q, k, v rows: eight threads per token, 16 dims each as two runs of 8; run
+  // q and k rows (v's below): eight threads per token, 16 dims each as two runs of 8; run
   // j of thread p is unit p % 4 of the 32 dims 32 (2 j + p / 4) ..
   const int t = tid >> 3, p = tid & 7;
   const bool tok_ok = t < n_valid;
@@ -289,26 +296,21 @@ __global__ __launch_bounds__(CP_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A
     const long gi = ((long)b * A.seq + t0 + (ok ? lane : 0)) * A.heads + h;
     const float g_raw = A.g[gi], b_raw = A.beta[gi];
     const long tok = (long)b * A.seq + t0 + (tok_ok ? t : 0);
-    const float bv_raw = A.beta[tok * A.heads + h];
     const long qo = tok * A.q_stride + (long)(h % A.hk) * CK_D;
-    const long vo = tok * A.v_stride + (long)h * CK_D;
-    Raw8<T> xq[2], xk[2], xv[2];
+    Raw8<T> xq[2], xk[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int d = 8 * (p + 8 * j);
       xq[j].load(A.q + qo + d);
       xk[j].load(A.k + qo + d);
-      xv[j].load(A.v + vo + d);
     }
     __builtin_amdgcn_sched_barrier(0);
-    float kv[16], vv[16];
+    float kv[16];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       xq[j].get(qn + 8 * j);
       xk[j].get(kv + 8 * j);
-      xv[j].get(vv + 8 * j);
     }
-    const float bv = tok_ok ? bv_raw : 0.f;
 
     // gates; padding tokens carry g = 0 and beta = 0
     if (wid == 0) {
@@ -354,32 +356,19 @@ __global__ __launch_bounds__(CP_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A
     for (int i = 0; i < 16; ++i) {
       qn[i] = mul_rn(mul_rn(qn[i], rq), qscale);
       kv[i] = mul_rn(kv[i], rk);
-      vv[i] = vv[i] * bv;
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      const int d = 8 * (p + 8 * j), dj = 2 * j + (p >> 2);      // the run's 32 dims
-      float xq[8], xk[8];
+      const int d = 8 * (p + 8 * j);
+      float xq[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) { xq[e] = qn[8 * j + e]; xk[e] = kv[8 * j + e]; }
-      const Frag fq = split8(xq), fk = split8(xk);
+      for (int e = 0; e < 8; ++e) xq[e] = qn[8 * j + e];
+      const Frag fq = split8(xq);
       *reinterpret_cast<bf16x8_t*>(&sh.u.q.h[t * CK_HS + d]) = fq.hi;
       *reinterpret_cast<bf16x8_t*>(&sh.u.q.l[t * CK_HS + d]) = fq.lo;
-      *reinterpret_cast<bf16x8_t*>(&sh.kh[t * CK_HS + d]) = fk.hi;
-      *reinterpret_cast<bf16x8_t*>(&sh.kl[t * CK_HS + d]) = fk.lo;
-      // the [dim][token] copies only where this workgroup reads them: dims
-      // 32 dj .. of k for its k_dec quarter (dj == part) and, with parts, the w
-      // columns of parts 0-1 (k dims 64 part ..) and the u columns of parts 2-3
-      // (v dims 64 (part - 2) ..)
-      const bool all = A.parts == 1;
-      if (all || dj == part || (part < 2 && dj / 2 == part)) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) sh.kT[d + e][t] = kv[8 * j + e];
-      }
-      if (all || (part >= 2 && dj / 2 == part - 2)) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) sh.vT[d + e][t] = vv[8 * j + e];
-      }
+      *reinterpret_cast<float4*>(&sh.kv[t][d]) = make_float4(kv[8 * j], kv[8 * j + 1], kv[8 * j + 2], kv[8 * j + 3]);
+      *reinterpret_cast<float4*>(&sh.kv[t][d + 4]) =
+          make_float4(kv[8 * j + 4], kv[8 * j + 5], kv[8 * j + 6], kv[8 * j + 7]);
     }
   }
   QM_PHASE(1);
@@ -413,7 +402,15 @@ __global__ __launch_bounds__(CP_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A
       if (ti < 10) tile_ij(ti, I, J);
       else { I = ti == 10 ? 0 : 2; J = I + 1; }
       f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-      if (ti < 10) acc = gram16(sh.kh, sh.kl, 16 * J + r16, sh.u.q.h, sh.u.q.l, 16 * I + r16, g4);
+      if (ti < 10) {
+        Frag fk[4], fq[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          fk[s] = row_frag(&sh.kv[0][0], 16 * J + r16, s, g4);
+          fq[s] = tile_frag(sh.u.q.h, sh.u.q.l, 16 * I + r16, s, g4);
+        }
+        acc = gram16(fk, fq);
+      }
       // the decays' operands are read before any exponential, outside the
       // masks, so that their LDS latencies overlap
       const int i = 16 * I + r16;
@@ -432,57 +429,77 @@ __global__ __launch_bounds__(CP_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A
     }
   }
   QM_PHASE(3);
-  // L has its own LDS, so its tiles follow the q k^T tiles with no barrier
-  // (T takes q's space after the barrier below)
-  QM_PHASE(9);
-
-  float (&L)[CK_C][CK_LT] = sh.L;
-  float (&Tm)[CK_C][CK_LT] = sh.u.Tm;
-  // L = (k k^T) * beta_i * exp(cum_i - cum_j) for j < i
-  // ten tiles: wave w takes tile w, waves 4 and 5 (which had one q k^T tile
-  // fewer when a workgroup forms all of them) tiles 8 and 9 as well
-  for (int ti = wid; ti < 10; ti += ti == wid ? (wid == 4 || wid == 5 ? 4 : 10) : 10) {
-    int I, J;
-    tile_ij(ti, I, J);
-    const f32x4_t acc = gram16(sh.kh, sh.kl, 16 * I + r16, sh.kh, sh.kl, 16 * J + r16, g4);
-    const int j = 16 * J + r16;
-    const float cj = sh.cum[j];
-    const float4 ci = lds4(&sh.cum[16 * I + 4 * g4]), bi = lds4(&sh.beta[16 * I + 4 * g4]);
-    const float civ[4] = {ci.x, ci.y, ci.z, ci.w}, biv[4] = {bi.x, bi.y, bi.z, bi.w};
+  // L = (k k^T) * beta_i * exp(cum_i - cum_j) for j < i: ten tiles, wave w
+  // forms tile w, waves 4 and 5 (which had one q k^T tile fewer when a workgroup
+  // forms all of them) tiles 8 and 9 as well; q's space takes them when every
+  // wave is done with q
+  float (&L)[CK_C][CK_LT] = sh.u.m.L;
+  float (&Tm)[CK_C][CK_LT] = sh.u.m.Tm;
+  const int n_l = wid == 4 || wid == 5 ? 2 : 1;
+  f32x4_t lacc[2];
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int i = 16 * I + 4 * g4 + v;
-      const float val = (acc[v] * biv[v]) * expf(civ[v] - cj);
-      L[i][j] = i > j ? val : 0.f;
+  for (int n = 0; n < 2; ++n)
+    if (n < n_l) {
+      int I, J;
+      tile_ij(wid + 4 * n, I, J);
+      Frag fi[4], fj[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        fi[s] = row_frag(&sh.kv[0][0], 16 * I + r16, s, g4);
+        fj[s] = row_frag(&sh.kv[0][0], 16 * J + r16, s, g4);
+      }
+      lacc[n] = gram16(fi, fj);
+      const int j = 16 * J + r16;
+      const float cj = sh.cum[j];
+      const float4 ci = lds4(&sh.cum[16 * I + 4 * g4]), bi = lds4(&sh.beta[16 * I + 4 * g4]);
+      const float civ[4] = {ci.x, ci.y, ci.z, ci.w}, biv[4] = {bi.x, bi.y, bi.z, bi.w};
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float val = (lacc[n][v] * biv[v]) * expf(civ[v] - cj);
+        lacc[n][v] = 16 * I + 4 * g4 + v > j ? val : 0.f;
+      }
     }
-  }
+  QM_PHASE(9);
+  __syncthreads();
+#pragma unroll
+  for (int n = 0; n < 2; ++n)
+    if (n < n_l) {
+      int I, J;
+      tile_ij(wid + 4 * n, I, J);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) L[16 * I + 4 * g4 + v][16 * J + r16] = lacc[n][v];
+    }
   QM_PHASE(4);
   __syncthreads();
 
   if (wid == 0) {
     // (I + L_II)^-1 for the four diagonal blocks; lane = (block, column):
     // x_i = [i == col] - sum_{k<i} L_ik x_k
-    // the block's lower triangle is read first (rows in runs of 4, the
-    // zeros above the diagonal included), so that the substitution's
-    // dependent chain waits on no LDS read
+    // the block's lower triangle is read ahead (rows in runs of 4, the zeros
+    // above the diagonal included; rows 1..8, then 9..15: registers), so that
+    // the substitution's dependent chain waits on two LDS round trips alone
     const int I = g4, col = r16;
-    float4 lr[15][4];
-#pragma unroll
-    for (int i = 1; i < 16; ++i)
-#pragma unroll
-      for (int k4 = 0; k4 < (i + 3) / 4; ++k4) lr[i - 1][k4] = lds4(&L[16 * I + i][16 * I + 4 * k4]);
-    __builtin_amdgcn_sched_barrier(0);
     float x[16];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      float acc = i == col ? 1.f : 0.f;
+    for (int half = 0; half < 2; ++half) {
+      const int i0 = half ? 9 : 1, i1 = half ? 16 : 9;
+      float4 lr[8][4];
 #pragma unroll
-      for (int kk = 0; kk < i; ++kk) {
-        const float4 v = lr[i - 1][kk / 4];
-        const float l = kk % 4 == 0 ? v.x : kk % 4 == 1 ? v.y : kk % 4 == 2 ? v.z : v.w;
-        acc = fmaf(-l, x[kk], acc);
+      for (int i = i0; i < i1; ++i)
+#pragma unroll
+        for (int k4 = 0; k4 < (i + 3) / 4; ++k4) lr[i - i0][k4] = lds4(&L[16 * I + i][16 * I + 4 * k4]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = half ? i0 : 0; i < i1; ++i) {
+        float acc = i == col ? 1.f : 0.f;
+#pragma unroll
+        for (int kk = 0; kk < i; ++kk) {
+          const float4 v = lr[i - i0][kk / 4];
+          const float l = kk % 4 == 0 ? v.x : kk % 4 == 1 ? v.y : kk % 4 == 2 ? v.z : v.w;
+          acc = fmaf(-l, x[kk], acc);
+        }
+        x[i] = acc;
       }
-      x[i] = acc;
     }
 #pragma unroll
     for (int i = 0; i < 16; ++i) Tm[16 * I + i][16 * I + col] = x[i];
@@ -501,13 +518,20 @@ __global__ __launch_bounds__(CP_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A
       const int f = f0 + i;
       const int D = f >> 1, s = f & 1;
       const int c0 = 32 * s + 8 * g4;
-      const float* row = &sh.kT[16 * D + r16][0];
-      const float4 x0 = lds4(row + c0), x1 = lds4(row + c0 + 4);
-      float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+      float x[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] *= sh.kds[c0 + e];
+      for (int e = 0; e < 8; ++e) x[e] = sh.kv[c0 + e][16 * D + r16] * sh.kds[c0 + e];
       st_frag8(rec + CK_KD + f * FRAG2, lane, x);
     }
+  }
+  // the v rows come in under the rest of T and w (their place is k's, below)
+  const bool has_w = A.parts == 1 || part < 2, has_u = A.parts == 1 || part >= 2;
+  Raw8<T> xv[2];
+  {
+    const T* vp = A.v + ((long)b * A.seq + t0 + (tok_ok ? t : 0)) * A.v_stride + (long)h * CK_D;
+    if (has_u)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) xv[j].load(vp + 8 * (p + 8 * j));
   }
   QM_PHASE(5);
   __syncthreads();
@@ -536,22 +560,25 @@ __global__ __launch_bounds__(CP_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A
   QM_PHASE(7);
   // w = T (k beta e^cum) and u = T (v beta), as w^T = (k beta e^cum)^T T^T so
   // that a lane holds 4 consecutive dims of one token: quarter r holds column
-  // tiles 4 r .. 4 r + 3 of the 16 (w: 0..7, u: 8..15, 16 dims each), one per
-  // wave at a time; T is lower triangular, so row block I needs k-steps 0 .. I / 2
-  for (int tile = 4 * span * part + wid; tile < 4 * span * (part + 1); tile += CP_NT / 64) {
-    const bool is_u = tile >= 8;
+  // tiles 4 r .. 4 r + 3 of the 16 (w: 0..7, u: 8..15, 16 dims each), at most
+  // eight of either kind a workgroup, one per wave; T is lower triangular, so
+  // row block I needs k-steps 0 .. I / 2
+  auto column_tile = [&](int tile, auto is_u) __attribute__((always_inline)) {
     const int D = tile & 7;
-    const float* arow = is_u ? &sh.vT[16 * D + r16][0] : &sh.kT[16 * D + r16][0];
-    // every LDS read first (the A row and its scales, the T rows of the four
-    // row blocks), then the splits and products
-    float4 ar[2][2], sc[2][2], tr[4][2][2];
+    float x[2][8];
+    float4 tr[4][2][2];
 #pragma unroll
-    for (int s2 = 0; s2 < 2; ++s2) {
-      const int c = 32 * s2 + 8 * g4;
-      ar[s2][0] = lds4(arow + c);
-      ar[s2][1] = lds4(arow + c + 4);
-      sc[s2][0] = lds4(&sh.bec[c]);
-      sc[s2][1] = lds4(&sh.bec[c + 4]);
+    for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[s2][e] = sh.kv[32 * s2 + 8 * g4 + e][16 * D + r16];
+    if constexpr (!is_u.value) {
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2) {
+        const float4 y0 = lds4(&sh.bec[32 * s2 + 8 * g4]), y1 = lds4(&sh.bec[32 * s2 + 8 * g4 + 4]);
+        const float y[8] = {y0.x, y0.y, y0.z, y0.w, y1.x, y1.y, y1.z, y1.w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[s2][e] *= y[e];
+      }
     }
 #pragma unroll
     for (int I = 0; I < 4; ++I)
@@ -561,30 +588,18 @@ __global__ __launch_bounds__(CP_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A
         tr[I][s2][0] = lds4(&Tm[16 * I + r16][c]);
         tr[I][s2][1] = lds4(&Tm[16 * I + r16][c + 4]);
       }
-    __builtin_amdgcn_sched_barrier(0);
-    Frag a[2];
-#pragma unroll
-    for (int s2 = 0; s2 < 2; ++s2) {
-      float x[8] = {ar[s2][0].x, ar[s2][0].y, ar[s2][0].z, ar[s2][0].w,
-                    ar[s2][1].x, ar[s2][1].y, ar[s2][1].z, ar[s2][1].w};
-      const float y[8] = {sc[s2][0].x, sc[s2][0].y, sc[s2][0].z, sc[s2][0].w,
-                          sc[s2][1].x, sc[s2][1].y, sc[s2][1].z, sc[s2][1].w};
-      if (!is_u)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] *= y[e];
-      a[s2] = split8(x);
-    }
+    const Frag a[2] = {split8(x[0]), split8(x[1])};
 #pragma unroll
     for (int I = 0; I < 4; ++I) {
       f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int s2 = 0; s2 <= I / 2; ++s2) {
-        const float x[8] = {tr[I][s2][0].x, tr[I][s2][0].y, tr[I][s2][0].z, tr[I][s2][0].w,
+        const float y[8] = {tr[I][s2][0].x, tr[I][s2][0].y, tr[I][s2][0].z, tr[I][s2][0].w,
                             tr[I][s2][1].x, tr[I][s2][1].y, tr[I][s2][1].z, tr[I][s2][1].w};
-        acc = mfma3(a[s2], split8(x), acc);
+        acc = mfma3(a[s2], split8(y), acc);
       }
       // acc[v]: dim 16 D + 4 g4 + v of token 16 I + r16
-      if (is_u) {
+      if constexpr (is_u.value) {
         *reinterpret_cast<float4*>(rec + CK_U + (16 * I + r16) * CK_D + 16 * D + 4 * g4) =
             make_float4(acc[0], acc[1], acc[2], acc[3]);
       } else {
@@ -593,6 +608,25 @@ __global__ __launch_bounds__(CP_NT) void dn_chunk_prep_kernel(ChunkPrepArgs<T> A
         st_frag4(rec + CK_W + (I * 4 + D / 2) * FRAG2, r16 + 16 * lg, e0, acc[0], acc[1], acc[2], acc[3]);
       }
     }
+  };
+  const int n_col = span == 1 ? 4 : 8;       // column tiles of each kind
+  if (has_w) {
+    if (wid < n_col) column_tile(4 * span * part + wid, std::false_type{});
+    __syncthreads();                         // every wave is done with k
+  }
+  if (has_u) {
+    // without w tiles, k_dec's reads of k ended before the barriers above
+    const float bv = sh.beta[t];             // 0 for padding tokens
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      float vv[8];
+      xv[j].get(vv);
+      float* dst = &sh.kv[t][8 * (p + 8 * j)];
+      *reinterpret_cast<float4*>(dst) = make_float4(vv[0] * bv, vv[1] * bv, vv[2] * bv, vv[3] * bv);
+      *reinterpret_cast<float4*>(dst + 4) = make_float4(vv[4] * bv, vv[5] * bv, vv[6] * bv, vv[7] * bv);
+    }
+    __syncthreads();
+    if (wid < n_col) column_tile((span == 1 ? 4 * part : 8) + wid, std::true_type{});
   }
   QM_PHASE(8);
   QM_PHASE_FLUSH();
