@@ -22,9 +22,11 @@
 // three bf16 MFMAs where the same 16x16x32 product takes eight fp32
 // 16x16x4 MFMAs of twice the cycles each. Operand lanes: A[row l%16][k 8(l/16)
 // + e], B[k 8(l/16) + e][col l%16], e < 8; result rows 4(l/16)+i, col l%16.
-// The scan works on transposed products (S^T w^T, S^T q_dec^T, v_new^T qk^T,
-// v_new^T k_dec), so that the state's A operand and every record operand are
-// runs of 8 consecutive elements in memory.
+// The state and v_new lie in LDS as [column][dk] and [column][token], so that
+// they and every record operand are runs of 8 consecutive elements; either can
+// be the A or the B operand (the lane layouts are alike), and which it is says
+// whether a lane's 4 results lie along the row or the column: w S and k_dec^T
+// v_new come out along [column]'s rows, the output along its channels.
 #include "common.h"
 #include "qwen4mix_internal.h"
 
@@ -53,7 +55,7 @@ constexpr int CK_PARTS = 4;       // prep workgroups per chunk when chunks are f
 //   QD   q e^cum [tok][dk] (q l2-normalised, scaled by d^-1/2)          4 x 4
 //   QK   (q k^T)[i][j] * decay, j <= i          (i block, j step)       4 x 2
 //   KD   k e^(cum_last - cum), as [dk][tok]     (dk block, token step)  8 x 2
-//   U    u = T (v beta) [tok][dv], fp32 row-major
+//   U    u = T (v beta) as [dv][tok], fp32
 //   ECL  e^cum_last in element 0
 constexpr long FRAG2 = 512;
 constexpr long CK_W = 0;
@@ -558,8 +560,9 @@ __global__ __launch_bounds__(CP_NT, 4) void dn_chunk_prep_kernel(ChunkPrepArgs<T
   }
 
   QM_PHASE(7);
-  // w = T (k beta e^cum) and u = T (v beta), as w^T = (k beta e^cum)^T T^T so
-  // that a lane holds 4 consecutive dims of one token: quarter r holds column
+  // w = T (k beta e^cum), as w^T = (k beta e^cum)^T T^T so that a lane holds 4
+  // consecutive dims of one token, and u = T (v beta), a lane 4 consecutive
+  // tokens of one dim: quarter r holds column
   // tiles 4 r .. 4 r + 3 of the 16 (w: 0..7, u: 8..15, 16 dims each), at most
   // eight of either kind a workgroup, one per wave; T is lower triangular, so
   // row block I needs k-steps 0 .. I / 2
@@ -596,13 +599,14 @@ __global__ __launch_bounds__(CP_NT, 4) void dn_chunk_prep_kernel(ChunkPrepArgs<T
       for (int s2 = 0; s2 <= I / 2; ++s2) {
         const float y[8] = {tr[I][s2][0].x, tr[I][s2][0].y, tr[I][s2][0].z, tr[I][s2][0].w,
                             tr[I][s2][1].x, tr[I][s2][1].y, tr[I][s2][1].z, tr[I][s2][1].w};
-        acc = mfma3(a[s2], split8(y), acc);
+        acc = is_u.value ? mfma3(split8(y), a[s2], acc) : mfma3(a[s2], split8(y), acc);
       }
-      // acc[v]: dim 16 D + 4 g4 + v of token 16 I + r16
       if constexpr (is_u.value) {
-        *reinterpret_cast<float4*>(rec + CK_U + (16 * I + r16) * CK_D + 16 * D + 4 * g4) =
+        // acc[v]: token 16 I + 4 g4 + v of dim 16 D + r16
+        *reinterpret_cast<float4*>(rec + CK_U + (16 * D + r16) * CK_C + 16 * I + 4 * g4) =
             make_float4(acc[0], acc[1], acc[2], acc[3]);
       } else {
+        // acc[v]: dim 16 D + 4 g4 + v of token 16 I + r16
         int lg, e0;
         frag_slot(D, g4, lg, e0);
         st_frag4(rec + CK_W + (I * 4 + D / 2) * FRAG2, r16 + 16 * lg, e0, acc[0], acc[1], acc[2], acc[3]);
@@ -643,7 +647,7 @@ struct ChunkScanArgs {
 
 // A wave's record operands of one chunk, none of which depends on the
 // state: the W and QD fragments of its token block (dk steps 0..3), the QK
-// fragments of its token block (j steps 0..1), the KD fragments of its two dk
+// fragments of its token block (j steps 0..1, the second from block 2 on), the KD fragments of its two dk
 // blocks (token steps 0..1), its 4 values of u and e^cum_last.
 struct ScanOps {
   Frag w[4], qd[4], qk[2], kd[2][2];
@@ -659,12 +663,13 @@ __device__ __forceinline__ void load_scan_ops(const float* rec, int wid, int lan
     o.qd[s] = ld_frag(rec + CK_QD + (wid * 4 + s) * FRAG2, lane);
   }
 #pragma unroll
-  for (int s = 0; s < 2; ++s) o.qk[s] = ld_frag(rec + CK_QK + (wid * 2 + s) * FRAG2, lane);
+  for (int s = 0; s < 2; ++s)
+    if (s == 0 || wid >= 2) o.qk[s] = ld_frag(rec + CK_QK + (wid * 2 + s) * FRAG2, lane);
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int s = 0; s < 2; ++s) o.kd[t][s] = ld_frag(rec + CK_KD + ((2 * wid + t) * 2 + s) * FRAG2, lane);
-  o.u = *reinterpret_cast<const float4*>(rec + CK_U + (16 * wid + r16) * CK_D + col0 + 4 * g4);
+  o.u = *reinterpret_cast<const float4*>(rec + CK_U + (col0 + r16) * CK_C + 16 * wid + 4 * g4);
   o.ecl = rec[CK_ECL];
 }
 
@@ -677,21 +682,29 @@ __device__ __forceinline__ Frag lds_frag(const uint16_t* hi, const uint16_t* lo,
   return Frag{*reinterpret_cast<const bf16x8_t*>(hi + o), *reinterpret_cast<const bf16x8_t*>(lo + o)};
 }
 
-// columns c and c + 1 of row `r` of a [column][.] bf16 hi / lo tile pair from
-// two split values
-__device__ __forceinline__ void put2(uint16_t* hi, uint16_t* lo, int stride, int c, int r, float a, float b) {
-  unsigned hh, ll;
-  split2(a, b, hh, ll);
-  hi[c * stride + r] = static_cast<uint16_t>(hh);
-  hi[(c + 1) * stride + r] = static_cast<uint16_t>(hh >> 16);
-  lo[c * stride + r] = static_cast<uint16_t>(ll);
-  lo[(c + 1) * stride + r] = static_cast<uint16_t>(ll >> 16);
+// four consecutive elements (from r) of column c of a [column][.] bf16 hi / lo tile pair
+__device__ __forceinline__ void put4(uint16_t* hi, uint16_t* lo, int stride, int c, int r, float a, float b, float d,
+                                     float e) {
+  unsigned h0, l0, h1, l1;
+  split2(a, b, h0, l0);
+  split2(d, e, h1, l1);
+  *reinterpret_cast<uint2*>(hi + c * stride + r) = make_uint2(h0, h1);
+  *reinterpret_cast<uint2*>(lo + c * stride + r) = make_uint2(l0, l1);
 }
 
+// The record loads bound a chunk (109 KB for each of the eight column slices of
+// a head, from the die's cache at about 24 bytes a clock and compute unit),
+// then its dependent chain (state -> w S -> v_new -> state), 1.4 of 2.25 us a
+// chunk when timed without the loads, one wave per SIMD: so nothing is loaded
+// that no product takes, every operand is read before its first product, v_new
+// and the state come out of their products as 4 consecutive elements of a
+// tile's row (one 8-byte LDS write each of high and low parts), and the output's
+// products follow the ones that the chain needs. The chain alone: 1.42 -> 1.23
+// us; the rule over 4096 tokens in fp32 257 -> 240 us, 4000 in bf16 229 -> 224.
 template <typename T>
 __global__ __launch_bounds__(CK_NT) void dn_chunk_scan_kernel(ChunkScanArgs<T> A) {
   // the state slice S^T [column][dk] and the chunk's v_new^T [column][token],
-  // as bf16 high and low parts (the A operands of the transposed products)
+  // as bf16 high and low parts
   __shared__ __attribute__((aligned(16))) uint16_t sSh[CK_COLS * SC_SS], sSl[CK_COLS * SC_SS];
   __shared__ __attribute__((aligned(16))) uint16_t sVh[CK_COLS * SC_SV], sVl[CK_COLS * SC_SV];
   QM_PHASE_DECL
@@ -702,19 +715,18 @@ __global__ __launch_bounds__(CK_NT) void dn_chunk_scan_kernel(ChunkScanArgs<T> A
   const int sl = wg % NSL, bh = wg / NSL;
   const int h = bh % A.heads, b = bh / A.heads;
   const int col0 = sl * CK_COLS;
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g4 = lane >> 4, r16 = lane & 15;
   const float* recs = A.ws + (long)bh * A.n_chunks * CK_REC;
 
   // wave wid keeps dk rows 32 wid .. 32 wid + 31 of the slice as two result
-  // tiles of S^T: st[t][i] = S[dk 32 wid + 16 t + r16][column 4 g4 + i]
-  float* S = A.state + (long)bh * CK_D * CK_D + col0 + 4 * g4;
+  // tiles: st[t][i] = S[dk 32 wid + 16 t + 4 g4 + i][column r16]
+  float* S = A.state + (long)bh * CK_D * CK_D + (long)(32 * wid + 4 * g4) * CK_D + col0 + r16;
   f32x4_t st[2];
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const float4 x = *reinterpret_cast<const float4*>(S + (long)(32 * wid + 16 * t + r16) * CK_D);
-    st[t] = f32x4_t{x.x, x.y, x.z, x.w};
-  }
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) st[t][i] = S[(16 * t + i) * CK_D];
   // operands two chunks ahead: three register sets, the loop unrolled by
   // three so that no set is copied while its loads are in flight. The state
   // and the first two chunks' operands are requested together: the state
@@ -724,32 +736,45 @@ __global__ __launch_bounds__(CK_NT) void dn_chunk_scan_kernel(ChunkScanArgs<T> A
   load_scan_ops(recs + (long)min(1, A.n_chunks - 1) * CK_REC, wid, lane, r16, g4, col0, o1);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    put2(sSh, sSl, SC_SS, 4 * g4, 32 * wid + 16 * t + r16, st[t][0], st[t][1]);
-    put2(sSh, sSl, SC_SS, 4 * g4 + 2, 32 * wid + 16 * t + r16, st[t][2], st[t][3]);
-  }
+  for (int t = 0; t < 2; ++t)
+    put4(sSh, sSl, SC_SS, r16, 32 * wid + 16 * t + 4 * g4, st[t][0], st[t][1], st[t][2], st[t][3]);
   QM_PHASE(1);
 
   auto chunk = [&](int ci, const ScanOps& cur, ScanOps& ahead) {
     // chunk ci + 2's operands fly during this one
     if (ci + 2 < A.n_chunks) load_scan_ops(recs + (long)(ci + 2) * CK_REC, wid, lane, r16, g4, col0, ahead);
     __syncthreads();
-    // (w S)^T and (q_dec S)^T for tokens 16 wid ..: rows = columns 4 g4 + i,
-    // column = token 16 wid + r16
-    f32x4_t aw = {0.f, 0.f, 0.f, 0.f}, ao = {0.f, 0.f, 0.f, 0.f};
+    Frag sa[4];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const Frag sa = lds_frag(sSh, sSl, SC_SS, r16, s, g4);
-      aw = mfma3(sa, cur.w[s], aw);
-      ao = mfma3(sa, cur.qd[s], ao);
-    }
-    put2(sVh, sVl, SC_SV, 4 * g4, 16 * wid + r16, cur.u.x - aw[0], cur.u.y - aw[1]);
-    put2(sVh, sVl, SC_SV, 4 * g4 + 2, 16 * wid + r16, cur.u.z - aw[2], cur.u.w - aw[3]);
+    for (int s = 0; s < 4; ++s) sa[s] = lds_frag(sSh, sSl, SC_SS, r16, s, g4);
+    __builtin_amdgcn_sched_barrier(0);
+    // w S for tokens 16 wid ..: rows = tokens 16 wid + 4 g4 + i, column r16
+    f32x4_t aw = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < 4; ++s) aw = mfma3(cur.w[s], sa[s], aw);
+    put4(sVh, sVl, SC_SV, r16, 16 * wid + 4 * g4, cur.u.x - aw[0], cur.u.y - aw[1], cur.u.z - aw[2],
+         cur.u.w - aw[3]);
+    // (q_dec S)^T: rows = columns 4 g4 + i, column = token 16 wid + r16
+    f32x4_t ao = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < 4; ++s) ao = mfma3(sa[s], cur.qd[s], ao);
     __syncthreads();
+
+    // S = S e^cum_last + k_dec^T v_new on this wave's dk rows (the tile is
+    // only read again after the next chunk's first barrier)
+    const Frag va0 = lds_frag(sVh, sVl, SC_SV, r16, 0, g4), va1 = lds_frag(sVh, sVl, SC_SV, r16, 1, g4);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) st[t] = f32x4_t{st[t][0] * cur.ecl, st[t][1] * cur.ecl, st[t][2] * cur.ecl, st[t][3] * cur.ecl};
+#pragma unroll
+    for (int t = 0; t < 2; ++t) st[t] = mfma3(cur.kd[t][0], va0, st[t]);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      st[t] = mfma3(cur.kd[t][1], va1, st[t]);
+      put4(sSh, sSl, SC_SS, r16, 32 * wid + 16 * t + 4 * g4, st[t][0], st[t][1], st[t][2], st[t][3]);
+    }
 
     // out^T += v_new^T qk^T over the causal token steps (j <= i: steps 0 ..
     // wid / 2; the record's QK holds zeros above the diagonal)
-    const Frag va0 = lds_frag(sVh, sVl, SC_SV, r16, 0, g4), va1 = lds_frag(sVh, sVl, SC_SV, r16, 1, g4);
     ao = mfma3(va0, cur.qk[0], ao);
     if (wid >= 2) ao = mfma3(va1, cur.qk[1], ao);
     const int tok = A.t0 + ci * CK_C + 16 * wid + r16;
@@ -757,18 +782,6 @@ __global__ __launch_bounds__(CK_NT) void dn_chunk_scan_kernel(ChunkScanArgs<T> A
       T* o = A.out + (((long)b * A.seq + tok) * A.heads + h) * CK_D + col0 + 4 * g4;
 #pragma unroll
       for (int i = 0; i < 4; ++i) Act<T>::store(o, i, ao[i]);
-    }
-
-    // S^T = S^T e^cum_last + v_new^T k_dec on this wave's dk rows (the tile
-    // is only read again after the next chunk's first barrier)
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      f32x4_t acc = {st[t][0] * cur.ecl, st[t][1] * cur.ecl, st[t][2] * cur.ecl, st[t][3] * cur.ecl};
-      acc = mfma3(va0, cur.kd[t][0], acc);
-      acc = mfma3(va1, cur.kd[t][1], acc);
-      st[t] = acc;
-      put2(sSh, sSl, SC_SS, 4 * g4, 32 * wid + 16 * t + r16, acc[0], acc[1]);
-      put2(sSh, sSl, SC_SS, 4 * g4 + 2, 32 * wid + 16 * t + r16, acc[2], acc[3]);
     }
     if (ci < 12) QM_PHASE(2 + ci);
   };
@@ -785,8 +798,8 @@ __global__ __launch_bounds__(CK_NT) void dn_chunk_scan_kernel(ChunkScanArgs<T> A
 
 #pragma unroll
   for (int t = 0; t < 2; ++t)
-    *reinterpret_cast<float4*>(S + (long)(32 * wid + 16 * t + r16) * CK_D) =
-        make_float4(st[t][0], st[t][1], st[t][2], st[t][3]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S[(16 * t + i) * CK_D] = st[t][i];
   QM_PHASE(14);
   QM_PHASE_FLUSH_AT(4096u);
 }
