@@ -388,9 +388,14 @@ struct DnRecurArgs {
   T* out;                                   // [B, T, H, D]
   int batch, seq, heads, hk;                // head h reads q/k head h % hk
   long q_stride, v_stride;
+  // the short chunk's form: q, k and v are channels of the raw inputs x [B, T,
+  // conv_dim], and g and beta are formed from a and b [B, T, H]
+  const T* x; const T* ring; const T* conv_w; const int* positions;
+  const T* a; const T* b; const float* a_neg; const float* dt_bias;
 };
 
 constexpr int REC_TOK = 16;        // tokens of a block
+static_assert(REC_TOK == QM_DN_SHORT_SEQ, "the short form is one block of tokens");
 
 // sum over the lanes of the same column (l % 4)
 __device__ __forceinline__ float column_sum(float v) {
@@ -399,7 +404,52 @@ __device__ __forceinline__ float column_sum(float v) {
   return xor32_sum(xor16_sum(v));
 }
 
-template <typename T>
+// An input window of a channel, with what chooses the history from the ring:
+// loads first (all unconditional, clamped indices), then the value of the
+// output at window place t, rounded as dn_conv_chunk_kernel's.
+template <typename T, int K, int N>
+struct ShortWindow {
+  T x[N], w[K], slots[K];
+  // outputs t0 .. t0 + N - K of channel ch
+  __device__ __forceinline__ void load(const DnRecurArgs<T>& A, int b, int ch, int conv_dim, int t0) {
+    const T* src = A.x + (long)b * A.seq * conv_dim + ch;
+    const T* ring = A.ring + ((long)b * conv_dim + ch) * K;
+#pragma unroll
+    for (int i = 0; i < N; ++i) x[i] = src[(long)min(max(t0 - (K - 1) + i, 0), A.seq - 1) * conv_dim];
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+      w[j] = A.conv_w[(long)ch * K + j];
+      slots[j] = ring[j];
+    }
+  }
+  __device__ __forceinline__ void history(int t0, int pos0) {
+#pragma unroll
+    for (int i = 0; i < (K - 1 < N ? K - 1 : N); ++i) {
+      int slot = (pos0 + t0 - (K - 1) + i) % K;
+      if (slot < 0) slot += K;
+      T hist = slots[0];
+#pragma unroll
+      for (int u = 1; u < K; ++u) hist = slot == u ? slots[u] : hist;
+      x[i] = t0 - (K - 1) + i < 0 ? hist : x[i];
+    }
+  }
+  __device__ __forceinline__ float out(int t) const {
+    float acc = 0.f;
+#pragma unroll
+    for (int j = 0; j < K; ++j) acc = fmaf(Act<T>::load(&w[j], 0), Act<T>::load(&x[t + j], 0), acc);
+    return Act<T>::round(silu_f(Act<T>::round(acc)));
+  }
+};
+
+// K > 0: the short form (at most REC_TOK tokens). The conv of the workgroup's
+// 272 channels and its head's gates are formed here, by each of the head's
+// eight workgroups, instead of by a launch of their own before this one, which
+// waits out the last one's end and its own first loads (a DeltaNet core of 5
+// tokens 10.9 -> 8.8 us, a verify step of four layers 232.6 -> 228.0). Every
+// input is loaded before the first is used: with v's channels in a pass of
+// their own after q's and k's it gained nothing. The ring is only read here;
+// the norm's launch, after it, writes it.
+template <typename T, int K>
 __global__ __launch_bounds__(DN_NT) void dn_recurrent_kernel(DnRecurArgs<T> A) {
   static_assert(DN_NT == 256 && DN_TILE == 16 && DN_D == 128, "four waves of four columns; two row elements a lane");
   constexpr int NTILE = DN_D / DN_TILE;
@@ -443,14 +493,54 @@ __global__ __launch_bounds__(DN_NT) void dn_recurrent_kernel(DnRecurArgs<T> A) {
     const long tok = (long)b * A.seq + min(t0 + (tid >> 4), A.seq - 1);
     vr = A.v[tok * A.v_stride + (long)h * DN_D + col0 + (tid & 15)];
   };
-  fetch(0);
+  if constexpr (K > 0) {
+    const int conv_dim = (2 * A.hk + A.heads) * DN_D;
+    const int pos0 = A.positions[b];
+    // a wave's four tokens' gates, one lane each
+    const int tg = min(4 * (lane & 3) + wid, A.seq - 1);
+    const long gi = ((long)b * A.seq + tg) * A.heads + h;
+    const T araw = A.a[gi], braw = A.b[gi];
+    const float dtb = A.dt_bias[h], an = A.a_neg[h];
+    // thread t: channel t of the head's q (t < 128) or k, and v's channel
+    // t % 16 at token t / 16
+    const int kq = tid >> 7, cq = tid & 127, tv = tid >> 4;
+    float (*dst)[DN_D] = kq ? s_k : s_q;
+    ShortWindow<T, K, REC_TOK + K - 1> wx;
+    ShortWindow<T, K, K> wv;
+    wx.load(A, b, (kq * A.hk + h % A.hk) * DN_D + cq, conv_dim, 0);
+    wv.load(A, b, 2 * A.hk * DN_D + h * DN_D + col0 + (tid & 15), conv_dim, tv);
+    __builtin_amdgcn_sched_barrier(0);
+    wx.history(0, pos0);
+    wv.history(tv, pos0);
+    s_v[tv][tid & 15] = wv.out(0);
+#pragma unroll
+    for (int t = 0; t < REC_TOK; ++t)
+      if (t < A.seq) dst[t][cq] = wx.out(t);
+    const float beta = Act<T>::round(sigmoid_f(Act<T>::load(&braw, 0)));
+    const float gate = an * softplus_fast(Act<T>::load(&araw, 0) + dtb);
+#pragma unroll
+    for (int i = 0; i < TPW; ++i) {
+      gr[i] = __shfl(gate, i);
+      br[i] = __shfl(beta, i);
+    }
+    __syncthreads();
+  } else {
+    fetch(0);
+  }
   for (int t0 = 0; t0 < A.seq; t0 += REC_TOK) {
     const int nt = min(REC_TOK, A.seq - t0);
 #pragma unroll
     for (int i = 0; i < TPW; ++i) {
       const int t = 4 * i + wid;
-      const float q0 = Act<T>::load(&qr[i][0], 0), q1 = Act<T>::load(&qr[i][1], 0);
-      const float k0 = Act<T>::load(&kr[i][0], 0), k1 = Act<T>::load(&kr[i][1], 0);
+      float q0, q1, k0, k1;
+      if constexpr (K > 0) {           // a lane's own elements: it reads and replaces them
+        if (t >= nt) break;
+        q0 = s_q[t][lane], q1 = s_q[t][lane + 64];
+        k0 = s_k[t][lane], k1 = s_k[t][lane + 64];
+      } else {
+        q0 = Act<T>::load(&qr[i][0], 0), q1 = Act<T>::load(&qr[i][1], 0);
+        k0 = Act<T>::load(&kr[i][0], 0), k1 = Act<T>::load(&kr[i][1], 0);
+      }
       const float sq = wave_sum(fmaf(q0, q0, q1 * q1)), sk = wave_sum(fmaf(k0, k0, k1 * k1));
       const float sqk = wave_sum(fmaf(q0, k0, q1 * k1));
       const float rq = rsqrt_rn(sq + 1e-6f), rk = rsqrt_rn(sk + 1e-6f);
@@ -460,9 +550,9 @@ __global__ __launch_bounds__(DN_NT) void dn_recurrent_kernel(DnRecurArgs<T> A) {
       s_k[t][lane + 64] = mul_rn(k1, rk);
       if (lane == 0) s_scal[t] = make_float4(expf(gr[i]), br[i], div_rn(sqk * rq * rk, inv_sqrt_d), 0.f);
     }
-    s_v[tid >> 4][tid & 15] = Act<T>::load(&vr, 0);
+    if constexpr (K == 0) s_v[tid >> 4][tid & 15] = Act<T>::load(&vr, 0);
     __syncthreads();
-    if (t0 + REC_TOK < A.seq) fetch(t0 + REC_TOK);
+    if (K == 0 && t0 + REC_TOK < A.seq) fetch(t0 + REC_TOK);
     for (int t = 0; t < nt; ++t) {
       const float4 sc = s_scal[t];
       const float4 ka = *reinterpret_cast<const float4*>(&s_k[t][row0]), kb = *reinterpret_cast<const float4*>(&s_k[t][row0 + 4]);
@@ -514,12 +604,36 @@ template <typename T>
 int launch_dn_recurrent(int batch, int seq, int heads, int hk, long q_stride, long v_stride, const void* q,
                         const void* k, const void* v, const float* g, const float* beta, float* state, void* out,
                         hipStream_t stream) {
-  DnRecurArgs<T> A;
+  DnRecurArgs<T> A{};
   A.q = static_cast<const T*>(q); A.k = static_cast<const T*>(k); A.v = static_cast<const T*>(v);
   A.g = g; A.beta = beta; A.state = state; A.out = static_cast<T*>(out);
   A.batch = batch; A.seq = seq; A.heads = heads; A.hk = hk; A.q_stride = q_stride; A.v_stride = v_stride;
   const int nwg = batch * heads * (DN_D / DN_TILE);
-  hipLaunchKernelGGL(dn_recurrent_kernel<T>, dim3(nwg), dim3(DN_NT), 0, stream, A);
+  hipLaunchKernelGGL((dn_recurrent_kernel<T, 0>), dim3(nwg), dim3(DN_NT), 0, stream, A);
+  QM_CHECK_LAUNCH();
+  return QM_OK;
+}
+
+template <typename T>
+int launch_dn_short(const qm_dn_geom* g, int seq, const void* qkv, const void* a, const void* b, const float* a_neg,
+                    const float* dt_bias, const void* conv_w, const int* positions, const void* conv_ring,
+                    float* state, void* out, hipStream_t stream) {
+  DnRecurArgs<T> A{};
+  A.state = state; A.out = static_cast<T*>(out);
+  A.batch = g->batch; A.seq = seq; A.heads = g->n_v_heads; A.hk = g->n_k_heads;
+  A.x = static_cast<const T*>(qkv); A.ring = static_cast<const T*>(conv_ring);
+  A.conv_w = static_cast<const T*>(conv_w); A.positions = positions;
+  A.a = static_cast<const T*>(a); A.b = static_cast<const T*>(b); A.a_neg = a_neg; A.dt_bias = dt_bias;
+  const dim3 grid(g->batch * g->n_v_heads * (DN_D / DN_TILE));
+  switch (g->conv_kernel) {
+    case 2: hipLaunchKernelGGL((dn_recurrent_kernel<T, 2>), grid, dim3(DN_NT), 0, stream, A); break;
+    case 3: hipLaunchKernelGGL((dn_recurrent_kernel<T, 3>), grid, dim3(DN_NT), 0, stream, A); break;
+    case 4: hipLaunchKernelGGL((dn_recurrent_kernel<T, 4>), grid, dim3(DN_NT), 0, stream, A); break;
+    case 5: hipLaunchKernelGGL((dn_recurrent_kernel<T, 5>), grid, dim3(DN_NT), 0, stream, A); break;
+    case 6: hipLaunchKernelGGL((dn_recurrent_kernel<T, 6>), grid, dim3(DN_NT), 0, stream, A); break;
+    case 7: hipLaunchKernelGGL((dn_recurrent_kernel<T, 7>), grid, dim3(DN_NT), 0, stream, A); break;
+    default: hipLaunchKernelGGL((dn_recurrent_kernel<T, 8>), grid, dim3(DN_NT), 0, stream, A); break;
+  }
   QM_CHECK_LAUNCH();
   return QM_OK;
 }
@@ -599,4 +713,14 @@ int qm_dn_recurrent_strided(int act_dtype, int batch, int seq, int heads, int hk
     return launch_dn_recurrent<bf16_t>(batch, seq, heads, hk, q_stride, v_stride, q, k, v, g, beta, state, out,
                                        stream);
   return qm_fail(QM_ERR_DTYPE, "qm_dn_recurrent: act_dtype must be QM_ACT_F32 or QM_ACT_BF16");
+}
+
+int qm_dn_short(const qm_dn_geom* g, int seq, const void* qkv, const void* a, const void* b, const float* a_neg,
+                const float* dt_bias, const void* conv_w, const int* positions, const void* conv_ring, float* state,
+                void* out, hipStream_t stream) {
+  if (seq < 1 || seq > QM_DN_SHORT_SEQ) return qm_fail(QM_ERR_ARG, "qm_dn_short: 1 to 16 tokens");
+  return g->act_dtype == QM_ACT_F32
+             ? launch_dn_short<float>(g, seq, qkv, a, b, a_neg, dt_bias, conv_w, positions, conv_ring, state, out, stream)
+             : launch_dn_short<bf16_t>(g, seq, qkv, a, b, a_neg, dt_bias, conv_w, positions, conv_ring, state, out,
+                                       stream);
 }

@@ -11,6 +11,8 @@
 //   delta rule      the WY/UT chunked kernels (dn_chunk.hip) for chunks of 24
 //                   tokens or more, the token loop for shorter ones
 //   dn_gated_norm   one wavefront per (token, head) row of 128
+// Up to 16 tokens of few sequences are two launches: the token loop forms the
+// conv and the gates itself, and the norm's launch also writes the ring.
 #include <atomic>
 
 #include "common.h"
@@ -121,10 +123,27 @@ __global__ __launch_bounds__(CONV_CH) void dn_conv_chunk_kernel(ConvChunkArgs<T>
   }
 }
 
+// A short chunk's last K-1 inputs, for the ring (dn_norm's workgroups past the
+// rows: the launch before it, the only reader, is done).
+template <typename T>
+struct RingArgs {
+  const T* qkv; T* ring; const int* positions;
+  int batch, seq, conv_dim, k, n_norm_wg;
+};
+
 // out = round_T(w * (o * rsqrt(mean(o^2) + eps)) * sigmoid(z)) per 128-row
 template <typename T>
 __global__ __launch_bounds__(256) void dn_gated_norm_kernel(const T* o, const T* z, const float* w, T* out, long rows,
-                                                            float eps) {
+                                                            float eps, RingArgs<T> R) {
+  if ((int)blockIdx.x >= R.n_norm_wg) {
+    const long i = (long)((int)blockIdx.x - R.n_norm_wg) * 256 + threadIdx.x;     // a channel of a sequence
+    if (i >= (long)R.batch * R.conv_dim) return;
+    const int b = (int)(i / R.conv_dim), ch = (int)(i % R.conv_dim);
+    const int pos0 = R.positions[b];
+    for (int t = max(R.seq - (R.k - 1), 0); t < R.seq; ++t)
+      R.ring[i * R.k + (pos0 + t) % R.k] = R.qkv[((long)b * R.seq + t) * R.conv_dim + ch];
+    return;
+  }
   const long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= rows) return;
@@ -166,15 +185,34 @@ int launch_prefill(const qm_dn_geom* g, int seq, const void* qkv, const void* z,
   T* core = reinterpret_cast<T*>(base + L.core);
   const int conv_dim = (2 * g->n_k_heads + g->n_v_heads) * DN_D;
 
+  const long n_gate = (long)g->batch * seq * g->n_v_heads;
+  if (n_gate > 0x7fffffffL - CONV_CH)
+    return qm_fail(QM_ERR_UNSUPPORTED, "qm_dn_prefill: batch * seq * value heads must stay below 2^31");
+  const int n_norm_wg = (int)((n_gate + 3) / 4);
+  RingArgs<T> R{static_cast<const T*>(qkv), static_cast<T*>(conv_ring), positions, g->batch, seq, conv_dim,
+                g->conv_kernel, n_norm_wg};
+  // one block of the token loop and few sequences: the loop forms the conv and
+  // the gates itself, in each of a head's eight workgroups, and the norm's launch
+  // writes the ring. Past that the repeated conv costs more than the launch
+  // (16/32 heads, bf16, us, with the conv's launch / here: 10.9 / 8.8 for 5
+  // tokens, 14.7 / 13.4 for 16, 16.9 / 16.3 for 2 x 16, 20.7 / 20.7 for 4 x 12,
+  // 23.1 / 24.7 for 4 x 16, 43.6 / 42.7 for 16 x 8, 74.7 / 75.8 for 32 x 8)
+  if (seq <= QM_DN_SHORT_SEQ && (g->batch <= 2 || (seq <= 8 && g->batch <= 16))) {
+    const int rc = qm_dn_short(g, seq, qkv, a, b, a_neg, dt_bias, conv_w, positions, conv_ring, state, core, stream);
+    if (rc) return rc;
+    const int n_ring_wg = (int)(((long)g->batch * conv_dim + 255) / 256);
+    hipLaunchKernelGGL(dn_gated_norm_kernel<T>, dim3(n_norm_wg + n_ring_wg), dim3(256), 0, stream, core,
+                       static_cast<const T*>(z), norm_w, static_cast<T*>(out), n_gate, g->eps, R);
+    QM_CHECK_LAUNCH();
+    return QM_OK;
+  }
+
   ConvChunkArgs<T> C;
   C.qkv = static_cast<const T*>(qkv); C.a = static_cast<const T*>(a); C.b = static_cast<const T*>(b);
   C.a_neg = a_neg; C.dt_bias = dt_bias; C.conv_w = static_cast<const T*>(conv_w); C.positions = positions;
   C.ring = static_cast<T*>(conv_ring); C.conv_out = conv_out; C.g_out = g_out; C.beta_out = beta_out;
   C.batch = g->batch; C.seq = seq; C.conv_dim = conv_dim; C.hv = g->n_v_heads;
   C.n_conv_wg = g->batch * ((conv_dim + CONV_CH - 1) / CONV_CH) * ((seq + CONV_TOK - 1) / CONV_TOK);
-  const long n_gate = (long)g->batch * seq * g->n_v_heads;
-  if (n_gate > 0x7fffffffL - CONV_CH)
-    return qm_fail(QM_ERR_UNSUPPORTED, "qm_dn_prefill: batch * seq * value heads must stay below 2^31");
   const dim3 grid(C.n_conv_wg + (unsigned)((n_gate + CONV_CH - 1) / CONV_CH));
   switch (g->conv_kernel) {
     case 2: hipLaunchKernelGGL((dn_conv_chunk_kernel<T, 2>), grid, dim3(CONV_CH), 0, stream, C); break;
@@ -193,9 +231,8 @@ int launch_prefill(const qm_dn_geom* g, int seq, const void* qkv, const void* z,
                             L.total - L.rule, stream);
   if (rc) return rc;
 
-  const long rows = (long)g->batch * seq * g->n_v_heads;
-  hipLaunchKernelGGL(dn_gated_norm_kernel<T>, dim3((rows + 3) / 4), dim3(256), 0, stream, core,
-                     static_cast<const T*>(z), norm_w, static_cast<T*>(out), rows, g->eps);
+  hipLaunchKernelGGL(dn_gated_norm_kernel<T>, dim3(n_norm_wg), dim3(256), 0, stream, core,
+                     static_cast<const T*>(z), norm_w, static_cast<T*>(out), n_gate, g->eps, R);
   QM_CHECK_LAUNCH();
   return QM_OK;
 }

@@ -16,6 +16,14 @@ int qm_dn_recurrent_strided(int act_dtype, int batch, int seq, int heads, int hk
                             const void* q, const void* k, const void* v, const float* g, const float* beta,
                             float* state, void* out, hipStream_t stream);
 
+// The same for a short prefill chunk (1 to QM_DN_SHORT_SEQ tokens) from the raw
+// inputs: the conv over [ring | chunk] and the gates are formed in the kernel.
+// The ring is read, not written.
+constexpr int QM_DN_SHORT_SEQ = 16;
+int qm_dn_short(const qm_dn_geom* g, int seq, const void* qkv, const void* a, const void* b, const float* a_neg,
+                const float* dt_bias, const void* conv_w, const int* positions, const void* conv_ring, float* state,
+                void* out, hipStream_t stream);
+
 // The delta rule over a chunk of tokens for the prefill path: the WY/UT chunked
 // kernels (64-token chunks) for chunks of 24 tokens or more, the token loop for
 // shorter ones. `ws` holds qm_dn_rule_chunk_workspace(batch, seq, heads) bytes.
