@@ -610,7 +610,8 @@ __global__ __launch_bounds__(HR_NT) void hc_many_up_kernel(HrArgs<float> A) {
 // while the row tiles of a group pass; grid (hidden / 32, row groups), 16
 // waves, wave w takes tiles w, w + 16, ... of its group for all 32 positions
 // (the low-rank rows, loads of 16 rows x 64 bytes, are read once per 32
-// positions; once per 16 the kernel took 35 us at 2000 rows, now 18). Four waves a SIMD, so that one wave's loads
+// positions; once per 16 the kernel took 35 us at 2000 rows, now 18 alone and
+// 25 after the down product). Four waves a SIMD, so that one wave's loads
 // (hyper comes from HBM) run under the others' products and gates. Row r of up
 // tile j is position 8 (r / 4) + 4 j + r % 4, so that a lane ends up with 8
 // consecutive positions of a row: 16-byte loads of hyper and stores of mixed.
