@@ -56,6 +56,19 @@ def test_short_chunk_equals_its_tokens_in_a_longer_one(gpu, dtype, kernel, hk, h
     err = (got - want).abs().amax((0, 2)) / want.abs().amax((0, 2))
     assert float(err.max()) <= bar, err
     assert float((states[1] - states[0]).abs().max() / states[0].abs().max()) <= 1e-6
+    # outputs over the inputs' memory (not the short form): the same
+    def over():
+        x = [t[:, :seq].contiguous() for t in (qkv, z, a, b)]
+        ring, state = ring0.clone(), state0.clone()
+        ws = torch.empty(lib.qm_dn_prefill_workspace(ctypes.byref(geom), seq), dtype=torch.uint8, device=DEV)
+        native.call("qm_dn_prefill", ctypes.byref(geom), seq, *(native.ptr(t) for t in x), native.ptr(a_neg),
+                    native.ptr(dt_bias), native.ptr(conv_w), native.ptr(norm_w), native.ptr(pos0), native.ptr(ring),
+                    native.ptr(state), native.ptr(x[0]), native.ptr(ws), ws.numel(), native.stream_handle())
+        torch.cuda.synchronize()
+        return x[0].flatten()[:batch * seq * hv * 128].view(batch, seq, -1).float()
+
+    err = (over() - want[:, :seq]).abs().amax((0, 2)) / want[:, :seq].abs().amax((0, 2))
+    assert float(err.max()) <= bar, err
     # the last K - 1 inputs' slots (the remaining slot holds what the part before left there)
     for i in range(batch):
         for t in range(total - kernel + 1, total):

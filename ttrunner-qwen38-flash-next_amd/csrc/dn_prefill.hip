@@ -197,7 +197,13 @@ int launch_prefill(const qm_dn_geom* g, int seq, const void* qkv, const void* z,
   // (16/32 heads, bf16, us, with the conv's launch / here: 10.9 / 8.8 for 5
   // tokens, 14.7 / 13.4 for 16, 16.9 / 16.3 for 2 x 16, 20.7 / 20.7 for 4 x 12,
   // 23.1 / 24.7 for 4 x 16, 43.6 / 42.7 for 16 x 8, 74.7 / 75.8 for 32 x 8)
-  if (seq <= QM_DN_SHORT_SEQ && (g->batch <= 2 || (seq <= 8 && g->batch <= 16))) {
+  // (and the ring's inputs are read beside the outputs' stores, so not where the
+  // outputs take the inputs' memory)
+  const char* x0 = static_cast<const char*>(qkv);
+  const char* o0 = static_cast<const char*>(out);
+  const bool apart = o0 >= x0 + (size_t)g->batch * seq * conv_dim * sizeof(T) ||
+                     x0 >= o0 + (size_t)n_gate * DN_D * sizeof(T);
+  if (apart && seq <= QM_DN_SHORT_SEQ && (g->batch <= 2 || (seq <= 8 && g->batch <= 16))) {
     const int rc = qm_dn_short(g, seq, qkv, a, b, a_neg, dt_bias, conv_w, positions, conv_ring, state, core, stream);
     if (rc) return rc;
     const int n_ring_wg = (int)(((long)g->batch * conv_dim + 255) / 256);
