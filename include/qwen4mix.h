@@ -415,8 +415,8 @@ typedef struct qm_hc_geom {
   float eps;        /* rms_norm_eps of the stream norm                      */
 } qm_hc_geom;
 
-/* Bytes of workspace qm_hc_mix needs (normalised rows and the down product);
- * 0 if the geometry is unsupported. */
+/* Bytes of workspace qm_hc_mix needs (normalised rows and the low-rank values,
+ * or partial products); 0 if the geometry is unsupported. */
 size_t qm_hc_mix_workspace(const qm_hc_geom* g);
 
 /* The hyper-connection read gate, Qwen4ExpModel._gated_residual
@@ -430,7 +430,9 @@ size_t qm_hc_mix_workspace(const qm_hc_geom* g);
  *   with_inject (the layer mixers), unused otherwise (the final mixer).
  *   streams * hidden must be 1, 2, 4, 5, 8 or 10 times 2048 (bf16) or 1024
  *   (f32); hidden a multiple of 8; rank a multiple of 8 (4 for f32), <= 512.
- * Two launches; every pointer except inject and mixed 16-byte aligned. */
+ * Two or three launches; every pointer except inject and mixed 16-byte
+ * aligned. mixed may lie over hyper's memory (the final mixer's residual is
+ * done with; such a call of many rows takes the slower few-row kernels). */
 int qm_hc_mix(const qm_hc_geom* g, const void* hyper, const float* norm_w, const void* down_inject_w,
               int with_inject, const void* up_w, void* mixed, void* inject, void* workspace,
               size_t workspace_bytes, hipStream_t stream);

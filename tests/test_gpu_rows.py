@@ -126,3 +126,21 @@ def test_project_routes_by_rows(gpu):
             for t, name in zip(got, model.PROJ_GROUPS["dn_in"]):
                 want = torch.nn.functional.linear(hidden.float(), store.get(f"blk.0.{name}").to(DEV).float())
                 assert rel_err(t.detach(), want, 1e-2) < 1e-2, (seq, name)
+
+
+@pytest.mark.parametrize("dtype,rows,at", [(BF, 9, 0), (BF, 40, 3), (BF, 300, 0), (F32, 17, 1), (F32, 600, 0)])
+def test_hyper_mix_into_the_residuals_memory(gpu, dtype, rows, at):
+    """mixed over the memory of hyper (from its row ``at`` on): the bits of the
+    same rows in calls of 8, whose kernels read hyper before anything is stored
+    (the matrix-core kernels read it again beside the stores, and their sums have
+    another order)."""
+    qm = gpu
+    print(f"hc over its input {dtype} rows={rows} at={at}", flush=True)
+    store = gi.FakeStore(gi.hc_weights("output_hc", 5, dtype, hidden=2048, with_inject=False))
+    model = qm.Qwen4MixModel(qm.MixConfig(), store, device=DEV)
+    hyper = gi.normal(gi.rng(rows), (1, rows, 4 * 2048), 1.0).to(dtype).to(DEV)
+    want = torch.cat([model._gated_residual(h, None, "attn")[0] for h in hyper.split(8, 1)], 1)
+    over = hyper.flatten()[at * 4 * 2048:][:rows * 2048].view(1, rows, 2048)
+    mixed, _, _ = model._gated_residual(hyper, None, "attn", mixed=over)
+    torch.cuda.synchronize()
+    assert mixed.data_ptr() == over.data_ptr() and torch.equal(mixed, want)

@@ -199,10 +199,7 @@ int launch_prefill(const qm_dn_geom* g, int seq, const void* qkv, const void* z,
   // 23.1 / 24.7 for 4 x 16, 43.6 / 42.7 for 16 x 8, 74.7 / 75.8 for 32 x 8)
   // (and the ring's inputs are read beside the outputs' stores, so not where the
   // outputs take the inputs' memory)
-  const char* x0 = static_cast<const char*>(qkv);
-  const char* o0 = static_cast<const char*>(out);
-  const bool apart = o0 >= x0 + (size_t)g->batch * seq * conv_dim * sizeof(T) ||
-                     x0 >= o0 + (size_t)n_gate * DN_D * sizeof(T);
+  const bool apart = !qm_overlap(out, (size_t)n_gate * DN_D * sizeof(T), qkv, (size_t)g->batch * seq * conv_dim * sizeof(T));
   if (apart && seq <= QM_DN_SHORT_SEQ && (g->batch <= 2 || (seq <= 8 && g->batch <= 16))) {
     const int rc = qm_dn_short(g, seq, qkv, a, b, a_neg, dt_bias, conv_w, positions, conv_ring, state, core, stream);
     if (rc) return rc;

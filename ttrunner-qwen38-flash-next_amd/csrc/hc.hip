@@ -462,7 +462,10 @@ extern "C" int qm_hc_mix(const qm_hc_geom* g, const void* hyper, const float* no
     return qm_fail(QM_ERR_ARG, "qm_hc_mix: hyper, weights and workspace must be 16-byte aligned");
   if (with_inject && !inject) return qm_fail(QM_ERR_ARG, "qm_hc_mix: with_inject needs an inject output");
   if (workspace_bytes < hc_layout(*g).total) return qm_fail(QM_ERR_WORKSPACE, "qm_hc_mix: workspace too small");
-  if (hc_takes_rows(*g) && aligned16(mixed))
+  // those kernels read hyper again beside the stores of mixed; here the first
+  // launch alone reads it
+  const size_t mixed_bytes = (size_t)g->rows * g->hidden * (g->act_dtype == QM_ACT_BF16 ? 2 : 4);
+  if (hc_takes_rows(*g) && aligned16(mixed) && !qm_overlap(mixed, mixed_bytes, hyper, g->streams * mixed_bytes))
     return qm_hc_mix_rows(*g, hyper, norm_w, down_inject_w, with_inject, up_w, mixed, inject, workspace, stream);
   if (g->act_dtype == QM_ACT_BF16)
     return run_mix<bf16_t>(*g, hyper, norm_w, down_inject_w, with_inject, up_w, mixed, inject, workspace, stream);

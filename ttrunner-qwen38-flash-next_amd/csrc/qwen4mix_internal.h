@@ -10,6 +10,15 @@ int qm_fail(int code, const char* msg);
 
 inline size_t qm_align256(size_t n) { return (n + 255) & ~static_cast<size_t>(255); }
 
+// Whether na bytes at a and nb bytes at b share memory: a caller may give an
+// output the memory of inputs that an entry point is done with, and a path that
+// reads them beside its output stores is then not taken.
+inline bool qm_overlap(const void* a, size_t na, const void* b, size_t nb) {
+  const char* x = static_cast<const char*>(a);
+  const char* y = static_cast<const char*>(b);
+  return x < y + nb && y < x + na;
+}
+
 // The delta-rule token loop over strided q/k/v rows (q/k head h % hk): shared
 // by qm_dn_recurrent and the prefill path.
 int qm_dn_recurrent_strided(int act_dtype, int batch, int seq, int heads, int hk, long q_stride, long v_stride,
