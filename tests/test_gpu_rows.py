@@ -144,3 +144,36 @@ def test_hyper_mix_into_the_residuals_memory(gpu, dtype, rows, at):
     mixed, _, _ = model._gated_residual(hyper, None, "attn", mixed=over)
     torch.cuda.synchronize()
     assert mixed.data_ptr() == over.data_ptr() and torch.equal(mixed, want)
+
+
+@pytest.mark.parametrize("rows", [9, 17, 193])
+def test_bf16_gates_equal_the_precise_chains(gpu, rows):
+    """Every bf16 value but the NaNs as the gate's input, 2048 a call: low-rank
+    value 1 (silu(1.28125) rounds to it) times an up weight of that value, so the
+    output is the rounded sigmoid itself. The matrix-core kernels' short form
+    gives the bits of the vector kernels' precise one (8 rows)."""
+    qm = gpu
+    k = 4 * 2048
+    values = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(BF)
+    values = torch.where(values.isnan(), torch.zeros_like(values), values).to(DEV)
+    norm_w = torch.ones(k, device=DEV)
+    down = torch.zeros(320, k, dtype=BF, device=DEV)
+    down[0, 0] = 4 * 1.28125
+    hyper = torch.ones(rows, k, dtype=BF, device=DEV)
+    up = torch.zeros(k, 320, dtype=BF, device=DEV)
+    print(f"gates of {rows} rows", flush=True)
+
+    def mix(n):
+        g = qm.native.HcGeom(n, 4, 2048, 320, qm.native.act_code(BF), 1e-6)
+        ws = torch.empty(qm.native.load().qm_hc_mix_workspace(ctypes.byref(g)), dtype=torch.uint8, device=DEV)
+        out = torch.empty(n, 2048, dtype=BF, device=DEV)
+        qm.native.call("qm_hc_mix", ctypes.byref(g), hyper.data_ptr(), norm_w.data_ptr(), down.data_ptr(), 0,
+                       up.data_ptr(), out.data_ptr(), None, ws.data_ptr(), ws.numel(), qm.native.stream_handle())
+        torch.cuda.synchronize()
+        return out.view(torch.int16)
+
+    for v in values.split(2048):
+        up[:, 0] = v.repeat(4)
+        want = mix(8)
+        assert torch.equal(want[0].view(BF).float(), torch.sigmoid(v.float()).to(BF).float()) or v.float().amin() < -87
+        assert torch.equal(mix(rows), want[:1].expand(rows, -1))
