@@ -124,7 +124,9 @@ size_t qm_dn_chunked_workspace(int batch, int seq, int heads, int head_dim);
 /* The same rule in the chunked WY/UT form, 64-token chunks:
  * chunk_gated_delta_rule (reference/layers.py:195-275). Same arguments and
  * result (to float32 rounding) as qm_dn_recurrent, plus a workspace of
- * qm_dn_chunked_workspace() bytes (no initial contents needed). */
+ * qm_dn_chunked_workspace() bytes (no initial contents needed). out may lie
+ * over q, k, v, g or beta (every input is read before an output is stored;
+ * such a call over a long sequence is the slower for it). */
 int qm_dn_chunked(int act_dtype, int batch, int seq, int heads, int head_dim, const void* q, const void* k,
                   const void* v, const float* g, const float* beta, float* state, void* out, void* workspace,
                   size_t workspace_bytes, hipStream_t stream);

@@ -72,3 +72,39 @@ def test_prefill_rule_at_the_dispatch(gpu, seq):
     assert float((got.float() - want.float()).abs().max() / want.float().abs().max()) < 2e-2
     assert float((many[0].recurrent_state - one[0].recurrent_state).abs().max()) < 1e-3
     assert torch.equal(many[0].conv_state, one[0].conv_state)
+
+
+@pytest.mark.parametrize("over", ["v", "q", "g"])
+def test_chunked_rule_into_its_inputs_memory(gpu, over):
+    """2304 tokens of 32 heads are more records than one segment takes (160 MB).
+    Outputs whose first half lies over the second half of an input: the bits of
+    the same call with outputs of their own."""
+    native = gpu.native
+    bf = torch.bfloat16
+    heads, seq = 32, 2304
+    print(f"chunked rule over {over}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(9)
+    r = lambda *s: torch.randn(*s, generator=gen, device=DEV)  # noqa: E731
+    n = seq * heads * 128
+    x = {i: r(1, seq, heads, 128).to(bf) for i in "qkv"}
+    x["g"], x["beta"] = -r(1, seq, heads).abs(), torch.sigmoid(r(1, seq, heads))
+    state0 = r(1, heads, 128, 128) * 0.1
+    lib = native.load()
+    ws = torch.empty(lib.qm_dn_chunked_workspace(1, seq, heads, 128), dtype=torch.uint8, device=DEV)
+
+    def run(x, out):
+        state = state0.clone()
+        native.call("qm_dn_chunked", native.act_code(bf), 1, seq, heads, 128, *(x[i].data_ptr() for i in
+                    ("q", "k", "v", "g", "beta")), state.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel(),
+                    native.stream_handle())
+        torch.cuda.synchronize()
+        return out.clone(), state
+
+    want, want_state = run(x, torch.empty(n, dtype=bf, device=DEV))
+    # the input at the start of a buffer, the outputs from the middle of the input on
+    size = x[over].numel() * x[over].element_size()
+    buf = torch.empty(size // 2 + 2 * n, dtype=torch.uint8, device=DEV)
+    held = buf[:size].view(x[over].dtype).view(x[over].shape)
+    held.copy_(x[over])
+    got, state = run(dict(x, **{over: held}), buf[size // 2:].view(bf))
+    assert torch.equal(got, want) and torch.equal(state, want_state)

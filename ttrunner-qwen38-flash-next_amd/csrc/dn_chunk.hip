@@ -819,7 +819,16 @@ int launch_chunked(int batch, int seq, int heads, int hk, long q_stride, long v_
                    hipStream_t stream) {
   const int n_total = (seq + CK_C - 1) / CK_C;
   const size_t chunk_bytes = (size_t)batch * heads * CK_REC * sizeof(float);
-  const size_t n_seg = (n_total * chunk_bytes + CK_SEG_BYTES - 1) / CK_SEG_BYTES;
+  // a segment's outputs are stored before the next one's inputs are read: outputs
+  // that lie over inputs take one segment, whose prep reads them all first
+  const size_t rows = (size_t)batch * seq, gates = rows * heads * sizeof(float);
+  const size_t out_bytes = rows * heads * CK_D * sizeof(T);
+  const size_t qk_bytes = ((rows - 1) * q_stride + hk * CK_D) * sizeof(T);
+  const size_t v_bytes = ((rows - 1) * v_stride + heads * CK_D) * sizeof(T);
+  const bool over = qm_overlap(out, out_bytes, q, qk_bytes) || qm_overlap(out, out_bytes, k, qk_bytes) ||
+                    qm_overlap(out, out_bytes, v, v_bytes) || qm_overlap(out, out_bytes, g, gates) ||
+                    qm_overlap(out, out_bytes, beta, gates);
+  const size_t n_seg = over ? 1 : (n_total * chunk_bytes + CK_SEG_BYTES - 1) / CK_SEG_BYTES;
   const int seg = n_seg < (size_t)n_total ? (int)((n_total + n_seg - 1) / n_seg) : 1;
   for (int c0 = 0; c0 < n_total; c0 += seg) {
     const int n_chunks = seg < n_total - c0 ? seg : n_total - c0;
