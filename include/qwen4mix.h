@@ -350,7 +350,8 @@ size_t qm_qsa_attend_chunk_workspace(const qm_qsa_geom* g, int seq);
  *   [B, S] from qm_qsa_select; out [B, S, Hq*d] act.
  * The workspace holds a slot table per (row, block), which every call writes
  * afresh: nothing in it is kept between calls, so one workspace serves chunks
- * of any length that fit it. Do not let two calls on it overlap. */
+ * of any length that fit it. Do not let two calls on it overlap. out may lie
+ * over q (it is stored when the attention has read it), not over qg. */
 int qm_qsa_attend_chunk(const qm_qsa_geom* g, int seq, const void* q, const void* qg, const void* k_pool,
                         const void* v_pool, const int* positions, const int* page_table, const int* ids,
                         const int* n_sel, void* out, void* workspace, size_t workspace_bytes, hipStream_t stream);

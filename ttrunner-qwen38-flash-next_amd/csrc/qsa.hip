@@ -3666,7 +3666,11 @@ int attend_chunk(const qm_qsa_geom* g, int seq, const void* q, const void* qg, c
   A.nwg_sel = g->max_blocks;
   A.seg_spans = CA_SEG_SPANS;
   const size_t row_bytes = (size_t)g->batch * g->n_kv_heads * nslot * GQA * QSA_D * sizeof(uint16_t);
-  const size_t n_part = (seq * row_bytes + CA_PART_BYTES - 1) / CA_PART_BYTES;
+  // a part's outputs are stored before the next one's queries are read: outputs
+  // that lie over q take one part
+  const size_t q_elems = (size_t)g->batch * seq * g->n_heads * QSA_D;
+  const bool over = qm_overlap(out, q_elems * (g->act_dtype == QM_ACT_F32 ? 4 : 2), q, q_elems * 2 * sizeof(uint16_t));
+  const size_t n_part = over ? 1 : (seq * row_bytes + CA_PART_BYTES - 1) / CA_PART_BYTES;
   const int part = (int)(((seq + n_part - 1) / n_part + 127) / 128 * 128);
   for (int row0 = 0; row0 < seq; row0 += part) {
     A.row0 = row0;
