@@ -63,3 +63,29 @@ def test_bind_refuses_what_one_sequence_refuses(gpu):
     x = [torch.zeros(1, 1, n, dtype=torch.bfloat16, device=DEV) for n in (16 * 512, 512, 512, 512, 128)]
     with pytest.raises(qm.native.QmError):
         p.bind(*x)
+
+
+@pytest.mark.parametrize("batch,pos", [(2, 300), (9, 700), (9, 2500)])
+def test_eager_decode_buffers_are_a_layers_own(gpu, monkeypatch, batch, pos):
+    """Eager decode of two layers, by either route: no scratch buffer of one
+    layer's step is the other's, so that the layers may run on two streams."""
+    qm = gpu
+    print(f"buffers of eager decode, batch {batch} at {pos}", flush=True)
+    model = qm.Qwen4MixModel(qm.MixConfig(), gi.FakeStore({**gi.qsa_weights(3, 90, torch.bfloat16),
+                                                           **gi.qsa_weights(7, 91, torch.bfloat16)}), device=DEV)
+    cache = qm.MixHybridCache(8, model.config, batch, 4096, DEV)
+    x = [torch.zeros(batch, 1, n, dtype=torch.bfloat16, device=DEV) for n in (16 * 512, 512, 512, 512, 128)]
+    taken = {}
+    inner = model._workspace
+
+    def record(name, nbytes):
+        buf = inner(name, nbytes)
+        taken.setdefault(layer, set()).add(buf.data_ptr())
+        return buf
+
+    monkeypatch.setattr(model, "_workspace", record)
+    for layer in (3, 7):
+        cache[layer].ensure_qsa(batch, torch.bfloat16)
+        model.qsa_core(*x, layer, cache, pos)
+    torch.cuda.synchronize()
+    assert taken[3] and taken[7] and not taken[3] & taken[7]

@@ -395,8 +395,10 @@ class Qwen4MixModel:
                         native.ptr(chunk_ws), chunk_ws.numel(), stream)
         else:
             # one row (a decode step past the one-launch kernel's range): a
-            # score buffer makes qm_qsa_select spread the scores over the blocks
-            scores = (self._workspace(f"qsa_scores_{batch}_{cache.max_blocks}", batch * cache.max_blocks * 4)
+            # score buffer makes qm_qsa_select spread the scores over the
+            # blocks. A decode step's buffers are the layer's and the batch's own
+            # on either path, so that layers may decode on streams of their own
+            scores = (self._workspace(f"qsa_scores_{layer}_{batch}", batch * cache.max_blocks * 4)
                       if seq == 1 else None)
             native.call("qm_qsa_select", ctypes.byref(g), seq, native.ptr(iq_out), native.ptr(lc.block_keys),
                         native.ptr(pos), native.ptr(lc.page_table), native.ptr(ids), native.ptr(n_sel),
@@ -422,7 +424,8 @@ class Qwen4MixModel:
                             native.ptr(chunk_ws), chunk_ws.numel(), stream)
             return out
         splits = lib.qm_qsa_attend_splits(ctypes.byref(g), query_offset, query_offset + seq - 1)
-        ws = self._workspace("qsa_attend", lib.qm_qsa_attend_workspace(ctypes.byref(g), seq, splits))
+        ws = self._workspace(f"qsa_attend_{layer}_{batch}" if seq == 1 else "qsa_attend",
+                             lib.qm_qsa_attend_workspace(ctypes.byref(g), seq, splits))
         if out is None:
             out = torch.empty(batch, seq, c.num_attention_heads * c.head_dim, dtype=dt, device=self.device)
         native.call("qm_qsa_attend", ctypes.byref(g), seq, native.ptr(q_out), native.ptr(qg), native.ptr(lc.k_pool),
