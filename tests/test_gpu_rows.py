@@ -177,3 +177,57 @@ def test_bf16_gates_equal_the_precise_chains(gpu, rows):
         want = mix(8)
         assert torch.equal(want[0].view(BF).float(), torch.sigmoid(v.float()).to(BF).float()) or v.float().amin() < -87
         assert torch.equal(mix(rows), want[:1].expand(rows, -1))
+
+
+def test_project_stays_visible_to_torch(gpu, monkeypatch):
+    """What intercepts, casts or records F.linear sees the projections of 5 rows
+    too: autocast, dispatch and function modes, tensor subclasses, jit.trace,
+    fake tensors. Without any, and with a default device, they are one launch."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    qm = gpu
+    model = qm.Qwen4MixModel(qm.MixConfig(), gi.FakeStore(gi.dn_weights(0, 31, BF)), device=DEV, max_ctx=256)
+    x, y = (gi.normal(gi.rng(s), (1, 5, gi.HIDDEN)).to(BF).to(DEV) for s in (1, 2))
+    n = len(model.PROJ_GROUPS["dn_in"])
+    inner, native_calls, seen = qm.native.call, [], []
+    monkeypatch.setattr(qm.native, "call", lambda name, *a: (native_calls.append(name), inner(name, *a))[1])
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            if func is torch.nn.functional.linear:
+                seen.append("linear")
+            return func(*args, **(kwargs or {}))
+
+    class Sub(torch.Tensor):
+        pass
+
+    want = model.project(x, 0, "dn_in")
+    assert native_calls == ["qm_gemm_rows"]
+    with torch.device(DEV):
+        model.project(x, 0, "dn_in")
+    assert native_calls == ["qm_gemm_rows"] * 2
+    native_calls.clear()
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert [t.dtype for t in model.project(x, 0, "dn_in")] == [torch.float16] * n
+    with Dispatch():
+        model.project(x, 0, "dn_in")
+    assert sum("mm" in s for s in seen) == n
+    seen.clear()
+    with Function():
+        model.project(x, 0, "dn_in")
+    assert seen == ["linear"] * n
+    assert all(type(t) is Sub for t in model.project(x.as_subclass(Sub), 0, "dn_in"))
+    traced = torch.jit.trace(lambda t: tuple(model.project(t, 0, "dn_in")), (x,), check_trace=False)
+    for a, b in zip(traced(y), model.project(y, 0, "dn_in")):
+        assert rel_err(a, b, 1e-2) < 1e-2
+    native_calls.clear()
+    with FakeTensorMode(allow_non_fake_inputs=True) as mode:
+        fake = model.project(mode.from_tensor(x), 0, "dn_in")
+    assert [t.shape for t in fake] == [t.shape for t in want] and not native_calls
+    torch.cuda.synchronize()

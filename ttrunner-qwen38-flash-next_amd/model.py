@@ -27,6 +27,8 @@ import ctypes
 
 import torch
 import torch.nn.functional as F
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import native
 from .cache import MixHybridCache
@@ -123,13 +125,24 @@ class Qwen4MixModel:
 
     @staticmethod
     def _plain_input(x: torch.Tensor, w: torch.Tensor) -> bool:
-        """Whether the product can bypass F.linear: nothing here is differentiated
-        or transformed, and the operands are aligned device memory."""
+        """Whether the product can bypass F.linear: nothing here is differentiated,
+        transformed, cast, recorded or intercepted, and the operands are aligned
+        device memory."""
+        if type(x) not in (torch.Tensor, torch.nn.Parameter):
+            return False
         if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
             return False
         if torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0:
             return False
-        return x.device == w.device and x.is_cuda and x.data_ptr() % 16 == 0
+        if torch.is_autocast_enabled("cuda") or torch.jit.is_tracing() or torch.compiler.is_compiling():
+            return False
+        if torch._C._len_torch_dispatch_stack():
+            return False
+        # (a default device is a function mode too, one that leaves F.linear alone)
+        if torch._C._len_torch_function_stack() and not all(
+                isinstance(m, DeviceContext) for m in _get_current_function_mode_stack()):
+            return False
+        return x.is_cuda and x.device == w.device and x.data_ptr() % 16 == 0
 
     def project(self, x: torch.Tensor, layer: int, group: str) -> list:
         """The group's projections of x [B, S, K] (F.linear with each weight), as
@@ -140,8 +153,8 @@ class Qwen4MixModel:
         w, rows = self._wcat(layer, group, dt)
         batch, seq, k = x.shape
         entry = self._proj_entry(dt, batch * seq, k, len(rows))
-        xc = x.contiguous() if entry else x
-        if entry == "qm_gemv" or (entry and self._plain_input(xc, w)):
+        if entry == "qm_gemv" or (entry and self._plain_input(x, w)):
+            xc = x.contiguous()
             outs = [torch.empty(batch, seq, r, dtype=dt, device=self.device) for r in rows]
             seg_rows = (ctypes.c_int * len(rows))(*rows)
             seg_out = (ctypes.c_void_p * len(rows))(*[o.data_ptr() for o in outs])
