@@ -440,6 +440,15 @@ int qm_hc_mix(const qm_hc_geom* g, const void* hyper, const float* norm_w, const
               int with_inject, const void* up_w, void* mixed, void* inject, void* workspace,
               size_t workspace_bytes, hipStream_t stream);
 
+/* qm_hc_mix by the kernels that it takes for as_rows rows: a row's results are
+ * then, bit for bit, those of a call of as_rows rows (a verify step's drafted
+ * tokens those of their single steps), where qm_hc_mix sums in another order
+ * from 9 rows on and again from 193 (bf16) or 513 (f32). Slower than qm_hc_mix
+ * where that would take other kernels. */
+int qm_hc_mix_as(const qm_hc_geom* g, int as_rows, const void* hyper, const float* norm_w, const void* down_inject_w,
+                 int with_inject, const void* up_w, void* mixed, void* inject, void* workspace,
+                 size_t workspace_bytes, hipStream_t stream);
+
 /* Qwen4ExpModel._reinject (reference/model.py:79-81):
  * out[m][s * hidden + h] = hyper[m][s * hidden + h] + branch[m][h] * inject[m][s],
  * each product and sum rounded to act. hyper/out [M, streams * hidden],

@@ -189,6 +189,34 @@ def test_step_n_matches_single_steps(stack, k):
     restore(cache, snap)
 
 
+@pytest.mark.parametrize("k", [9, 14])
+def test_step_n_of_longer_drafts_matches_single_steps(stack, k):
+    """The same with the row counts at which qm_hc_mix itself takes other kernels
+    than a single step's."""
+    test_step_n_matches_single_steps(stack, k)
+
+
+@pytest.mark.parametrize("k", [9, 14])
+def test_step_n_graph_equals_step_n_of_longer_drafts(stack, k):
+    """The captured verify step of such a draft leaves step_n's rows and first
+    layer's state, bit for bit, on every replay."""
+    qm, model, cache = stack
+    snap = snapshot(cache)
+    x = inputs(1, k=k, seed=17)[0]
+    print(f"step_n_graph k={k}", flush=True)
+    want = qm.decoder.MixDecoder(model, cache).step_n(x).clone()
+    state = cache[0].recurrent_state.clone()
+    restore(cache, snap)
+    dec = qm.decoder.MixDecoder(model, cache)
+    held = dec.snapshot()
+    for _ in range(3):
+        got = dec.step_n_graph(x).clone()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want) and torch.equal(cache[0].recurrent_state, state)
+        dec.restore(held)
+    restore(cache, snap)
+
+
 def _export(cache):
     """The device caches as the reference's layer caches (reference/cache.py:19-29), on the CPU."""
     from oracle.cache import OracleHybridCache

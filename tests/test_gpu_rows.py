@@ -231,3 +231,22 @@ def test_project_stays_visible_to_torch(gpu, monkeypatch):
         fake = model.project(mode.from_tensor(x), 0, "dn_in")
     assert [t.shape for t in fake] == [t.shape for t in want] and not native_calls
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("dtype", [BF, F32])
+@pytest.mark.parametrize("rows,as_rows", [(9, 1), (14, 1), (14, 2), (33, 8), (200, 9), (530, 192), (20, 1000)])
+def test_hyper_mix_as_has_the_bits_of_that_row_count(gpu, dtype, rows, as_rows):
+    """qm_hc_mix_as over ``rows`` rows == qm_hc_mix over the same rows, as_rows at
+    a time, mixed and inject, bit for bit."""
+    qm = gpu
+    print(f"mix of {rows} rows as {as_rows} {dtype}", flush=True)
+    store = gi.FakeStore(gi.hc_weights("blk.5.hc_attn", 5, dtype, hidden=2048))
+    model = qm.Qwen4MixModel(qm.MixConfig(), store, device=DEV)
+    n = max(rows, as_rows)
+    n += -n % as_rows
+    hyper = gi.normal(gi.rng(rows), (1, n, 4 * 2048), 1.0).to(dtype).to(DEV)
+    parts = [model._gated_residual(h, 5, "attn") for h in hyper.split(as_rows, 1)]
+    mixed, _, inject = model._gated_residual(hyper[:, :rows], 5, "attn", as_rows=as_rows)
+    torch.cuda.synchronize()
+    assert torch.equal(mixed, torch.cat([p[0] for p in parts], 1)[:, :rows])
+    assert torch.equal(inject, torch.cat([p[2] for p in parts], 1)[:, :rows])

@@ -359,14 +359,18 @@ const char* hc_check(const qm_hc_geom* g) {
 // Where the matrix-core kernels (hc_rows.hip) take over. They would be faster
 // from 4 rows on (whole mix, us, here and there: bf16 11.5 / 10.5 at 4 rows,
 // 12.7 / 10.6 at 5, 24.7 / 10.9 at 14; float 18.9 / 17.4 at 5, 35.6 / 18.2 at
-// 14), but these kernels give a row the same bits at every row count, and a
-// verify step's few drafted tokens should see the inputs that their single
-// steps saw: with another order of the sums the first layer's states came out
-// 1.4e-3 apart instead of below 1e-3. So up to 8 rows stay here.
+// 14; one row 12 us slower over a step of four layers), but these kernels give a
+// row the same bits at every row count, and a verify step's few drafted tokens
+// should see the inputs that their single steps saw. So up to 8 rows stay here,
+// and longer drafts by qm_hc_mix_as: with the matrix cores' order of the sums
+// the first layer's states of 9 to 40 tokens and of as many single steps came
+// out up to 1.7e-3 apart (20 seeds), with these up to 6e-4 (a verify step of four
+// layers 230 / 252 us for 9 tokens, 240 / 285 for 14).
 constexpr int HC_ROWS_MIN = 9;
 
-bool hc_takes_rows(const qm_hc_geom& g) {
-  return g.rows >= HC_ROWS_MIN && qm_hc_rows_covers(g) && qm_hc_rows_workspace(g) <= hc_layout(g).total;
+// as_rows: the row count by which the kernels are chosen
+bool hc_takes_rows(const qm_hc_geom& g, int as_rows) {
+  return as_rows >= HC_ROWS_MIN && qm_hc_rows_covers(g) && qm_hc_rows_workspace(g) <= hc_layout(g).total;
 }
 
 template <typename T, int MG, int NQ>
@@ -451,10 +455,11 @@ extern "C" size_t qm_hc_mix_workspace(const qm_hc_geom* g) {
   return hc_layout(*g).total;
 }
 
-extern "C" int qm_hc_mix(const qm_hc_geom* g, const void* hyper, const float* norm_w, const void* down_inject_w,
-                         int with_inject, const void* up_w, void* mixed, void* inject, void* workspace,
-                         size_t workspace_bytes, hipStream_t stream) {
+extern "C" int qm_hc_mix_as(const qm_hc_geom* g, int as_rows, const void* hyper, const float* norm_w,
+                            const void* down_inject_w, int with_inject, const void* up_w, void* mixed, void* inject,
+                            void* workspace, size_t workspace_bytes, hipStream_t stream) {
   if (const char* why = hc_check(g)) return qm_fail(QM_ERR_ARG, why);
+  if (as_rows <= 0) return qm_fail(QM_ERR_ARG, "qm_hc_mix_as: as_rows must be positive");
   if (!hyper || !norm_w || !down_inject_w || !up_w || !mixed || !workspace)
     return qm_fail(QM_ERR_ARG, "qm_hc_mix: null pointer");
   if (!aligned16(hyper) || !aligned16(norm_w) || !aligned16(down_inject_w) || !aligned16(up_w) ||
@@ -465,11 +470,21 @@ extern "C" int qm_hc_mix(const qm_hc_geom* g, const void* hyper, const float* no
   // those kernels read hyper again beside the stores of mixed; here the first
   // launch alone reads it
   const size_t mixed_bytes = (size_t)g->rows * g->hidden * (g->act_dtype == QM_ACT_BF16 ? 2 : 4);
-  if (hc_takes_rows(*g) && aligned16(mixed) && !qm_overlap(mixed, mixed_bytes, hyper, g->streams * mixed_bytes))
-    return qm_hc_mix_rows(*g, hyper, norm_w, down_inject_w, with_inject, up_w, mixed, inject, workspace, stream);
+  if (hc_takes_rows(*g, as_rows) && aligned16(mixed) &&
+      !qm_overlap(mixed, mixed_bytes, hyper, g->streams * mixed_bytes))
+    return qm_hc_mix_rows(*g, as_rows, hyper, norm_w, down_inject_w, with_inject, up_w, mixed, inject, workspace,
+                          stream);
   if (g->act_dtype == QM_ACT_BF16)
     return run_mix<bf16_t>(*g, hyper, norm_w, down_inject_w, with_inject, up_w, mixed, inject, workspace, stream);
   return run_mix<float>(*g, hyper, norm_w, down_inject_w, with_inject, up_w, mixed, inject, workspace, stream);
+}
+
+extern "C" int qm_hc_mix(const qm_hc_geom* g, const void* hyper, const float* norm_w, const void* down_inject_w,
+                         int with_inject, const void* up_w, void* mixed, void* inject, void* workspace,
+                         size_t workspace_bytes, hipStream_t stream) {
+  if (const char* why = hc_check(g)) return qm_fail(QM_ERR_ARG, why);
+  return qm_hc_mix_as(g, g->rows, hyper, norm_w, down_inject_w, with_inject, up_w, mixed, inject, workspace,
+                      workspace_bytes, stream);
 }
 
 extern "C" int qm_hc_reinject(const qm_hc_geom* g, const void* hyper, const void* branch, const void* inject,

@@ -710,7 +710,7 @@ template <> struct HrFew<bf16_t> { static constexpr int ROWS = 192; };
 template <> struct HrFew<float> { static constexpr int ROWS = 512; };
 
 template <typename T>
-int run_rows(const qm_hc_geom& g, const void* hyper, const float* norm_w, const void* w_di, int with_inject,
+int run_rows(const qm_hc_geom& g, int as_rows, const void* hyper, const float* norm_w, const void* w_di, int with_inject,
              const void* w_up, void* mixed, void* inject, void* ws, hipStream_t stream) {
   const HrLayout L = hr_layout(g);
   char* base = static_cast<char*>(ws);
@@ -723,7 +723,7 @@ int run_rows(const qm_hc_geom& g, const void* hyper, const float* norm_w, const 
   A.M = g.rows; A.streams = g.streams; A.hidden = g.hidden; A.rank = g.rank;
   A.n_rows = g.rank + (with_inject ? g.streams : 0); A.np = L.np; A.eps = g.eps;
   const int n_tiles = (A.n_rows + 15) / 16;
-  if (g.rows <= HrFew<T>::ROWS) {
+  if (as_rows <= HrFew<T>::ROWS) {
     constexpr int VE = Chunk<T>::VE;
     const dim3 gd(n_tiles, g.streams, (g.rows + 15) / 16), gu(g.hidden / 16, (g.rows + 15) / 16);
     if (g.hidden == 2048)
@@ -777,9 +777,9 @@ bool qm_hc_rows_covers(const qm_hc_geom& g) {
 
 size_t qm_hc_rows_workspace(const qm_hc_geom& g) { return hr_layout(g).total; }
 
-int qm_hc_mix_rows(const qm_hc_geom& g, const void* hyper, const float* norm_w, const void* w_di, int with_inject,
-                   const void* w_up, void* mixed, void* inject, void* ws, hipStream_t stream) {
+int qm_hc_mix_rows(const qm_hc_geom& g, int as_rows, const void* hyper, const float* norm_w, const void* w_di,
+                   int with_inject, const void* w_up, void* mixed, void* inject, void* ws, hipStream_t stream) {
   if (g.act_dtype == QM_ACT_BF16)
-    return run_rows<bf16_t>(g, hyper, norm_w, w_di, with_inject, w_up, mixed, inject, ws, stream);
-  return run_rows<float>(g, hyper, norm_w, w_di, with_inject, w_up, mixed, inject, ws, stream);
+    return run_rows<bf16_t>(g, as_rows, hyper, norm_w, w_di, with_inject, w_up, mixed, inject, ws, stream);
+  return run_rows<float>(g, as_rows, hyper, norm_w, w_di, with_inject, w_up, mixed, inject, ws, stream);
 }

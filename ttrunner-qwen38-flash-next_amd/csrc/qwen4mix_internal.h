@@ -51,8 +51,9 @@ int qm_zero_words(void* p, long n_words, hipStream_t stream);
 
 // The hyper-connection mix over many token rows on the matrix cores
 // (hc_rows.hip): the geometries its kernels cover, the scratch they need, and
-// the launches. hyper, norm_w, w_di, w_up, mixed and ws are 16-byte aligned.
+// the launches (chosen by as_rows). hyper, norm_w, w_di, w_up, mixed and ws are
+// 16-byte aligned.
 bool qm_hc_rows_covers(const qm_hc_geom& g);
 size_t qm_hc_rows_workspace(const qm_hc_geom& g);
-int qm_hc_mix_rows(const qm_hc_geom& g, const void* hyper, const float* norm_w, const void* w_di, int with_inject,
-                   const void* w_up, void* mixed, void* inject, void* ws, hipStream_t stream);
+int qm_hc_mix_rows(const qm_hc_geom& g, int as_rows, const void* hyper, const float* norm_w, const void* w_di,
+                   int with_inject, const void* w_up, void* mixed, void* inject, void* ws, hipStream_t stream);

@@ -190,12 +190,13 @@ class Qwen4MixModel:
         c = self.config
         return native.HcGeom(rows, c.hc_count, c.hidden_size, c.hc_lowrank, native.act_code(dtype), c.rms_norm_eps)
 
-    def _gated_residual(self, hyper: torch.Tensor, layer, kind: str, mixed=None, inject=None):
+    def _gated_residual(self, hyper: torch.Tensor, layer, kind: str, mixed=None, inject=None, as_rows=None):
         """reference/model.py:53-77: (mixed [.., hidden], hyper, inject [.., hc_count] or None).
 
-        One qm_hc_mix call (two launches): the per-stream norm, the down and
-        inject products and their gates, the up product and the gated mean.
-        ``mixed``/``inject`` may be preallocated outputs."""
+        One qm_hc_mix call (two or three launches): the per-stream norm, the down
+        and inject products and their gates, the up product and the gated mean.
+        ``mixed``/``inject`` may be preallocated outputs. With ``as_rows`` a row
+        has the bits of a call of that many rows (qm_hc_mix_as)."""
         c = self.config
         dt = hyper.dtype
         lead = hyper.shape[:-1]
@@ -208,8 +209,8 @@ class Qwen4MixModel:
             mixed = torch.empty(*lead, c.hidden_size, dtype=dt, device=self.device)
         if with_inject and inject is None:
             inject = torch.empty(*lead, c.hc_count, dtype=dt, device=self.device)
-        native.call("qm_hc_mix", ctypes.byref(g), native.ptr(hyper_c), native.ptr(norm_w), native.ptr(di),
-                    int(with_inject), native.ptr(up), native.ptr(mixed), native.ptr(inject) if with_inject else None,
+        native.call("qm_hc_mix_as", ctypes.byref(g), as_rows or rows, native.ptr(hyper_c), native.ptr(norm_w),
+                    native.ptr(di), int(with_inject), native.ptr(up), native.ptr(mixed), native.ptr(inject) if with_inject else None,
                     native.ptr(ws), ws.numel(), native.stream_handle(self.device))
         return mixed, hyper, (inject if with_inject else None)
 
