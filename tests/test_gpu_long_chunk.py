@@ -1,5 +1,7 @@
 """Prefill chunks whose rows go through the chunk attention in parts (more than
-280 MB of partial outputs: about 1090 rows of one sequence, 540 of two)."""
+280 MB of partial outputs: 1024 rows of one sequence, 512 of two), against the
+same tokens in chunks of 300 rows, which are one part and which test_gpu_qsa.py
+compares with the oracle."""
 
 from __future__ import annotations
 
@@ -25,6 +27,29 @@ def _setup(qm, dtype, batch, seed):
     cache = qm.MixHybridCache(LAYER + 1, model.config, batch, 4096, DEV, dtype, page_table="random", seed=3)
     gen = torch.Generator(device=DEV).manual_seed(seed)
     return model, cache, lambda n: [torch.randn(batch, n, w, generator=gen, device=DEV).to(dtype) for w in WIDTHS]
+
+
+@pytest.mark.parametrize("dtype,batch,seq", [(BF, 1, 1024), (BF, 1, 1025), (BF, 1, 1333), (BF, 1, 2172), (F32, 1, 1333),
+                                             (BF, 2, 700), (F32, 2, 530), (BF, 9, 260)])
+def test_parts_equal_shorter_chunks(gpu, dtype, batch, seq):
+    """Row by row: a wrong row of a part would hide in the whole. A row's partials
+    and selection do not depend on the rows beside it, so bf16 differs by at most
+    one rounding (2^-8) and float32 by the merge's order (1e-6)."""
+    qm = gpu
+    pos = 1500                                       # the selection is on from token 2112
+    print(f"chunk of {seq} rows in parts, batch {batch} {dtype}", flush=True)
+    outs, caches = [], []
+    for step in (seq, 300):
+        model, cache, rand = _setup(qm, dtype, batch, 6)
+        model.qsa_core(*rand(pos), LAYER, cache, 0)
+        x = rand(seq)
+        outs.append(torch.cat([model.qsa_core(*(t[:, r:r + step].contiguous() for t in x), LAYER, cache, pos + r)
+                               for r in range(0, seq, step)], 1).float())
+        caches.append(cache[LAYER])
+    torch.cuda.synchronize()
+    err = (outs[0] - outs[1]).abs().amax(-1) / outs[1].abs().amax(-1)
+    assert float(err.max()) <= (2 ** -8 if dtype == BF else 1e-6)
+    assert torch.equal(caches[0].k_pool, caches[1].k_pool) and torch.equal(caches[0].block_keys, caches[1].block_keys)
 
 
 @pytest.mark.parametrize("dtype,at", [(BF, 0.5), (F32, 0.5), (F32, 0.0)])

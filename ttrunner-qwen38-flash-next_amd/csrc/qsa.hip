@@ -3605,10 +3605,12 @@ constexpr int COMBINE_MANY_ROWS = 256;
 // rows a workgroup 63.5; 1999 rows over 127 blocks, one workgroup per block and
 // kv head: 297 us, now 207).
 constexpr int CA_SEG_SPANS = 1;
-// A long chunk's rows go through the attention and the merge in parts whose
-// partial outputs (270 KB a row) stay in the 256 MB memory-side cache from the
-// one to the other, each over the last one's: 1999 rows (540 MB) 207 + 96 us in
-// two parts, 193 + 150 in one, 233 + 111 in four.
+// A long chunk's rows go through the attention and the merge in parts, each part's
+// partial outputs (270 KB a row) over the last one's, so that most of a part is
+// still in the 256 MB memory-side cache when the merge reads it: 1999 rows (540
+// MB) 207 + 96 us in two parts of up to 277 MB, 193 + 150 in one, 233 + 111 in
+// four. At most this many bytes a part, of whole 128-row spans; one span of more
+// than 8 sequences is more.
 constexpr size_t CA_PART_BYTES = 280ull << 20;
 
 template <typename T>
@@ -3670,8 +3672,10 @@ int attend_chunk(const qm_qsa_geom* g, int seq, const void* q, const void* qg, c
   // that lie over q take one part
   const size_t q_elems = (size_t)g->batch * seq * g->n_heads * QSA_D;
   const bool over = qm_overlap(out, q_elems * (g->act_dtype == QM_ACT_F32 ? 4 : 2), q, q_elems * 2 * sizeof(uint16_t));
-  const size_t n_part = over ? 1 : (seq * row_bytes + CA_PART_BYTES - 1) / CA_PART_BYTES;
-  const int part = (int)(((seq + n_part - 1) / n_part + 127) / 128 * 128);
+  const size_t most = CA_PART_BYTES / row_bytes / 128 * 128;
+  const int max_part = over || most > (size_t)seq ? seq : most < 128 ? 128 : (int)most;
+  const int n_part = (seq + max_part - 1) / max_part;
+  const int part = ((seq + n_part - 1) / n_part + 127) / 128 * 128;      // several: not above max_part
   for (int row0 = 0; row0 < seq; row0 += part) {
     A.row0 = row0;
     A.rows = part < seq - row0 ? part : seq - row0;
