@@ -49,8 +49,8 @@ def test_recurrent_rule_blocks(gpu, dtype, batch, heads, seq):
 
 @pytest.mark.parametrize("seq", [15, 16, 23, 24, 25])
 def test_prefill_rule_at_the_dispatch(gpu, seq):
-    """qm_dn_prefill either side of the line between the token loop and the
-    chunked rule (24 tokens): the same prompt one token at a time through the
+    """qm_dn_prefill either side of the lines between its forms (16 tokens: the
+    loop forms the conv itself; 32: the chunked rule): the same prompt one token at a time through the
     decode path. bf16 outputs within 2e-2 of the largest value, the state within
     1e-3 (the bars of the decode and prefill tests)."""
     qm = gpu
@@ -72,6 +72,11 @@ def test_prefill_rule_at_the_dispatch(gpu, seq):
     assert float((got.float() - want.float()).abs().max() / want.float().abs().max()) < 2e-2
     assert float((many[0].recurrent_state - one[0].recurrent_state).abs().max()) < 1e-3
     assert torch.equal(many[0].conv_state, one[0].conv_state)
+
+
+@pytest.mark.parametrize("seq", [17, 31, 32, 33, 34])
+def test_prefill_rule_at_the_chunked_line(gpu, seq):
+    test_prefill_rule_at_the_dispatch(gpu, seq)
 
 
 @pytest.mark.parametrize("over", ["v", "q", "g"])

@@ -42,8 +42,12 @@ constexpr int CP_NT = 512;        // prep: eight waves (the rule over 4096 token
 constexpr int CK_LD = CK_D + 4;   // LDS row stride of [token][dim] tiles, floats
 constexpr int CK_LT = CK_C + 4;   // LDS row stride of [.][token] tiles, floats
 constexpr int CK_COLS = 16;       // d_v columns per scan workgroup
-constexpr int CK_MIN_SEQ = 24;    // shorter prefill chunks take the token loop (us, loop / chunked, 32 heads in
-                                  // bf16: 11.9 / 16.9 at 16 tokens, 15.9 / 17.0 at 24, 18.1 / 17.0 at 32)
+// Shorter prefill chunks take the token loop, which works in blocks of 16 tokens:
+// two of them are the faster, three are not (kernels alone, 32 heads, us, loop /
+// chunked: bf16 12.4 / 14.4 at 24 tokens, 14.2 / 14.5 at 32, 18.0 / 14.6 at 40;
+// float 13.9 / 14.4 at 32, 18.0 / 14.7 at 40; four sequences in bf16 29.4 / 31.0
+// at 32, 37.1 / 31.8 at 40).
+constexpr int CK_MIN_SEQ = 33;
 constexpr int CK_PARTS = 4;       // prep workgroups per chunk when chunks are few
 
 // One record per (sequence, head, chunk), in floats. A fragment pair is the

@@ -368,7 +368,7 @@ __global__ __launch_bounds__(DN_DEC_NT) void dn_decode_kernel(
 // ---------------------------------------------------------------------------
 // Multi-token recurrence on already split and expanded q, k, v (the free
 // function recurrent_gated_delta_rule, reference/layers.py:155-192, and the
-// prefill path's chunks under 24 tokens). A workgroup keeps 16 state columns of
+// prefill path's chunks of up to 32 tokens). A workgroup keeps 16 state columns of
 // a head in registers across the tokens: wave w four of them, lane l rows
 // 8 (l / 4) .. + 7 of column l % 4. Nothing but the state depends on the tokens
 // before, so the norms, gates and dot products of a block of up to 16 tokens

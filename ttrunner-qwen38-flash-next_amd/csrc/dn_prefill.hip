@@ -8,7 +8,7 @@
 //                   thread loads its channel's window inputs at once, then
 //                   writes 16 outputs; the first token block writes the ring;
 //                   the same grid computes beta and g for every (token, head)
-//   delta rule      the WY/UT chunked kernels (dn_chunk.hip) for chunks of 24
+//   delta rule      the WY/UT chunked kernels (dn_chunk.hip) for chunks of 33
 //                   tokens or more, the token loop for shorter ones
 //   dn_gated_norm   one wavefront per (token, head) row of 128
 // Up to 16 tokens of few sequences are two launches: the token loop forms the

@@ -34,7 +34,7 @@ int qm_dn_short(const qm_dn_geom* g, int seq, const void* qkv, const void* a, co
                 void* out, hipStream_t stream);
 
 // The delta rule over a chunk of tokens for the prefill path: the WY/UT chunked
-// kernels (64-token chunks) for chunks of 24 tokens or more, the token loop for
+// kernels (64-token chunks) for chunks of 33 tokens or more, the token loop for
 // shorter ones. `ws` holds qm_dn_rule_chunk_workspace(batch, seq, heads) bytes.
 size_t qm_dn_rule_chunk_workspace(int batch, int seq, int heads);
 int qm_dn_rule_chunk(int act_dtype, int batch, int seq, int heads, int hk, long q_stride, long v_stride,
