@@ -1,6 +1,6 @@
-"""The route of a QSA decode batch: plans of up to 8 sequences (5 with the
-selection on, and 640 scored blocks in all) run in one launch, larger ones as
-prep + select + attend; both give the same step, and bind() takes either."""
+"""The route of a QSA decode batch: small batches over few blocks run in one
+launch (Qwen4MixModel.fused_decode_fits), larger ones as prep + select + attend;
+both give the same step, and bind() takes either."""
 
 from __future__ import annotations
 
@@ -51,6 +51,37 @@ def test_batch_routes_agree(gpu, dtype, batch, pos, one_launch):
         caches.append(cache[LAYER])
     assert float((outs[0] - outs[1]).abs().max() / outs[1].abs().max()) < 2e-2
     assert torch.equal(caches[0].k_pool, caches[1].k_pool) and torch.equal(caches[0].v_pool, caches[1].v_pool)
+
+
+@pytest.mark.parametrize("batch,blocks,one_launch", [
+    (1, 640, True), (1, 641, False), (2, 512, True), (2, 513, False), (3, 341, True), (3, 342, False), (4, 256, True),
+    (4, 257, False), (5, 129, False), (5, 128, True), (7, 128, True), (8, 128, False), (7, 65, True), (6, 64, False),
+    (5, 64, True), (8, 32, True), (9, 32, False), (8, 0, True)])
+def test_route_at_its_lines(gpu, batch, blocks, one_launch):
+    """Both routes of a step either side of every line of the rule, on caches of
+    seeded random blocks: the same output within the decode tests' 2e-2."""
+    qm = gpu
+    plan = import_module(qm.__name__ + ".plan")
+    print(f"route of {batch} x {blocks} blocks", flush=True)
+    pos = blocks * 64 + 40
+    model = qm.Qwen4MixModel(qm.MixConfig(), gi.FakeStore(gi.qsa_weights(LAYER, 90, torch.bfloat16)), device=DEV)
+    gen = torch.Generator(device=DEV).manual_seed(batch + blocks)
+    r = lambda *s: torch.randn(*s, generator=gen, device=DEV).to(torch.bfloat16)  # noqa: E731
+    cache = qm.MixHybridCache(LAYER + 1, model.config, batch, 49152, DEV, page_table="random", seed=4)
+    lc = cache[LAYER]
+    lc.keys, lc.values, lc.indexer_keys = r(batch, 2, pos, 256), r(batch, 2, pos, 256), r(batch, pos, 128)
+    lc.block_keys.copy_(torch.randn(lc.block_keys.shape, generator=gen, device=DEV))
+    x = [r(batch, 1, n) for n in (16 * 512, 512, 512, 512, 128)]
+    outs = []
+    for fused in (None, not one_launch):
+        p = plan.QsaDecodePlan(model, cache, LAYER, pos, torch.bfloat16, fused=fused)
+        assert p.fused == (one_launch if fused is None else fused)
+        p.positions.fill_(pos)
+        p.run(*x)
+        torch.cuda.synchronize()
+        assert p.check() == []
+        outs.append(p.out.float().clone())
+    assert float((outs[0] - outs[1]).abs().max() / outs[1].abs().max()) < 2e-2
 
 
 def test_bind_refuses_what_one_sequence_refuses(gpu):

@@ -453,20 +453,27 @@ class Qwen4MixModel:
         return (c.indexer_compress_ratio in (32, 64) and cache.max_blocks <= 4096
                 and cache.max_ctx <= 4096 * c.indexer_compress_ratio and c.block_topk <= 510)
 
-    # Up to this many eligible blocks, over all sequences of the batch, the
-    # one-launch decode is the faster path: each of its workgroups scores and
-    # ranks every eligible block of its sequence itself, so its time grows with
-    # the context (one sequence, cold, MI355X: 11.0 us at 127 blocks, 25.3 at
-    # 511, 36.8 at 1023, 60.6 at 2047), while prep + the scores spread over the
-    # blocks + the ranking + the attention stay near 28-35 us. A batch
-    # multiplies the workgroups too, past what the device holds at once (us, one
-    # launch / split path: 312 blocks 26 / 23 for 2 sequences, 58 / 28 for 8,
-    # 162 / 44 for 24; 127 blocks 20 / 25 for 4, 36 / 29 for 8, 190 / 69 for 48).
+    # Where the one-launch decode is the faster path. Each of its workgroups
+    # scores and ranks every eligible block of its sequence itself, so its time
+    # grows with the context, and with the batch past what the device holds at
+    # once; prep + the scores spread over the blocks + the ranking + the attention
+    # stay near 21-29 us (bf16, cold, MI355X, us, one launch / split path; float
+    # within 1 us of it):
+    # one sequence: 18.6 / 23.3 at 511 blocks, 21.3 / 23.9 at 640, 23.4 / 23.4 at
+    # 700, 28.7 / 24.1 at 1023
     FUSED_MAX_BLOCKS = 640
-    # ... and up to this many sequences, with the selection on (62 blocks: 20 /
-    # 23 for 4, 35 / 28 for 8) and off (31 blocks: 22 / 24 for 8, 43 / 30 for
-    # 16; 4 blocks: 12 / 20 for 4, 22 / 21 for 8, 122 / 25 for 48)
-    FUSED_MAX_BATCH_SCORED, FUSED_MAX_BATCH = 5, 8
+    # more than 128 blocks (ranked by buckets): up to 4 sequences and 1024 blocks
+    # in all (2 x 512: 22.1 / 24.8; 3 x 300: 21.2 / 25.0; 4 x 256: 23.4 / 26.2;
+    # 5 x 140: 29.8 / 26.4)
+    FUSED_COUNTED_BLOCKS, FUSED_MAX_BATCH_RANKED, FUSED_MAX_BLOCKS_IN_ALL = 128, 4, 1024
+    # up to 128 (by counting, the split path's slowest ranking): 5 sequences, 7
+    # from 65 blocks on (5 x 62: 22.5 / 26.3; 6 x 127: 25.0 / 28.6; 7 x 127: 26.0 /
+    # 29.1; 8 x 62: 32.3 / 28.4; 6 and 7 sequences of fewer blocks gain 1 to 2 us
+    # at most and keep the split path)
+    FUSED_MAX_BATCH_SCORED, FUSED_MAX_BATCH_COUNTED = 5, 7
+    # the selection off: 8 (31 blocks: 21.0 / 25.0, 9 sequences 27.6 / 26.1; 4
+    # blocks: 21.6 / 21.4, 9 sequences 26.3 / 22.1)
+    FUSED_MAX_BATCH = 8
 
     def fused_decode_fits(self, cache, max_position=None, batch=None) -> bool:
         """Whether qm_qsa_decode covers this cache's geometry (and, given a
@@ -478,8 +485,13 @@ class Qwen4MixModel:
         if max_position is not None:
             batch = cache.batch if batch is None else batch
             blocks = (max_position + 1) // c.indexer_compress_ratio
-            most = self.FUSED_MAX_BATCH if blocks <= c.block_topk else self.FUSED_MAX_BATCH_SCORED
-            fits = fits and batch * blocks <= self.FUSED_MAX_BLOCKS and batch <= most
+            if blocks <= c.block_topk:
+                most = self.FUSED_MAX_BATCH
+            elif blocks > self.FUSED_COUNTED_BLOCKS:
+                most = min(self.FUSED_MAX_BATCH_RANKED, self.FUSED_MAX_BLOCKS_IN_ALL // blocks)
+            else:
+                most = self.FUSED_MAX_BATCH_COUNTED if blocks > 64 else self.FUSED_MAX_BATCH_SCORED
+            fits = fits and blocks <= self.FUSED_MAX_BLOCKS and batch <= most
         return fits
 
     def decode_group_fits(self, splits: int, dtype) -> bool:
