@@ -403,6 +403,50 @@ def test_rows_at_different_positions_match_single_rows(stack):
     assert dec.positions.cpu().tolist() == [500, 500] and dec.row_positions == [500, 500]
 
 
+def test_a_server_batch_matches_single_rows(stack):
+    """A 12-row decoder with its rows at different positions, whose captured step
+    takes the many-rows kernels throughout (mix, projections, the reinjection's
+    epilogue, the split QSA decode), against single-row decoders over slot views
+    of an identical cache: every row of the residual within 2e-2 over three
+    replays, with the single rows' eager work between them."""
+    qm, model, _ = stack
+    c = model.config
+    rows = [1100 - 37 * i for i in range(12)]
+
+    def make():
+        cache = qm.cache.MixHybridCache(N_LAYERS, c, batch=len(rows), max_ctx=2048, device=DEV, dtype=BF,
+                                        page_table="random", seed=5)
+        g = torch.Generator(device=DEV).manual_seed(23)
+        r = lambda t, scale=1.0: t.copy_(torch.randn(t.shape, generator=g, device=DEV) * scale)  # noqa: E731
+        for l in range(N_LAYERS):
+            lc = cache[l]
+            if c.is_full_attention(l):
+                lc.ensure_qsa(len(rows), BF)
+                for t in (lc.k_pool, lc.v_pool, lc.raw_keys, lc.block_keys):
+                    r(t)
+                lc.blocks_valid = max(rows) // c.indexer_compress_ratio
+            else:
+                lc.ensure_dn(len(rows), BF)
+                r(lc.recurrent_state, 0.02)
+                r(lc.conv_ring)
+            lc.n_tokens = max(rows)
+        cache.slot_tokens[:] = rows
+        return cache
+
+    batch_cache, single_cache = make(), make()
+    dec = qm.decoder.MixDecoder(model, batch_cache, positions=rows)
+    singles = [qm.decoder.MixDecoder(model, single_cache.slot_view(i)) for i in range(len(rows))]
+    g = torch.Generator(device=DEV).manual_seed(12)
+    for step in range(3):
+        print(f"server batch: step {step}", flush=True)
+        h = torch.randn(len(rows), 1, c.hc_count * c.hidden_size, generator=g, device=DEV).to(BF)
+        got = dec.step(h).clone()
+        for i in range(len(rows)):
+            want = singles[i].step_eager(h[i:i + 1])
+            torch.cuda.synchronize()
+            assert rel_err(got[i], want[0], 2e-2) < 2e-2, (step, i)
+
+
 def _dn_state(cache):
     return [(lc.recurrent_state.clone(), lc.conv_ring.clone()) for lc in cache.layers if lc.recurrent_state is not None]
 

@@ -56,6 +56,13 @@ def test_hyper_mix_rows_match_oracle(gpu, dtype, hidden, rows):
             assert rel_err(inject, want_inject, tol) < tol
 
 
+@pytest.mark.parametrize("dtype,hidden,rows", [(BF, 2048, 1041), (BF, 2048, 2000), (BF, 2560, 800), (F32, 2048, 1100)])
+def test_hyper_mix_of_long_prompts_matches_oracle(gpu, dtype, hidden, rows):
+    """Rows past one round of the many-rows kernel's row groups (1024 rows in bf16,
+    768 at hidden 2560), where its waves take a second tile."""
+    test_hyper_mix_rows_match_oracle(gpu, dtype, hidden, rows)
+
+
 def _gemm_rows(qm, w, x, rows):
     m, k = x.shape
     outs = [torch.full((m, r), float("nan"), dtype=x.dtype, device=DEV) for r in rows]

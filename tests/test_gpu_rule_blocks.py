@@ -79,6 +79,58 @@ def test_prefill_rule_at_the_chunked_line(gpu, seq):
     test_prefill_rule_at_the_dispatch(gpu, seq)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("batch,heads,seq", [(2, 32, 1216), (3, 24, 1000), (1, 100, 7808)])
+def test_chunked_rule_in_segments(gpu, dtype, batch, heads, seq):
+    """The chunked rule over more records than one segment takes, for several
+    sequences and (7808 tokens of 100 heads) with a last segment of two chunks,
+    whose preparation is split in four, against the token loop. Per token, of its
+    largest value: the chunked form's operands have 16 bits (2^-16, summed over 64
+    tokens: a few times that), and bf16 rounds both outputs, each by up to half a
+    step of its 8 bits (2^-8)."""
+    from importlib import import_module
+    layers = import_module(gpu.__name__ + ".layers")
+    print(f"segments {dtype} batch={batch} heads={heads} seq={seq}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(seq + heads)
+    r = lambda *s: torch.randn(*s, generator=gen, device=DEV)  # noqa: E731
+    q, k, v = (r(batch, seq, heads, 128).to(dtype) for _ in range(3))
+    g, beta = -r(batch, seq, heads).abs(), torch.sigmoid(r(batch, seq, heads))
+    S = r(batch, heads, 128, 128) * 0.1
+    want, want_S = layers.recurrent_gated_delta_rule(q, k, v, g, beta, S)
+    out, state = layers.chunk_gated_delta_rule(q, k, v, g, beta, S)
+    torch.cuda.synchronize()
+    bar = 8 * 2 ** -16 + (2 * 2 ** -8 if dtype == torch.bfloat16 else 0)
+    err = (out.float() - want.float()).abs().amax((2, 3)) / want.float().abs().amax((2, 3))
+    print(f"  worst token {float(err.max()):.2e}", flush=True)
+    assert float(err.max()) < bar
+    assert float((state - want_S).abs().max() / want_S.abs().max()) < 8 * 2 ** -16
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_prefill_in_segments_equals_shorter_calls(gpu, dtype):
+    """Two prompts of 1216 tokens through a DeltaNet core (16 q/k heads for 32
+    value heads; two segments) == their first 640 and last 576 tokens in calls of
+    one segment each, whose chunks are the same."""
+    qm = gpu
+    import os
+    import sys
+    sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden"))
+    import inputs as gi
+    seq, cut = 1216, 640
+    print(f"prefill in segments {dtype}", flush=True)
+    model = qm.Qwen4MixModel(qm.MixConfig(), gi.FakeStore(gi.dn_weights(0, 7, dtype)), device=DEV, max_ctx=64)
+    gen = torch.Generator(device=DEV).manual_seed(3)
+    x = [torch.randn(2, seq, n, generator=gen, device=DEV).to(dtype) for n in (8192, 4096, 32, 32)]
+    one, two = (qm.MixHybridCache(1, model.config, 2, 2048, DEV, dtype) for _ in range(2))
+    got = model.dn_core(*x, 0, one[0])
+    want = torch.cat([model.dn_core(*(t[:, s].contiguous() for t in x), 0, two[0])
+                      for s in (slice(0, cut), slice(cut, seq))], 1)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    assert torch.equal(one[0].recurrent_state, two[0].recurrent_state)
+    assert torch.equal(one[0].conv_state, two[0].conv_state)
+
+
 @pytest.mark.parametrize("over", ["v", "q", "g"])
 def test_chunked_rule_into_its_inputs_memory(gpu, over):
     """2304 tokens of 32 heads are more records than one segment takes (160 MB).

@@ -75,3 +75,44 @@ def test_short_chunk_equals_its_tokens_in_a_longer_one(gpu, dtype, kernel, hk, h
             slot = (int(pos0[i]) + t) % kernel
             assert torch.equal(rings[1][i, :, slot], qkv[i, t])
             assert torch.equal(rings[0][i, :, slot], qkv[i, t])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("batch,seq", [(2, 9), (3, 9), (2, 16), (3, 16), (2, 17), (3, 8), (16, 8), (17, 8), (16, 9), (17, 1)])
+def test_batches_at_the_short_forms_lines(gpu, dtype, batch, seq):
+    """Batches either side of where the short form stops (2 sequences, 16 up to 8
+    tokens): each sequence's outputs, state and ring are those of a call of its
+    own, which takes the short form up to 16 tokens. Bars as above."""
+    native = import_module(gpu.__name__ + ".native")
+    print(f"short chunk {dtype} batch={batch} seq={seq}", flush=True)
+    hk, hv, kernel = 2, 4, 4
+    conv_dim = (2 * hk + hv) * 128
+    gen = torch.Generator(device=DEV).manual_seed(seq * 32 + batch)
+    r = lambda *s: torch.randn(*s, generator=gen, device=DEV)  # noqa: E731
+    x = [r(batch, seq, n).to(dtype) for n in (conv_dim, hv * 128, hv, hv)]
+    a_neg, dt_bias, norm_w, conv_w = -r(hv).abs(), r(hv), r(128), r(conv_dim, kernel).to(dtype)
+    ring0, state0 = r(batch, conv_dim, kernel).to(dtype), r(batch, hv, 128, 128) * 0.1
+    pos0 = torch.arange(batch, dtype=torch.int32, device=DEV) * 37
+
+    def run(rows):
+        n = len(range(batch)[rows])
+        geom = native.DnGeom(n, hv, hk, 128, kernel, native.act_code(dtype), 1e-6)
+        xs, ring, state, pos = [t[rows].contiguous() for t in x], ring0[rows].clone(), state0[rows].clone(), pos0[rows].clone()
+        out = torch.empty(n, seq, hv * 128, dtype=dtype, device=DEV)
+        ws = torch.empty(native.load().qm_dn_prefill_workspace(ctypes.byref(geom), seq), dtype=torch.uint8, device=DEV)
+        native.call("qm_dn_prefill", ctypes.byref(geom), seq, *(native.ptr(t) for t in xs), native.ptr(a_neg),
+                    native.ptr(dt_bias), native.ptr(conv_w), native.ptr(norm_w), native.ptr(pos), native.ptr(ring),
+                    native.ptr(state), native.ptr(out), native.ptr(ws), ws.numel(), native.stream_handle())
+        torch.cuda.synchronize()
+        return out.float(), state, ring
+
+    got = run(slice(0, batch))
+    want = [torch.cat(t) for t in zip(*(run(slice(i, i + 1)) for i in range(batch)))]
+    err = (got[0] - want[0]).abs().amax(2) / want[0].abs().amax(2)
+    assert float(err.max()) <= (1e-6 if dtype == torch.float32 else 2 ** -8)
+    assert float((got[1] - want[1]).abs().max() / want[1].abs().max()) <= 1e-6
+    # every slot but the one that holds no past input, which only a longer chunk's ring write may touch
+    for i in range(batch):
+        for j in range(1, kernel):
+            slot = (int(pos0[i]) + seq - j) % kernel
+            assert torch.equal(got[2][i, :, slot], want[2][i, :, slot])
