@@ -320,7 +320,10 @@ int qm_qsa_decode(const qm_qsa_geom* g, const void* qg, const void* k_new, const
 /* Bytes of workspace qm_qsa_attend needs for `seq` query rows and `splits`. */
 size_t qm_qsa_attend_workspace(const qm_qsa_geom* g, int seq, int splits);
 /* Split count (workgroups per row and kv head) covering every query row at
- * positions first_position .. last_position. */
+ * positions first_position .. last_position. The counts are not monotone (a
+ * position that completes a block attends no tail): a plan for positions up to
+ * last_position takes first_position = last_position - ratio (at least 0), which
+ * bounds every earlier one. */
 int qm_qsa_attend_splits(const qm_qsa_geom* g, int first_position, int last_position);
 
 /* Paged GQA attention of `seq` query rows per sequence over each row's item

@@ -120,3 +120,30 @@ def test_eager_decode_buffers_are_a_layers_own(gpu, monkeypatch, batch, pos):
         model.qsa_core(*x, layer, cache, pos)
     torch.cuda.synchronize()
     assert taken[3] and taken[7] and not taken[3] & taken[7]
+
+
+@pytest.mark.parametrize("batch,top,low", [(6, 2559, 2500), (9, 4095, 2113), (2, 41087, 41003), (1, 41087, 41050)])
+def test_split_plan_covers_positions_below_its_largest(gpu, batch, top, low):
+    """A split plan whose largest position completes a block, and so attends no
+    tail, at positions that do: the same as the plan for that position. (Sized
+    for its largest position alone, such a plan left out the tail, the newest
+    tokens.)"""
+    qm = gpu
+    plan = import_module(qm.__name__ + ".plan")
+    print(f"split plan for {top} at {low}, batch {batch}", flush=True)
+    model = qm.Qwen4MixModel(qm.MixConfig(), gi.FakeStore(gi.qsa_weights(LAYER, 90, torch.bfloat16)), device=DEV)
+    gen = torch.Generator(device=DEV).manual_seed(top)
+    r = lambda *s: torch.randn(*s, generator=gen, device=DEV).to(torch.bfloat16)  # noqa: E731
+    cache = qm.MixHybridCache(LAYER + 1, model.config, batch, 45056, DEV, page_table="random", seed=4)
+    lc = cache[LAYER]
+    lc.keys, lc.values, lc.indexer_keys = r(batch, 2, low, 256), r(batch, 2, low, 256), r(batch, low, 128)
+    lc.block_keys.copy_(torch.randn(lc.block_keys.shape, generator=gen, device=DEV))
+    x = [r(batch, 1, n) for n in (16 * 512, 512, 512, 512, 128)]
+    outs = []
+    for max_position in (low, top):
+        p = plan.QsaDecodePlan(model, cache, LAYER, max_position, torch.bfloat16, fused=False)
+        p.positions.fill_(low)
+        p.run(*x)
+        torch.cuda.synchronize()
+        outs.append(p.out.float().clone())
+    assert float((outs[1] - outs[0]).abs().max() / outs[0].abs().max()) < 2e-2

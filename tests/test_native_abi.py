@@ -128,6 +128,19 @@ def test_workspace_sizes_are_sane(qm):
     assert lib.qm_qsa_items_stride(ctypes.byref(q)) == 1 + 64 + 3
 
 
+def test_attend_splits_of_a_plan_cover_every_position(qm):
+    """The items of a range that starts a block before its end bound those of every
+    earlier position (a decode plan's positions), tails included."""
+    n = qm.native
+    lib = n.load()
+    for ratio, budget in ((64, 2048), (32, 256), (4, 64)):
+        q = n.QsaGeom(1, 16, 2, 256, 64, 4, 128, ratio, budget, 64, 128, 8192, 8192 // ratio, n.QM_ACT_BF16, 1e-6)
+        most = 0
+        for p in range(0, 3000):
+            most = max(most, lib.qm_qsa_attend_splits(ctypes.byref(q), p, p))
+            assert lib.qm_qsa_attend_splits(ctypes.byref(q), max(0, p - ratio), p) >= most, (ratio, p)
+
+
 def test_rope_tables_bit_identical_to_reference(qm):
     meta = json.load(open(os.path.join(ROOT, "tests", "golden", "golden_meta.json")))
     if meta["torch"] != torch.__version__ or meta["cpu_capability"] != torch.backends.cpu.get_cpu_capability():

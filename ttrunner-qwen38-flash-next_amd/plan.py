@@ -104,7 +104,10 @@ class QsaDecodePlan:
         dev = model.device
         self.geom = model.qsa_geom(cache, dtype)
         lib = native.load()
-        self.splits = lib.qm_qsa_attend_splits(ctypes.byref(self.geom), max_position, max_position)
+        # a position that completes a block attends no tail, so the largest position
+        # need not have the most items; the last ``ratio`` positions bound all before
+        first = max(0, max_position - model.config.indexer_compress_ratio)
+        self.splits = lib.qm_qsa_attend_splits(ctypes.byref(self.geom), first, max_position)
         self.ws = torch.zeros(lib.qm_qsa_attend_workspace(ctypes.byref(self.geom), 1, self.splits),
                               dtype=torch.uint8, device=dev)
         self.dec_splits = lib.qm_qsa_decode_splits(ctypes.byref(self.geom), max_position)
