@@ -18,7 +18,7 @@
 // Measured with weights from memory, against the library's GEMMs that served
 // these row counts (us): DeltaNet input projections (50 MB) 45.3 -> 13.8 at 16
 // rows (3.7 TB/s), 44.7 -> 17.5 at 32, 45.5 -> 26.2 at 64 (the weights are read
-// once per 32 rows; once per 16 it was 20.6 and 33.9); output projection (17 MB) 11.8 -> 6.5 at 16,
+// once per 32 rows; once per 16, as at other k, it was 20.6 and 33.9); output projection (17 MB) 11.8 -> 6.5 at 16,
 // with the reinjection's own launch (4.7 us) gone as well.
 #include "rows_mma.h"
 #include "qwen4mix_internal.h"

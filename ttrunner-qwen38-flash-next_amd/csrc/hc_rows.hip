@@ -24,7 +24,7 @@
 //
 // The whole mix, before (hc.hip at every row count) and now, us, rank 320,
 // 4 x 2048, weights in cache: bf16 24.7 -> 10.9 at 14 rows, 66.8 -> 15.1 at 64,
-// 122 -> 24 at 128, 272 -> 42 at 300, 1761 -> 62 at 2000 (340 TFLOP/s); float
+// 122 -> 24 at 128, 272 -> 42 at 300, 1761 -> 63 at 2000 (335 TFLOP/s); float
 // 35.6 -> 18.2 at 14, 239 -> 56 at 128, 545 -> 123 at 300, 3580 -> 474 at 2000.
 //
 // Roundings are where hc.hip makes them; only the order of the float sums

@@ -12,8 +12,8 @@ return values, so an engine written against the reference can call them:
 
 Weights come from ``store.get(f"blk.{layer}.{suffix}")`` as in
 reference/model.py:45-49 and are copied to the device once. The projections
-(``F.linear``) run as PyTorch-ROCm GEMMs; everything between them -- conv ring,
-gates, delta rule, norms, rope, paging, indexer scoring, top-k, attention,
+(``F.linear``) of up to 64 rows run in the library's own kernels, of more as
+PyTorch-ROCm GEMMs; everything between them -- conv ring, gates, delta rule, norms, rope, paging, indexer scoring, top-k, attention,
 output gate -- runs in the HIP kernels of libqwen4mix.so. There is no other
 implementation to fall back to: a missing library or a failed call raises.
 
