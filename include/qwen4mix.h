@@ -325,6 +325,9 @@ size_t qm_qsa_attend_workspace(const qm_qsa_geom* g, int seq, int splits);
  * last_position takes first_position = last_position - ratio (at least 0), which
  * bounds every earlier one. */
 int qm_qsa_attend_splits(const qm_qsa_geom* g, int first_position, int last_position);
+/* Attention items of a row that this many splits cover; the output of a row with
+ * more is NaN. */
+int qm_qsa_attend_items(int splits);
 
 /* Paged GQA attention of `seq` query rows per sequence over each row's item
  * list (its selected blocks plus its tail block), then the sigmoid output gate

@@ -147,3 +147,27 @@ def test_split_plan_covers_positions_below_its_largest(gpu, batch, top, low):
         torch.cuda.synchronize()
         outs.append(p.out.float().clone())
     assert float((outs[1] - outs[0]).abs().max() / outs[0].abs().max()) < 2e-2
+
+
+def test_split_plan_reports_a_position_beyond_it(gpu):
+    """A batch past its plan's position: NaN and a fault in check(), as from a
+    one-launch plan; the rows within it are served, and a later step is clean."""
+    qm = gpu
+    plan = import_module(qm.__name__ + ".plan")
+    batch = 9
+    print("split plan, a position beyond it", flush=True)
+    model = qm.Qwen4MixModel(qm.MixConfig(), gi.FakeStore(gi.qsa_weights(LAYER, 90, torch.bfloat16)), device=DEV)
+    model.rope.get(4096)                     # the plan's tables cover the position all the same
+    cache = qm.MixHybridCache(LAYER + 1, model.config, batch, 4096, DEV, page_table="random", seed=4)
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    x = [torch.randn(batch, 1, n, generator=gen, device=DEV).to(torch.bfloat16)
+         for n in (16 * 512, 512, 512, 512, 128)]
+    p = plan.QsaDecodePlan(model, cache, LAYER, 500, torch.bfloat16)
+    assert not p.fused and p.batched
+    p.positions.fill_(500)
+    p.positions[3] = 900
+    out = p.run(*x).float()
+    assert out[3].isnan().all() and not out[[0, 1, 2, 4, 5, 6, 7, 8]].isnan().any()
+    assert len(p.check()) == 1 and p.check() == []
+    p.positions.fill_(500)
+    assert not p.run(*x).isnan().any() and p.check() == []

@@ -1677,6 +1677,9 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void qsa_attend_kernel(AttnArgs A) 
 #pragma unroll
     for (int w = 0; w < ATT_WAVES; ++w)
       if (s_m[w][hh] != -INFINITY) L += s_l[w][hh] * __expf(s_m[w][hh] - Mh);
+    // more items than the grid covers (a plan sized for smaller positions): the
+    // row's output is poisoned, as the one-launch decode's
+    if (n_items > A.splits * ATT_WAVES) L = __builtin_nanf("");
     A.part_ml[(pbase + hh) * 2 + 0] = Mh;
     A.part_ml[(pbase + hh) * 2 + 1] = L;
   }
@@ -3515,6 +3518,8 @@ extern "C" int qm_qsa_attend_splits(const qm_qsa_geom* g, int first_position, in
   const int splits = (items + ATT_WAVES - 1) / ATT_WAVES;
   return splits < 1 ? 1 : splits;
 }
+
+extern "C" int qm_qsa_attend_items(int splits) { return splits * ATT_WAVES; }
 
 extern "C" size_t qm_qsa_attend_workspace(const qm_qsa_geom* g, int seq, int splits) {
   if (!g || splits <= 0 || seq <= 0) return 0;

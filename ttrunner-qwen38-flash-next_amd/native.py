@@ -67,6 +67,7 @@ SIGNATURES = {
     "qm_qsa_decode_front": (_i, [ctypes.POINTER(QsaGeom)] + [_vp] * 22 + [_vp]),
     "qm_qsa_select": (_i, [ctypes.POINTER(QsaGeom), _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "qm_qsa_attend_workspace": (_sz, [ctypes.POINTER(QsaGeom), _i, _i]),
+    "qm_qsa_attend_items": (_i, [_i]),
     "qm_qsa_attend_splits": (_i, [ctypes.POINTER(QsaGeom), _i, _i]),
     "qm_qsa_attend": (_i, [ctypes.POINTER(QsaGeom), _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _vp, _sz, _vp]),
     "qm_qsa_attend_chunk_workspace": (_sz, [ctypes.POINTER(QsaGeom), _i]),

@@ -205,12 +205,17 @@ class QsaDecodePlan:
         return BoundCall("qm_qsa_decode", *self._decode_args(qg, k, v, iq, ik))
 
     def check(self, reset: bool = True) -> list:
-        """Hand-off faults of this plan's fused launches since the last check
-        (a sync): waits that gave up, positions beyond the plan's splits."""
-        if not self.fused:
-            return []
-        return native.qsa_decode_faults(self.geom, self.dec_splits, self.dec_ws, reset, f"layer {self.layer}",
-                                        self.model.device)
+        """Faults of this plan's launches since the last check (a sync): waits that
+        gave up, positions beyond the plan's splits (of the last step alone on the
+        split path, which has no counters); their outputs are NaN."""
+        name = f"layer {self.layer}"
+        if self.fused:
+            return native.qsa_decode_faults(self.geom, self.dec_splits, self.dec_ws, reset, name, self.model.device)
+        counts = self.items[:, 0, 0]
+        over = int((counts > native.load().qm_qsa_attend_items(self.splits)).sum())
+        if reset:
+            counts.zero_()
+        return [f"{name}: {over} rows had more attention items than their {self.splits} splits cover"] if over else []
 
     def run(self, qg, k, v, iq, ik, stream=None):
         s = stream if stream is not None else native.stream_handle(self.model.device)
