@@ -124,6 +124,7 @@ class QsaDecodePlan:
         # and the attention (the scores' buffer makes qm_qsa_select split them)
         self.scores = None if self.fused else torch.empty(batch, 1, cache.max_blocks, dtype=torch.float32,
                                                            device=dev)
+        # on the split path too: decode() may be called on any plan that fits one launch
         self.dec_ws = torch.zeros(lib.qm_qsa_decode_workspace(ctypes.byref(self.geom), self.dec_splits),
                                   dtype=torch.uint8, device=dev)
         self.positions = torch.zeros(batch, dtype=torch.int32, device=dev)
